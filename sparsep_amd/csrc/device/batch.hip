@@ -127,7 +127,12 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
     std::vector<Acc> acc;
     for (int i = 0; i < nprob; i++) {
         const sp_plan *p = plans[i];
-        const Work &w = p->work;
+        // one launch group for all even-row problems of a chunk width: the row kernel also for one
+        // right-hand side (a group of wide tiles and its fix-up beside it: 158 against 154 us for
+        // 24 problems of up to 2M entries)
+        const bool rows = p->many && p->many->work.kind == WK_CSR_VEC;
+        const PlanWork &pw = rows ? *p->many : p->group(k[i]);
+        const Work &w = pw.work;
         b->algo_bytes += p->algo_bytes + (uint64_t)(k[i] - 1) * ((uint64_t)p->nrows + p->ncols) * sp_dtype_size(dt);
         const int kmax = max_rhs_chunk(w);
         for (int done = 0; done < k[i];) {
@@ -158,21 +163,21 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
             g.w.chunk = g.w.chunk && w.chunk;
             Acc &a = acc[gi];
             const uint32_t pid0 = (uint32_t)a.probs.size();
-            for (const spd::Prob &P0 : p->h_probs) {
+            for (const spd::Prob &P0 : pw.h_probs) {
                 spd::Prob P = P0;
                 P.ldx = k[i];
                 P.ldy = k[i];
                 a.probs.push_back(P);
                 g.slots.push_back({(uint32_t)i, P0.xoff * k[i] + done, P0.yoff * k[i] + done});
             }
-            for (uint32_t u : p->h_unit_pid) a.unit_pid.push_back(u + pid0);
-            a.c0.insert(a.c0.end(), p->h_c0.begin(), p->h_c0.end());
-            a.c1.insert(a.c1.end(), p->h_c1.begin(), p->h_c1.end());
-            a.c2.insert(a.c2.end(), p->h_c2.begin(), p->h_c2.end());
+            for (uint32_t u : pw.h_unit_pid) a.unit_pid.push_back(u + pid0);
+            a.c0.insert(a.c0.end(), pw.h_c0.begin(), pw.h_c0.end());
+            a.c1.insert(a.c1.end(), pw.h_c1.begin(), pw.h_c1.end());
+            a.c2.insert(a.c2.end(), pw.h_c2.begin(), pw.h_c2.end());
             g.w.hcol_max = std::max(g.w.hcol_max, w.hcol_max);
-            for (size_t z = 0; z < p->h_zrow.size(); z++) {
-                a.zpid.push_back(p->h_zpid[z] + pid0);
-                a.zrow.push_back(p->h_zrow[z]);
+            for (size_t z = 0; z < pw.h_zrow.size(); z++) {
+                a.zpid.push_back(pw.h_zpid[z] + pid0);
+                a.zrow.push_back(pw.h_zrow[z]);
             }
             done += kc;
         }
@@ -187,7 +192,7 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
         w.nunits = (uint32_t)a.unit_pid.size();
         w.nzero = (uint32_t)a.zrow.size();
         // persistent grid: enough workgroups to fill every CU several times over
-        w.grid_cap = (uint32_t)std::max(1, ctx->num_cus) * (w.kind == WK_CSR_HOT ? 1 : 8);
+        w.grid_cap = (uint32_t)std::max(1, ctx->num_cus) * (w.kind == WK_CSR_HOT ? 1 : 8);  // (wide tiles: one each)
         if (w.kind == WK_CSR_HOT) {
             // every slot stages its own x (a plan may appear in several slots)
             for (spd::Prob &P : a.probs) {
@@ -203,9 +208,7 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
         if (!a.c1.empty() && (rc = bupload(b, a.c1, &w.d_c1))) break;
         if (!a.c2.empty() && (rc = bupload(b, a.c2, &w.d_c2))) break;
         if (w.nzero && ((rc = bupload(b, a.zpid, &w.d_zpid)) || (rc = bupload(b, a.zrow, &w.d_zrow)))) break;
-        const bool carries = w.kind == WK_CSR_MERGE || w.kind == WK_COO_SEG || w.kind == WK_BCOO_SEG || w.kind == WK_CSR_HOT ||
-                             w.kind == WK_BCSR_SEG;
-        if (carries) {
+        if (has_carries(w.kind)) {
             const uint32_t S = (w.kind == WK_BCOO_SEG || w.kind == WK_BCSR_SEG) ? w.R : 1;
             const size_t n = (size_t)std::max<uint32_t>(w.nunits, 1) * S;
             const size_t asz = (dt == SP_I64 || dt == SP_F64) ? 8 : 4;
@@ -213,21 +216,11 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
             if ((rc = balloc(b, n * 4, (void **)&w.d_carry_row))) break;
             if ((rc = balloc(b, n * g.kc * asz, &w.d_carry_val))) break;
         }
-        if (w.kind == WK_CSR_MERGE && !w.nzero && w.nunits) {
-            // the rows crossing tiles as runs (unit t carries the row at its end coordinate),
-            // as a single plan lists them: each run's carries are added with independent loads
-            // instead of a walk over the units that stops at the run's end
-            std::vector<spd::Run> runs;
-            for (uint32_t t = 0; t < w.nunits; t++) {
-                const uint32_t pid = a.unit_pid[t], r = a.c0[(size_t)t + pid + 1];
-                const spd::Prob &P = a.probs[pid];
-                if (r >= P.nrows || r >= P.nrows_elem) continue;
-                if (!runs.empty()) {
-                    spd::Run &q = runs.back();
-                    if (q.pid == pid && q.row == r && q.t0 + q.n == t) { q.n++; continue; }
-                }
-                runs.push_back(spd::Run{pid, t, 1, r, P.yoff + (int64_t)r, P.ldy, 0});
-            }
+        if (((w.kind == WK_CSR_MERGE && !w.nzero) || w.kind == WK_WIDE) && w.nunits) {
+            // the rows crossing tiles as runs, as a single plan lists them: each run's carries
+            // are added with independent loads instead of a walk over the units that stops at
+            // the run's end
+            const std::vector<spd::Run> runs = crossing_runs(w.kind, a.probs, a.unit_pid, a.c0, a.c2);
             w.nruns = (uint32_t)runs.size();
             if ((rc = bupload(b, runs, &w.d_runs))) break;
         }

@@ -110,6 +110,9 @@ template <typename T> using gptr = __attribute__((address_space(1))) T *;
 template <typename T> __device__ __forceinline__ gptr<const T> gp(const T *p) { return (gptr<const T>)p; }
 template <typename T> __device__ __forceinline__ gptr<T> gp(T *p) { return (gptr<T>)p; }
 
+// Read-only data at an address that is the same in every lane (scalar loads).
+template <typename T> using cptr = __attribute__((address_space(4))) T *;
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 

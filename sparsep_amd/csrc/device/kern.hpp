@@ -45,8 +45,8 @@ struct Prob {
     int64_t xoff, yoff;    // element offsets into the per-call x / y bases
     int32_t ldx, ldy;      // leading dimensions when x / y come from pointer tables
     uint32_t pbits;        // CSR merge tiles in column order: cind holds col << pbits | position in tile
-    uint32_t nhcol;        // hot-x CSR: number of staged ("hot") columns
-    const uint32_t *hcol;  // hot-x CSR: the staged columns, slot order
+    uint32_t nhcol;        // hot-x CSR: number of staged ("hot") columns; wide tiles: entries per tile
+    const uint32_t *hcol;  // hot-x CSR: the staged columns, slot order; wide tiles: base column per 64 words
     void *xh;              // hot-x CSR: x at the staged columns, written before each launch
 };
 
@@ -565,6 +565,194 @@ __global__ __launch_bounds__(HOT_TPB) void csr_hot_kernel(const Prob *__restrict
         cv[q] = cv2[q];
         vv[q] = vv2[q];
     }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// CSR and COO, wide column-ordered tiles (one right-hand side).  A tile of
+// NT * IPT consecutive entries is stored by ascending column, so that one
+// gather instruction reads 64 neighbouring columns; the wider the tile, the
+// fewer cache lines a gather touches (R-MAT 2^20, 128-byte lines per entry:
+// 0.66 at 2048 entries, 0.57 at 4096, 0.46 at 8192, 0.36 at 16384), and the
+// requests from the L1s to the L2 bound a matrix with scattered columns.
+//
+// Layout (wide_sort_kernel): groups of 256 words, NT * IPT words per tile;
+// word 4 l + i of group g (of G) is entry l of run i G + g, the runs being the
+// tile's entries in column order cut into 64s: lane l loads its four keys and
+// its four values as one piece each, gather i of the wave still covers 64
+// consecutive columns, and every wave has runs from all parts of the tile, the
+// crowded columns and the sparse ones.  A key is (column - base) << pbits
+// | slot, base the first column of the entry's run (P.hcol, one per 64 words),
+// so the tile width does not limit the matrix's columns; the slot is the LDS
+// place of the entry's row-order position (wide_slot).  A run that would span
+// too many columns ends early.  Words left over repeat an entry of their run:
+// they store the same product to the same slot once more, so no lane checks
+// bounds.  A tile holds P.nhcol entries, NT * IPT at most and 256 less where
+// columns need more than 32 - pbits bits, which leaves room for four early ends.
+//
+// Products go to their slots in LDS.  Each thread then takes its IPT
+// consecutive entries in 16-byte reads; one stored word per thread (P.ptr)
+// says which of them end a row (low half) and how many rows of the tile end
+// before it (high half), so no row pointer is searched or compared: a running
+// sum in registers, a segmented scan of the open ends over lanes and then
+// waves, the row sums to LDS in row order, and from there to y: P.rind holds
+// for every row 1 + the number of its sum in the tile where the row ends, or 0
+// for a row without entries.  The open end of a tile is its carry; which row
+// it belongs to is known to the plan (its run list).
+// ---------------------------------------------------------------------------
+// Slot of row-order position pos: a thread's 16-byte pieces are exchanged by a
+// function of the thread, so that 16 neighbouring threads' reads of piece c
+// fall into different banks.  ce = values per piece, cpt = pieces per thread.
+__host__ __device__ __forceinline__ constexpr uint32_t wide_slot(uint32_t pos, uint32_t ce, uint32_t cpt) {
+    return pos ^ (((pos / (ce * cpt) / (16 / cpt)) & (cpt - 1)) * ce);
+}
+// Groups in use of a tile of nb entries: one more than they fill, for runs that end early.
+__host__ __device__ __forceinline__ constexpr uint32_t wide_groups(uint32_t nb, uint32_t words) {
+    return (nb + 255) / 256 < words / 256 ? (nb + 255) / 256 + 1 : words / 256;
+}
+
+template <typename A> __device__ __forceinline__ A shfl_any(A v, int src) {
+    if constexpr (sizeof(A) == 4) {
+        return __builtin_bit_cast(A, __shfl(__builtin_bit_cast(int, v), src, WAVE));
+    } else {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)u, src, WAVE);
+        const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(u >> 32), src, WAVE);
+        return __builtin_bit_cast(A, ((uint64_t)hi << 32) | lo);
+    }
+}
+
+// Inclusive segmented sum over N lanes (a power of two): bit l of `ends` says
+// that lane l's value starts anew.
+template <int N, typename A> __device__ __forceinline__ A open_scan(A v, uint64_t ends, int lane) {
+    const uint64_t upto = ends & ((2ull << lane) - 1);
+    const int st = upto ? 63 - __builtin_clzll(upto) : 0;
+#pragma unroll
+    for (int off = 1; off < N; off <<= 1) {
+        const A ov = shfl_up_any(v, off);
+        if (lane - off >= st) v = ov + v;
+    }
+    return v;
+}
+
+template <typename T, int NT, int IPT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void wide_kernel(
+    const Prob *__restrict__ probs, const uint32_t *__restrict__ unit_pid, const uint32_t *__restrict__ cent,
+    const uint32_t *__restrict__ crow, Ptrs<T> io, acc_t<T> *__restrict__ carry_val) {
+    using A = acc_t<T>;
+    constexpr int TILE = NT * IPT, NW = NT / WAVE;
+    constexpr int R = IPT / 4;  // groups of 256 entries per wave
+    constexpr int CE = 16 / (int)sizeof(A), CPT = IPT / CE;
+    static_assert(IPT % 4 == 0 && (CPT & (CPT - 1)) == 0 && CPT <= 16 && IPT <= 16, "whole groups and pieces");
+    typedef A AP __attribute__((ext_vector_type(CE)));
+    __shared__ __align__(16) A s_buf[TILE];
+    __shared__ A s_wv[NW];
+    __shared__ uint32_t s_wf[NW];
+    const int tid = threadIdx.x, lane = tid % WAVE;
+    const uint32_t wid = (uint32_t)__builtin_amdgcn_readfirstlane(tid / WAVE);
+    const uint32_t t = blockIdx.x;  // one tile per workgroup
+    const uint32_t pid = unit_pid ? unit_pid[t] : 0u, ci = t + pid;
+    const Prob P = probs[pid];
+    const gptr<const T> __restrict__ x = gp(io.x(pid, P));
+    const gptr<T> __restrict__ y = gp(io.y(pid, P));
+    const gptr<const uint16_t> __restrict__ rmap = gp((const uint16_t *)P.rind);
+    const gptr<const T> __restrict__ vals = gp((const T *)P.val);
+    const int ldx = io.lx(P), ldy = io.ly(P);
+    const uint32_t j0 = cent[ci], nb = cent[ci + 1] - j0, r0 = crow[ci], nr = crow[ci + 1] - r0;
+    const uint32_t tl = j0 / P.nhcol, pb = P.pbits, pmask = (1u << pb) - 1;  // tile of its problem
+    const uint32_t G = wide_groups(nb, TILE);  // groups in use
+    const uint32_t word = ldg(gp(P.ptr) + (size_t)tl * NT + tid);
+    const gptr<const uint32_t> __restrict__ keys = gp(P.cind) + (size_t)tl * TILE;
+    const gptr<const T> __restrict__ tv = vals + (size_t)tl * TILE;
+    const cptr<const u32x4> base = (cptr<const u32x4>)gp(P.hcol) + (size_t)tl * (TILE / 256);
+    // All keys and values of the tile go out first, then the gathers, two groups at a time (16
+    // entries per thread fit the 64 registers that eight waves per SIMD leave).
+    auto sweep = [&](auto one_c) {
+        constexpr bool ONE = decltype(one_c)::value;  // x contiguous: 32-bit offsets from the base column
+        constexpr int U = 2;
+        uint32_t key[R][4];
+        T v[R][4];
+#pragma unroll
+        for (int r = 0; r < R; r++) {  // waves past the last group take it again
+            const uint32_t g = min(wid + r * NW, G - 1);
+            const u32x4 w = __builtin_nontemporal_load((gptr<const u32x4>)(keys + 256 * g) + lane);
+#pragma unroll
+            for (int i = 0; i < 4; i++) key[r][i] = w[i];
+            ldg_n<T, 4>(tv + 256 * g + 4 * lane, v[r]);
+        }
+#pragma unroll
+        for (int q0 = 0; q0 < R; q0 += U) {
+            T xv[U][4];
+#pragma unroll
+            for (int r = 0; r < U; r++) {
+                const u32x4 bs = base[min(wid + (q0 + r) * NW, G - 1)];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if constexpr (ONE)
+                        xv[r][i] = *(gptr<const T>)((gptr<const char>)(x + bs[i]) + (key[q0 + r][i] >> pb) * (uint32_t)sizeof(T));
+                    else
+                        xv[r][i] = x[((size_t)bs[i] + (key[q0 + r][i] >> pb)) * (size_t)ldx];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < U; r++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) s_buf[key[q0 + r][i] & pmask] = mul<T>(v[q0 + r][i], xv[r][i]);
+            __builtin_amdgcn_sched_barrier(0);  // the next gathers stay behind: more in flight would spill
+        }
+    };
+    if (ldx == 1) sweep(std::true_type{});
+    else sweep(std::false_type{});
+    __syncthreads();
+
+    // running sums of this thread's entries, starting anew after each row end (what lies past the
+    // tile's entries reaches neither a row nor the carry)
+    const uint32_t mask = word & 0xFFFFu;
+    A p[IPT];
+#pragma unroll
+    for (int c = 0; c < CPT; c++) {
+        const AP q = *(const AP *)(s_buf + wide_slot(tid * IPT + c * CE, CE, CPT));
+#pragma unroll
+        for (int i = 0; i < CE; i++) p[c * CE + i] = q[i];
+    }
+#pragma unroll
+    for (int q = 1; q < IPT; q++) p[q] = (mask >> (q - 1) & 1) ? p[q] : p[q - 1] + p[q];
+    const A open = (mask >> (IPT - 1) & 1) ? A(0) : p[IPT - 1];
+    const uint64_t ends = __ballot(mask != 0);
+    const A v = open_scan<WAVE>(open, ends, lane);
+    if (lane == WAVE - 1) {
+        s_wv[wid] = v;
+        s_wf[wid] = ends != 0;
+    }
+    __syncthreads();
+    // open ends of the waves, scanned by every wave for itself (lane w holds wave w)
+    const uint64_t wends = __ballot(lane < NW && s_wf[lane % NW]);
+    const A wv = open_scan<NW>(s_wv[lane % NW], wends, lane);
+    const A cross = wid ? shfl_any(wv, (int)wid - 1) : A(0);
+    const A pv = shfl_up_any(v, 1);
+    const bool before = ends & ((1ull << lane) - 1);  // a row ends in this wave before this thread
+    A cin = lane ? pv : A(0);
+    if (!before) cin = cross + cin;
+    uint32_t ord = word >> 16;
+#pragma unroll
+    for (int q = 0; q < IPT; q++)
+        if (mask >> q & 1) {
+            s_buf[ord++] = cin + p[q];
+            cin = A(0);
+        }
+    // the thread of the tile's last entry holds its open end
+    if ((uint32_t)tid == (nb - 1) / IPT) carry_val[t] = ends & ((2ull << lane) - 1) ? v : cross + v;
+    __syncthreads();
+
+    // the rows that end in this tile and the empty ones among them, eight per thread at a time
+    // (a tile of a graph's sparse end has several rows per entry)
+    for (uint32_t k0 = tid; k0 < nr; k0 += 8 * NT) {
+        uint32_t m[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) m[i] = ldg(rmap + r0 + min(k0 + i * NT, nr - 1));
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (k0 + i * NT < nr) y[(size_t)(r0 + k0 + i * NT) * ldy] = m[i] ? to_val<T>(s_buf[m[i] - 1]) : T(0);
     }
 }
 

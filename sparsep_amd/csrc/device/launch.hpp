@@ -74,6 +74,19 @@ static int launch_main(const Work &w, hipStream_t s, Ptrs<T> io) {
             return SP_ERR_UNSUPPORTED;  // one right-hand side per pass (max_rhs_chunk)
         }
     }
+    if (w.kind == WK_WIDE) {
+        if constexpr (K == 1) {
+            const uint32_t *upid = w.nprob == 1 ? nullptr : w.d_unit_pid;  // one problem: pid 0
+#define SPD_WIDE(NTv, Iv) \
+    if (w.lanes == NTv && w.ipt == Iv) { hipLaunchKernelGGL((wide_kernel<T, NTv, Iv>), dim3(w.nunits), dim3(NTv), 0, s, w.d_prob, upid, w.d_c0, w.d_c1, io, cv); return hipGetLastError() == hipSuccess ? SP_OK : SP_ERR_HIP; }
+            if constexpr (sizeof(T) == 8) { SPD_WIDE(256, 8) SPD_WIDE(1024, 8) }  // (wide_shape's choices)
+            else { SPD_WIDE(512, 8) SPD_WIDE(256, 16) SPD_WIDE(1024, 16) }
+#undef SPD_WIDE
+            return SP_ERR_ARG;
+        } else {
+            return SP_ERR_UNSUPPORTED;  // one right-hand side per pass (max_rhs_chunk)
+        }
+    }
     switch (w.kind) {
     case WK_CSR_MERGE: {
         const uint32_t *upid = w.nprob == 1 ? nullptr : w.d_unit_pid;  // one problem: pid 0
@@ -296,7 +309,7 @@ static int launch_chunk(const Work &w, sp_ctx *ctx, Ptrs<T> io) {
         if (rc) return rc;
     }
     mark_dominant(ctx);
-    if (w.d_runs) {  // CSR merge with its run list
+    if (w.d_runs) {  // CSR merge and wide tiles with their run list
         if (w.nruns) {
             using A = acc_t<T>;
             hipLaunchKernelGGL((run_fixup_kernel<T, K>), dim3((w.nruns + 255) / 256), dim3(256), 0, s, w.d_runs, w.nruns,
@@ -305,8 +318,7 @@ static int launch_chunk(const Work &w, sp_ctx *ctx, Ptrs<T> io) {
         }
         return SP_OK;
     }
-    const bool carries = w.kind == WK_CSR_MERGE || w.kind == WK_COO_SEG || w.kind == WK_BCOO_SEG || w.kind == WK_CSR_HOT ||
-                         w.kind == WK_BCSR_SEG;
+    const bool carries = has_carries(w.kind);
     const uint32_t S = (w.kind == WK_BCOO_SEG || w.kind == WK_BCSR_SEG) ? w.R : 1;
     const uint64_t nthreads = (carries ? (uint64_t)S * w.nunits : 0) + w.nzero;
     if (nthreads) {

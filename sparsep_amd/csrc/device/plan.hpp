@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
 #include <vector>
 
 #include "sparsep.h"
@@ -32,7 +33,14 @@ inline void mark_dominant(sp_ctx *c) {
     if (c->mark_mid) (void)hipEventRecord(c->ev_mid, c->stream);
 }
 
-struct sp_plan {
+// A launch group and the host copies of its arrays (batches concatenate them).
+struct PlanWork {
+    Work work;
+    std::vector<spd::Prob> h_probs;
+    std::vector<uint32_t> h_unit_pid, h_c0, h_c1, h_c2, h_zpid, h_zrow;
+};
+
+struct sp_plan : PlanWork {  // (the base: the main launch group)
     sp_ctx *ctx = nullptr;
     int id = 0, dtype = 0, algo = 0;
     sp_opts opts{};
@@ -43,10 +51,13 @@ struct sp_plan {
     uint32_t nparts = 0, nsub = 0, lanes = 0, ipt = 0, vert = 0, ntiles = 0;
     uint32_t launches = 1;
 
-    Work work;                // the main launch group
-    // host copies of the work arrays (batches concatenate them)
-    std::vector<spd::Prob> h_probs;
-    std::vector<uint32_t> h_unit_pid, h_c0, h_c1, h_c2, h_zpid, h_zrow;
+    // wide tiles take one right-hand side: several run on this row-ordered group
+    std::unique_ptr<PlanWork> many;
+    // the group that a call with k right-hand sides runs
+    const PlanWork &group(int k) const {
+        if (k > 1 && many) return *many;
+        return *this;
+    }
     // 2D tilings: the work writes per-stripe partial rows into ypart
     // ([vert][nrows][k]); a reduction adds them into y in stripe order.
     bool tiled = false;
@@ -55,6 +66,7 @@ struct sp_plan {
     uint32_t ypart_k = 0;     // right-hand sides ypart currently holds
 
     std::vector<void *> allocs;
+
 };
 
 // Allocation helpers (record in plan->allocs, respect mem_cap_bytes).
@@ -72,6 +84,13 @@ int build_bcsr_plan(sp_plan *p, const sp_bcsr *B);
 int build_bcoo_plan(sp_plan *p, const sp_bcoo *B);
 int build_tiled_plan(sp_plan *p, const sp_coo *A);
 int run_plan(sp_plan *p, const void *x, void *y, int k, int ldx, int ldy);
+
+// Wide column-ordered tiles (wide.hip): sorts the device's row-ordered entries into tiles of
+// `words` words holding `entries` each and writes keys, values and base columns; ipt = entries
+// per thread, sa = bytes per accumulator; SP_ERR_RANGE when a tile's columns are too far apart.
+int launch_wide_sort(hipStream_t s, const uint32_t *cind, const void *vals, size_t sv, uint32_t nnz, uint32_t entries,
+                     uint32_t words, uint32_t pbits, uint32_t ipt, size_t sa, uint32_t *key, void *val, uint32_t *base,
+                     uint32_t *flag);
 
 // Utility kernels (util.hip).
 int launch_fill_zero(hipStream_t s, void *ptr, uint64_t bytes);

@@ -16,6 +16,23 @@ using spd::merge_search;
 using spd::Prob;
 using spd::TPB;
 
+std::vector<spd::Run> crossing_runs(int kind, const std::vector<Prob> &probs, const std::vector<uint32_t> &unit_pid,
+                                    const std::vector<uint32_t> &c0, const std::vector<uint32_t> &c2) {
+    std::vector<spd::Run> runs;  // consecutive units carrying the same row form one run
+    for (uint32_t t = 0; t < (uint32_t)unit_pid.size(); t++) {
+        const uint32_t pid = unit_pid[t];
+        const uint32_t r = kind == WK_WIDE ? c2[(size_t)t + pid] : c0[(size_t)t + pid + 1];
+        const Prob &P = probs[pid];
+        if (r >= P.nrows || r >= P.nrows_elem) continue;
+        if (!runs.empty()) {
+            spd::Run &b = runs.back();
+            if (b.pid == pid && b.row == r && b.t0 + b.n == t) { b.n++; continue; }
+        }
+        runs.push_back(spd::Run{pid, t, 1, r, P.yoff + (int64_t)r, P.ldy, 0});
+    }
+    return runs;
+}
+
 namespace {
 
 size_t acc_size(int dt) { return (dt == SP_I64 || dt == SP_F64) ? 8 : 4; }
@@ -64,7 +81,7 @@ struct Builder {
             if ((rc = plan_upload(p, zrow.data(), zrow.size() * 4, (void **)&w.d_zrow))) return rc;
         }
         if (carries) {
-            w.carry_k = (kind == WK_BCOO_SEG || kind == WK_BCSR_SEG) ? 1 : 8;
+            w.carry_k = (kind == WK_BCOO_SEG || kind == WK_BCSR_SEG || kind == WK_WIDE) ? 1 : 8;
             // atomic merges write no carries (batches allocate their own)
             if (p->algo != SP_ALGO_SEGMENTED_ATOMIC) {
                 const size_t n = (size_t)std::max<uint32_t>(w.nunits, 1) * slots;
@@ -72,23 +89,11 @@ struct Builder {
                 if ((rc = plan_alloc(p, n * w.carry_k * acc_size(p->dtype), &w.d_carry_val))) return rc;
             }
         }
-        if (kind == WK_CSR_MERGE && carries && !w.nzero) {
-            // tile t carries row c0[t + pid + 1] when that row exists; consecutive
-            // tiles carrying the same row form one run
-            std::vector<spd::Run> runs;
-            for (uint32_t t = 0; t < w.nunits; t++) {
-                const uint32_t pid = unit_pid[t], r = c0[(size_t)t + pid + 1];
-                const Prob &P = probs[pid];
-                if (r >= P.nrows || r >= P.nrows_elem) continue;
-                if (!runs.empty()) {
-                    spd::Run &b = runs.back();
-                    if (b.pid == pid && b.row == r && b.t0 + b.n == t) { b.n++; continue; }
-                }
-                runs.push_back(spd::Run{pid, t, 1, r, P.yoff + (int64_t)r, P.ldy, 0});
-            }
+        if (((kind == WK_CSR_MERGE && !w.nzero) || kind == WK_WIDE) && carries) {
+            const std::vector<spd::Run> runs = crossing_runs(kind, probs, unit_pid, c0, c2);
             w.nruns = (uint32_t)runs.size();
             if ((rc = plan_upload(p, runs.data(), runs.size() * sizeof(spd::Run), (void **)&w.d_runs))) return rc;
-            p->launches = 1 + (w.nruns ? 1 : 0);
+            p->launches = 1 + (w.nruns ? 1 : 0) + (w.nzero ? 1 : 0);
         } else {
             p->launches = 1 + ((carries || w.nzero) ? 1 : 0);
         }
@@ -340,6 +345,143 @@ void hot_tiles(const sp_csr *A, const std::vector<uint32_t> &cnnz, uint32_t pb, 
     for (auto &t : th) t.join();
 }
 
+// Threads and entries per thread of a wide tile; nt 0: no wide tiles.
+struct WideShape {
+    uint32_t nt = 0, ipt = 0;
+};
+
+// Cache lines of x that 64 consecutive entries touch, per entry, in row order (from up to 512
+// evenly spread samples).
+double row_lines(const uint32_t *colind, uint32_t nnz, size_t sv) {
+    const uint32_t windows = std::min<uint32_t>(nnz / 64, 512);
+    if (!windows) return 0.0;
+    uint64_t lines = 0;
+    for (uint32_t w = 0; w < windows; w++) {
+        const uint32_t *c = colind + (uint64_t)w * (nnz / 64) / windows * 64;
+        uint64_t l[64];
+        for (int i = 0; i < 64; i++) l[i] = (uint64_t)c[i] * sv / 128;
+        std::sort(l, l + 64);
+        lines += std::unique(l, l + 64) - l;
+    }
+    return (double)lines / (64.0 * windows);
+}
+
+// Whether an automatic 1D CSR/COO plan takes wide tiles, and which.  Against the kernels that
+// the row-ordered group would take (us per SpMV, before -> wide):
+//   skewed rows and COO from 32K entries on: R-MAT 2^12 x 8 FP32 CSR 8.4 -> 6.5, 2^16 x 16
+//     11.0 -> 8.2, 2^18 x 16 FP64 28.8 -> 22.7, 2^20 x 16 FP32 72.6 -> 62.1; COO 5-point stencil
+//     700^2 14.2 -> 9.6
+//   even rows: their single launch needs no fix-up, which decides small matrices (5-point
+//     stencil 256^2 INT32, 0.3M entries: 5.0 against 6.4; 5001 rows of 33 entries: 6.6 against
+//     6.8), so from 192K entries for rows of 16 or more (banded 5999 x 33 INT16 7.6 -> 6.6, 20999
+//     x 33 FP32 9.8 -> 6.8, 199999 x 33 23.7 -> 14.2) and from 1M for shorter ones (5-point
+//     stencil 700^2 FP32 15.3 -> 11.4, 1400^2 58 -> 26)
+//   rows made of aligned four-column runs keep their four-value x loads (the caller's check)
+// Shape: scattered columns (over 0.3 lines per entry in row order; R-MAT 0.84, banded and
+// stencils up to 0.2) want the widest tile once it leaves enough of them (R-MAT 2^20: 74.8 with
+// 4096 entries, 66.4 with 8192, 62.1 with 16384; uniform INT8 9.9M entries: 29.5, 22.9, 23.0;
+// but 2.9M entries INT16: 13.8 with 4096, 16.4 with 16384); local ones 16 entries per thread in
+// the smallest workgroup (199999 x 33 FP32: 14.2 with 256 threads, 16.4 with 1024), 8-byte sums
+// 8 per thread (20.1 against 24.3).
+WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
+    const sp_opts &o = p->opts;
+    // any knob asked for keeps its kernel; a memory cap keeps one copy of the matrix
+    if (p->algo != SP_ALGO_AUTO || o.items_per_lane || o.lanes_per_row || o.nparts || o.nsub || o.lds_slice ||
+        o.mem_cap_bytes)
+        return {};
+    const uint32_t least = coo || skewed ? 32u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
+    if (nnz < least) return {};
+    const bool scattered = row_lines(colind, nnz, sp_dtype_size(p->dtype)) > 0.3;
+    if (acc_size(p->dtype) == 8) return scattered && nnz >= 2u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
+    if (scattered && nnz >= 3u << 20) return {1024, 16};
+    return !scattered && nnz >= 1u << 20 ? WideShape{256, 16} : WideShape{512, 8};
+}
+
+// Gives a plan whose row-ordered group is built (one problem) wide tiles for one right-hand
+// side; the row-ordered group stays for several.  SP_ERR_RANGE: not a matrix for wide tiles
+// (columns of a tile too far apart, or one tile with most of the matrix's empty rows).
+int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
+    const size_t sv = sp_dtype_size(p->dtype), sa = acc_size(p->dtype);
+    Prob P = p->h_probs[0];
+    const uint32_t words = s.nt * s.ipt, nnz = P.nent;
+    uint32_t pb = 0;
+    while ((1u << pb) < words) pb++;
+    const uint32_t tile = P.ncols_elem <= (1ull << (32 - pb)) ? words : words - 256;  // entries per tile
+    const uint32_t nt = (uint32_t)(((uint64_t)nnz + tile - 1) / tile);
+    const uint64_t tot = (uint64_t)nt * words;
+    // the word of every thread, every row's sum, the first row of each tile's rows (those that end
+    // in it and the empty ones after each), the row it carries out
+    std::vector<uint32_t> word((size_t)nt * s.nt, 0), cent, crow, carry(nt + 1, spd::NONE);
+    std::vector<uint16_t> rmap(P.nrows, 0);
+    crow.push_back(0);
+    for (uint32_t i = 0, ord = 0; i < P.nrows; i++) {
+        if (rowptr[i + 1] == rowptr[i]) continue;
+        const uint32_t e = rowptr[i + 1] - 1, t = e / tile, at = e % tile;
+        while (crow.size() <= t) {  // row i is the first that ends in tile t
+            crow.push_back(i);
+            ord = 0;
+        }
+        uint32_t &w = word[(size_t)t * s.nt + at / s.ipt];
+        w |= 1u << (at % s.ipt);
+        rmap[i] = (uint16_t)++ord;
+        for (uint32_t q = rowptr[i] / tile; q < t; q++) carry[q] = i;
+    }
+    while (crow.size() <= nt) crow.push_back(P.nrows);
+    crow[nt] = P.nrows;
+    for (uint32_t t = 0; t < nt; t++) {
+        if (crow[t + 1] - crow[t] > 16 * tile) return SP_ERR_RANGE;
+        cent.push_back(t * tile);
+        uint32_t ord = 0;
+        for (size_t k = (size_t)t * s.nt; k < (size_t)(t + 1) * s.nt; k++) {
+            const uint32_t m = word[k];
+            word[k] = ord << 16 | m;
+            ord += (uint32_t)__builtin_popcount(m);
+        }
+    }
+    cent.push_back(nnz);
+    int rc;
+    void *key, *val, *base, *drmap, *dword, *flag;
+    if ((rc = plan_alloc(p, tot * 4, &key)) || (rc = plan_alloc(p, tot * sv, &val)) ||
+        (rc = plan_alloc(p, tot / 64 * 4, &base)) || (rc = plan_alloc(p, 4, &flag)) ||
+        (rc = plan_upload(p, rmap.data(), rmap.size() * 2, &drmap)) ||
+        (rc = plan_upload(p, word.data(), word.size() * 4, &dword)))
+        return rc;
+    // on the null stream, as the uploads before it
+    if ((rc = launch_wide_sort(nullptr, P.cind, P.val, sv, nnz, tile, words, pb, s.ipt, sa, (uint32_t *)key, val,
+                               (uint32_t *)base, (uint32_t *)flag)))
+        return rc;
+    P.ptr = (const uint32_t *)dword;
+    P.rind = (const uint32_t *)drmap;
+    P.cind = (const uint32_t *)key;
+    P.val = val;
+    P.hcol = (const uint32_t *)base;
+    P.nhcol = tile;
+    P.pbits = pb;
+    p->many = std::make_unique<PlanWork>(std::move(*static_cast<PlanWork *>(p)));
+    static_cast<PlanWork &>(*p) = PlanWork{};
+    Builder b(p);
+    b.add(P, cent, &crow, &carry);
+    p->work.lanes = s.nt;
+    p->work.ipt = s.ipt;
+    p->algo = SP_ALGO_SEGMENTED_SORTED;
+    p->lanes = 0;
+    p->ipt = words / TPB;
+    p->ntiles = nt;
+    p->nsub = s.nt;
+    return b.finish(WK_WIDE, true, 1);
+}
+
+// Undoes a plan's groups (a wide layout that did not fit).
+void drop_groups(sp_plan *p, const sp_opts &opts, int algo) {
+    for (void *d : p->allocs) (void)hipFree(d);
+    p->allocs.clear();
+    p->device_bytes = 0;
+    p->many.reset();
+    static_cast<PlanWork &>(*p) = PlanWork{};
+    p->opts = opts;
+    p->algo = algo;
+}
+
 bool coo_sorted(const sp_coo *A) {
     for (uint32_t k = 1; k < A->nnz; k++) {
         if (A->rowind[k] < A->rowind[k - 1]) return false;
@@ -353,7 +495,8 @@ bool coo_sorted(const sp_coo *A) {
 // ---------------------------------------------------------------------------
 // CSR (ids 0, 1)
 // ---------------------------------------------------------------------------
-int build_csr_plan(sp_plan *p, const sp_csr *A) {
+// With `wide`, a plan that takes wide tiles gets its row-ordered group here and the shape in *wide.
+static int build_csr_group(sp_plan *p, const sp_csr *A, WideShape *wide) {
     const size_t sv = sp_dtype_size(A->dtype);
     if (!A->rowptr || (A->nnz && (!A->colind || !A->values))) return SP_ERR_ARG;
     if (A->rowptr[0] != 0 || A->rowptr[A->nrows] != A->nnz) return SP_ERR_ARG;
@@ -365,6 +508,8 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
         uint32_t maxlen = 0;
         for (uint32_t i = 0; i < A->nrows; i++) maxlen = std::max(maxlen, A->rowptr[i + 1] - A->rowptr[i]);
         const double avg = A->nrows ? (double)A->nnz / A->nrows : 0.0;
+        if (wide && !quad_rows(A->rowptr, A->nrows, A->colind, A->nnz, A->ncols))
+            *wide = wide_shape(p, false, maxlen > 4 * avg + 64, A->colind, A->nrows, A->nnz);
         // Row-granular kernel for even row lengths up to a few million entries (one launch,
         // no carries); the merge-path kernel for skewed rows, and for large matrices, where
         // its deeper per-thread load batches win (27-point stencil, 113M entries: 1.3x).
@@ -389,7 +534,7 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
             const uint32_t I = pick_ipt(p->opts, 8);
             uint32_t pb = 0;
             while (I && (1u << pb) < TPB * I) pb++;
-            if (I && A->ncols <= (1ull << (32 - pb))) p->algo = SP_ALGO_SEGMENTED_SORTED;
+            if (I && A->ncols <= (1ull << (32 - pb)) && !(wide && wide->nt)) p->algo = SP_ALGO_SEGMENTED_SORTED;
         }
     }
     Prob P{};
@@ -502,10 +647,23 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     return b.finish(WK_CSR_MERGE, true, 1);
 }
 
+int build_csr_plan(sp_plan *p, const sp_csr *A) {
+    const sp_opts opts = p->opts;
+    const int algo = p->algo;
+    WideShape s;
+    int rc = build_csr_group(p, A, &s);
+    if (rc || !s.nt) return rc;
+    rc = add_wide(p, A->rowptr, s);
+    if (rc != SP_ERR_RANGE) return rc;
+    drop_groups(p, opts, algo);
+    return build_csr_group(p, A, nullptr);
+}
+
 // ---------------------------------------------------------------------------
 // COO (ids 2, 3, 4)
 // ---------------------------------------------------------------------------
-int build_coo_plan(sp_plan *p, const sp_coo *A0) {
+// (As build_csr_group; the row pointers go to *rowptr.)
+static int build_coo_group(sp_plan *p, const sp_coo *A0, WideShape *wide, std::vector<uint32_t> &rowptr) {
     const sp_coo *A = A0;
     sp_coo *sorted = nullptr;
     for (uint32_t k = 0; k < A0->nnz; k++)
@@ -521,7 +679,7 @@ int build_coo_plan(sp_plan *p, const sp_coo *A0) {
     }
     const size_t sv = sp_dtype_size(A->dtype);
     const uint32_t n = A->nrows, nnz = A->nnz;
-    std::vector<uint32_t> rowptr(n + 1, 0);
+    rowptr.assign((size_t)n + 1, 0);
     for (uint32_t k = 0; k < nnz; k++) rowptr[A->rowind[k] + 1]++;
     for (uint32_t i = 0; i < n; i++) rowptr[i + 1] += rowptr[i];
     Prob P{};
@@ -533,19 +691,21 @@ int build_coo_plan(sp_plan *p, const sp_coo *A0) {
         P.nrows = P.nrows_elem = n;
         P.nent = nnz;
         P.ncols_elem = A->ncols;
-        // 4 items per lane, the tuner's usual winner for 1D COO; skewed rows and more than 8M
-        // entries take 4096-entry tiles (16, run as 512 x 8: R-MAT 2^20 86 vs 109 us), as for CSR
         uint32_t maxlen = 0;
         for (uint32_t i = 0; i < n; i++) maxlen = std::max(maxlen, rowptr[i + 1] - rowptr[i]);
-        if (p->opts.items_per_lane == 0 && maxlen > 4.0 * nnz / std::max(n, 1u) + 64 && nnz > (8u << 20) &&
-            A->ncols <= (1u << 20) && p->algo != SP_ALGO_SEGMENTED)  // column-ordered 4096-entry tiles only
-            p->opts.items_per_lane = 16;
         // rows made of aligned runs of four columns: row-ordered chunk tiles reading x four
         // values per load (unless column order is asked for, or atomics), 8 items per lane
         // (27-point stencil 64^3 x 4: FP32 295-297 us against 363-366 us at 4 and 360 us for
         // column-ordered tiles; FP64 401-408 against 446-456 and 437-441 us)
         const bool quads = !atom && !p->opts.lds_slice && p->algo != SP_ALGO_SEGMENTED_SORTED &&
                            quad_rows(rowptr.data(), n, A->colind, nnz, A->ncols);
+        if (wide && !quads)
+            *wide = wide_shape(p, true, maxlen > 4.0 * nnz / std::max(n, 1u) + 64, A->colind, n, nnz);
+        // 4 items per lane, the tuner's usual winner for 1D COO; skewed rows and more than 8M
+        // entries take 4096-entry tiles (16, run as 512 x 8: R-MAT 2^20 86 vs 109 us), as for CSR
+        if (p->opts.items_per_lane == 0 && maxlen > 4.0 * nnz / std::max(n, 1u) + 64 && nnz > (8u << 20) &&
+            A->ncols <= (1u << 20) && p->algo != SP_ALGO_SEGMENTED)  // column-ordered 4096-entry tiles only
+            p->opts.items_per_lane = 16;
         const uint32_t I = pick_ipt(p->opts, quads ? 8 : 4);
         if (!I) { rc = SP_ERR_ARG; break; }
         p->ipt = p->work.ipt = I;
@@ -555,7 +715,7 @@ int build_coo_plan(sp_plan *p, const sp_coo *A0) {
         uint32_t pb = 0;
         while ((1u << pb) < tile) pb++;
         bool col_order = p->algo != SP_ALGO_SEGMENTED && A->ncols <= (1ull << (32 - pb));
-        if (quads) col_order = false;
+        if (quads || (wide && wide->nt)) col_order = false;  // (wide tiles: the row-ordered group)
         const uint32_t P1 = p->opts.nparts ? p->opts.nparts : 1;
         // part entry ranges
         std::vector<uint32_t> pe0(P1), pe1(P1);
@@ -630,6 +790,19 @@ int build_coo_plan(sp_plan *p, const sp_coo *A0) {
     } while (0);
     if (sorted) sp_free_coo(sorted);
     return rc;
+}
+
+int build_coo_plan(sp_plan *p, const sp_coo *A) {
+    const sp_opts opts = p->opts;
+    const int algo = p->algo;
+    WideShape s;
+    std::vector<uint32_t> rowptr;
+    int rc = build_coo_group(p, A, &s, rowptr);
+    if (rc || !s.nt) return rc;
+    rc = add_wide(p, rowptr.data(), s);
+    if (rc != SP_ERR_RANGE) return rc;
+    drop_groups(p, opts, algo);
+    return build_coo_group(p, A, nullptr, rowptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -806,7 +979,7 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
 // ---------------------------------------------------------------------------
 int run_plan(sp_plan *p, const void *x, void *y, int k, int ldx, int ldy) {
     if (p->nrows == 0) return SP_OK;
-    if (!p->tiled) return run_work(p->work, p->ctx, x, y, nullptr, nullptr, k, ldx, ldy);
+    if (!p->tiled) return run_work(p->group(k).work, p->ctx, x, y, nullptr, nullptr, k, ldx, ldy);
     // 2D: partial rows per stripe into ypart, then the stripe-order reduction.
     const uint64_t need = (uint64_t)p->vert * p->nrows * (uint64_t)k * sp_dtype_size(p->dtype);
     if (need > p->ypart_bytes) {

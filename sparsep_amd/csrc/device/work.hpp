@@ -12,7 +12,7 @@
 struct sp_ctx;
 
 enum WorkKind { WK_CSR_MERGE = 0, WK_CSR_VEC = 1, WK_COO_SEG = 2, WK_BCSR_VEC = 3, WK_BCOO_SEG = 4, WK_CSR_HOT = 5,
-               WK_BCSR_SEG = 6 };
+               WK_BCSR_SEG = 6, WK_WIDE = 7 };
 
 struct Work {
     int kind = WK_CSR_MERGE;
@@ -21,9 +21,10 @@ struct Work {
     spd::Prob *d_prob = nullptr;
     uint32_t *d_unit_pid = nullptr;
     uint32_t *d_c0 = nullptr, *d_c1 = nullptr;  // coordinates, index unit + pid
-    uint32_t *d_c2 = nullptr;                   // hot-x CSR: staged entries per tile, index unit + pid
+    uint32_t *d_c2 = nullptr;                   // hot-x CSR: staged entries per tile; wide tiles: row
+                                                // carried out (NONE: none); index unit + pid
     uint32_t hcol_max = 0;                      // hot-x CSR: largest staged-column count of the problems
-    uint32_t ipt = 8, lanes = 1, R = 1, C = 1;
+    uint32_t ipt = 8, lanes = 1, R = 1, C = 1;  // (wide tiles: lanes = threads per workgroup)
     uint32_t *d_carry_row = nullptr;
     void *d_carry_val = nullptr;
     uint32_t carry_k = 0;  // right-hand sides the carry buffer holds
@@ -62,6 +63,7 @@ inline int max_rhs_chunk(const Work &w) {
     case WK_BCOO_SEG: return 1;
     case WK_BCSR_SEG: return 1;
     case WK_CSR_HOT: return 1;
+    case WK_WIDE: return 1;  // (plans with wide tiles keep a row-ordered work for several right-hand sides)
     default: return 8;
     }
 }
@@ -76,6 +78,11 @@ template <typename T>
 int run_work_t(const Work &w, sp_ctx *ctx, const void *xb, void *yb, const uintptr_t *xtab,
                const uintptr_t *ytab, int k, int ldx, int ldy);
 
+// Whether a kind leaves carries of rows that cross units to the fix-up.
+inline bool has_carries(int kind) {
+    return kind == WK_CSR_MERGE || kind == WK_COO_SEG || kind == WK_BCOO_SEG || kind == WK_CSR_HOT || kind == WK_BCSR_SEG ||
+           kind == WK_WIDE;
+}
 extern template int run_work_t<int8_t>(const Work &, sp_ctx *, const void *, void *, const uintptr_t *,
                                        const uintptr_t *, int, int, int);
 extern template int run_work_t<int16_t>(const Work &, sp_ctx *, const void *, void *, const uintptr_t *,
@@ -88,6 +95,11 @@ extern template int run_work_t<float>(const Work &, sp_ctx *, const void *, void
                                       const uintptr_t *, int, int, int);
 extern template int run_work_t<double>(const Work &, sp_ctx *, const void *, void *, const uintptr_t *,
                                        const uintptr_t *, int, int, int);
+
+// The rows that cross units of a group, as runs in unit order, where the plan knows which row
+// each unit carries: CSR merge tiles (the row at the end coordinate) and wide tiles (c2).
+std::vector<spd::Run> crossing_runs(int kind, const std::vector<spd::Prob> &probs, const std::vector<uint32_t> &unit_pid,
+                                    const std::vector<uint32_t> &c0, const std::vector<uint32_t> &c2);
 
 // Host view of one sub-problem while a Work is being built.
 struct HostProb {
