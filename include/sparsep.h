@@ -413,7 +413,11 @@ typedef enum sp_algo {
      * row order in LDS, giving the same sums in the same order.  1D CSR
      * and COO ids (0-4); needs ncols <= 2^32 / (256 * items_per_lane).
      * AUTO takes it in place of SEGMENTED wherever the columns fit (COO:
-     * any algo but SEGMENTED does). */
+     * any algo but SEGMENTED does).  AUTO with no other knob and no memory
+     * cap (CSR and COO ids, from a few thousand entries on) takes wide tiles
+     * for one right-hand side, of 2048 to 16384 entries whatever the column
+     * count: sums in a fixed order of their own, and a second copy of the
+     * matrix in row order for several right-hand sides. */
     SP_ALGO_SEGMENTED_SORTED = 3,
     /* SEGMENTED_SORTED with the most frequent columns' x entries staged in
      * LDS (up to 112 KB; 96 KB for 8-byte accumulators): one 1024-thread

@@ -123,6 +123,7 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
     struct Acc {
         std::vector<spd::Prob> probs;
         std::vector<uint32_t> unit_pid, c0, c1, c2, zpid, zrow;
+        std::vector<spd::Cross> cross;
     };
     std::vector<Acc> acc;
     for (int i = 0; i < nprob; i++) {
@@ -170,6 +171,21 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
                 a.probs.push_back(P);
                 g.slots.push_back({(uint32_t)i, P0.xoff * k[i] + done, P0.yoff * k[i] + done});
             }
+            if (w.kind == WK_PANEL) {  // (one problem) units and crossing rows at this width
+                const uint32_t E = spd::panel_entries(kc, (dt == SP_I64 || dt == SP_F64) ? 8 : 4), nent = pw.h_probs[0].nent;
+                for (spd::Cross C : pw.h_cross)
+                    if (C.b / E != C.e / E) {
+                        C.pid = pid0;
+                        C.ldy = k[i];
+                        C.unit0 = (uint32_t)a.unit_pid.size();
+                        a.cross.push_back(C);
+                    }
+                for (uint64_t e = 0; e < nent; e += E) {
+                    a.unit_pid.push_back(pid0);
+                    a.c0.push_back((uint32_t)e);
+                }
+                a.c0.push_back(nent);
+            }
             for (uint32_t u : pw.h_unit_pid) a.unit_pid.push_back(u + pid0);
             a.c0.insert(a.c0.end(), pw.h_c0.begin(), pw.h_c0.end());
             a.c1.insert(a.c1.end(), pw.h_c1.begin(), pw.h_c1.end());
@@ -216,6 +232,11 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
             if ((rc = balloc(b, n * 4, (void **)&w.d_carry_row))) break;
             if ((rc = balloc(b, n * g.kc * asz, &w.d_carry_val))) break;
         }
+        if (w.kind == WK_PANEL) {
+            const int ki = __builtin_ctz((unsigned)g.kc);
+            w.ncross[ki] = (uint32_t)a.cross.size();
+            if ((rc = bupload(b, a.cross, &w.d_cross[ki]))) break;
+        }
         if (((w.kind == WK_CSR_MERGE && !w.nzero) || w.kind == WK_WIDE) && w.nunits) {
             // the rows crossing tiles as runs, as a single plan lists them: each run's carries
             // are added with independent loads instead of a walk over the units that stops at
@@ -243,7 +264,12 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
         const size_t nbr = std::min(kBranches, b->groups.size());
         std::vector<size_t> order(b->groups.size());
         for (size_t gi = 0; gi < order.size(); gi++) order[gi] = gi;
-        auto work = [&](size_t gi) { return (uint64_t)b->groups[gi].w.nunits * (uint64_t)b->groups[gi].kc; };
+        // an entry's column and value, and its row of x: units hold different amounts of work
+        auto work = [&](size_t gi) {
+            uint64_t n = 0;
+            for (const spd::Prob &P : acc[gi].probs) n += (uint64_t)P.nent * std::max(b->groups[gi].w.R * b->groups[gi].w.C, 1u);
+            return n * (uint64_t)(2 + b->groups[gi].kc);
+        };
         std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t c) { return work(a) > work(c); });
         std::vector<uint64_t> load(nbr, 0);
         b->group_branch.assign(b->groups.size(), 0);

@@ -46,7 +46,8 @@ struct Prob {
     int32_t ldx, ldy;      // leading dimensions when x / y come from pointer tables
     uint32_t pbits;        // CSR merge tiles in column order: cind holds col << pbits | position in tile
     uint32_t nhcol;        // hot-x CSR: number of staged ("hot") columns; wide tiles: entries per tile
-    const uint32_t *hcol;  // hot-x CSR: the staged columns, slot order; wide tiles: base column per 64 words
+    const uint32_t *hcol;  // hot-x CSR: the staged columns, slot order; wide tiles: base column per 64 words;
+                           // panels: the rows without entries (nhcol of them)
     void *xh;              // hot-x CSR: x at the staged columns, written before each launch
 };
 
@@ -753,6 +754,182 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void wi
 #pragma unroll
         for (int i = 0; i < 8; i++)
             if (k0 + i * NT < nr) y[(size_t)(r0 + k0 + i * NT) * ldy] = m[i] ? to_val<T>(s_buf[m[i] - 1]) : T(0);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// CSR and COO with uneven rows, K = 1 .. 32 right-hand sides in one pass, entry
+// balanced.  A workgroup takes E consecutive entries in row order.  The lanes
+// of an entry read its x row in whole pieces of up to 16 bytes (LPE lanes per
+// entry, neighbouring lanes neighbouring pieces), so a cache line of x is
+// requested once per entry and not once per piece, and put the products into
+// LDS (16 KB whatever K: E = 4096 / K, half with 8-byte sums).  Thread (g, q)
+// then runs over the GE consecutive entries of group g for column q; one word
+// pair per 32 entries (P.ptr) says which of them end a row and how many rows
+// end before them, and the sums are joined over groups and waves as in
+// wide_kernel.  P.rind lists the rows with entries; those without (P.hcol,
+// P.nhcol of them) are zeroed in even shares by all workgroups.  Open ends are
+// carries for panel_fixup_kernel.
+// ---------------------------------------------------------------------------
+template <typename T, int K> struct Panel {
+    using A = acc_t<T>;
+    static constexpr int GE = 64 / (int)sizeof(A);        // entries per group: 16, or 8 with 8-byte sums
+    static constexpr int G = TPB / K;                     // groups
+    static constexpr int E = G * GE;                      // entries per workgroup
+    static constexpr int V = K * (int)sizeof(T) < 16 ? K : 16 / (int)sizeof(T);  // values per piece
+    static constexpr int LPE = K / V;                     // lanes per entry
+    // LDS place of entry e: groups whose threads share a wave read different banks
+    static constexpr int SW = (WAVE / K < GE ? WAVE / K : GE) - 1;
+    __device__ static __forceinline__ uint32_t slot(uint32_t e) { return e ^ ((e / GE) & SW); }
+};
+// Entries per workgroup for k right-hand sides and sa-byte sums (Panel<T, k>::E).
+inline uint32_t panel_entries(int k, size_t sa) { return (uint32_t)(TPB / k) * (64 / (uint32_t)sa); }
+
+template <typename T, int K>
+__global__ __launch_bounds__(TPB) void panel_kernel(const Prob *__restrict__ probs, const uint32_t *__restrict__ unit_pid,
+                                                    const uint32_t *__restrict__ cent, Ptrs<T> io,
+                                                    acc_t<T> *__restrict__ carry_val) {
+    using A = acc_t<T>;
+    using PN = Panel<T, K>;
+    constexpr int GE = PN::GE, E = PN::E, V = PN::V, LPE = PN::LPE, NW = TPB / WAVE, EPW = WAVE / LPE;
+    constexpr int STEPS = E / (NW * EPW), U = STEPS < 4 ? STEPS : 4;
+    static_assert(STEPS >= 1 && STEPS % U == 0, "whole steps");
+    typedef T TV __attribute__((ext_vector_type(V)));
+    __shared__ __align__(16) A s_buf[E * K];
+    __shared__ A s_wv[NW][K];
+    __shared__ uint32_t s_wf[NW];
+    const int tid = threadIdx.x, lane = tid % WAVE, wid = tid / WAVE;
+    const uint32_t t = blockIdx.x;
+    // one problem: tile t starts at entry t E; several: the unit tables
+    const uint32_t pid = unit_pid ? unit_pid[t] : 0u;
+    const Prob P = probs[pid];
+    const uint32_t j0 = cent ? cent[t + pid] : t * (uint32_t)E, nb = min((uint32_t)E, P.nent - j0);
+    const gptr<const T> __restrict__ x = gp(io.x(pid, P));
+    const gptr<T> __restrict__ y = gp(io.y(pid, P));
+    const gptr<const uint32_t> __restrict__ ci = gp(P.cind) + j0, rows = gp(P.rind), zrow = gp(P.hcol);
+    const gptr<const u32x2> __restrict__ words = (gptr<const u32x2>)gp(P.ptr);
+    const gptr<const T> __restrict__ va = gp((const T *)P.val) + j0;
+    const int ldx = io.lx(P), ldy = io.ly(P);
+    const int g = tid / K, q = tid % K;
+    const u32x2 word = words[(j0 + min((uint32_t)(g * GE), nb - 1)) / 32];
+    const uint32_t s0 = words[j0 / 32].y, s1 = words[min((j0 + (uint32_t)E) / 32, (P.nent + 31) / 32)].y;
+
+    const int el = lane / LPE, r = lane % LPE;
+    auto products = [&](auto wide_c) {
+        constexpr bool WIDE = decltype(wide_c)::value;  // whole pieces of x in one load
+#pragma unroll 1
+        for (int st = 0; st < STEPS; st += U) {
+            uint32_t c[U];
+            T v[U];
+            TV xv[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {  // past the tile's end: its last entry again, in places that nothing reads
+                const uint32_t e = min((uint32_t)(((st + u) * NW + wid) * EPW + el), nb - 1);
+                c[u] = ldg(ci + e);
+                v[u] = ldg(va + e);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const gptr<const T> px = x + (size_t)c[u] * ldx + V * r;
+                if constexpr (WIDE) {
+                    xv[u] = *(gptr<const TV>)px;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < V; i++) xv[u][i] = px[i];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                A *const d = s_buf + PN::slot(((st + u) * NW + wid) * EPW + el) * K + V * r;
+                A pr[V];
+#pragma unroll
+                for (int i = 0; i < V; i++) pr[i] = mul<T>(v[u], xv[u][i]);
+                if constexpr (V * sizeof(A) >= 16) {
+#pragma unroll
+                    for (int i = 0; i < V * (int)sizeof(A) / 16; i++) {
+                        u32x4 w;
+                        __builtin_memcpy(&w, (const char *)pr + 16 * i, 16);
+                        ((u32x4 *)d)[i] = w;
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < V; i++) d[i] = pr[i];
+                }
+            }
+        }
+    };
+    if ((uintptr_t)io.x(pid, P) % sizeof(TV) == 0 && ldx * sizeof(T) % sizeof(TV) == 0) products(std::true_type{});
+    else products(std::false_type{});
+    __syncthreads();
+
+    // running sums of this thread's column over its group, starting anew after each row end
+    const uint32_t sh = (uint32_t)(g * GE) % 32;  // the group's place in its word
+    const uint32_t mask = (uint32_t)(g * GE) < nb ? word.x >> sh & ((1u << GE) - 1) : 0u;
+    const uint32_t ord = word.y + (uint32_t)__builtin_popcount(word.x & ((1u << sh) - 1));
+    A p[GE];
+#pragma unroll
+    for (int s = 0; s < GE; s++) p[s] = s_buf[PN::slot(g * GE + s) * K + q];
+#pragma unroll
+    for (int s = 1; s < GE; s++) p[s] = (mask >> (s - 1) & 1) ? p[s] : p[s - 1] + p[s];
+    A v = (mask >> (GE - 1) & 1) ? A(0) : p[GE - 1];
+    const uint64_t ends = __ballot(mask != 0), upto = ends & ((2ull << lane) - 1);
+    const int from = upto ? (63 - __builtin_clzll(upto)) / K * K + q : 0;  // lane of the last group with an end
+#pragma unroll
+    for (int off = K; off < WAVE; off <<= 1) {
+        const A ov = shfl_up_any(v, off);
+        if (lane - off >= from) v = ov + v;
+    }
+    if (lane >= WAVE - K) s_wv[wid][q] = v;
+    if (lane == 0) s_wf[wid] = ends != 0;
+    __syncthreads();
+    A cross = A(0);  // the open end of the waves before
+    for (int w = wid - 1; w >= 0; w--) {
+        cross = s_wv[w][q] + cross;
+        if (s_wf[w]) break;
+    }
+    const A pv = shfl_up_any(v, K);
+    A cin = lane >= K ? pv : A(0);
+    if (!(ends & ((1ull << (lane - q)) - 1))) cin = cross + cin;
+    uint32_t o = ord - s0;
+#pragma unroll
+    for (int s = 0; s < GE; s++)
+        if (mask >> s & 1) {
+            s_buf[o++ * K + q] = cin + p[s];
+            cin = A(0);
+        }
+    if ((uint32_t)g == (nb - 1) / GE) carry_val[(size_t)t * K + q] = upto ? v : cross + v;
+    __syncthreads();
+
+    for (uint32_t i = tid; i < (s1 - s0) * K; i += TPB) y[(size_t)rows[s0 + i / K] * ldy + i % K] = to_val<T>(s_buf[i]);
+    const uint32_t tl = j0 / E, nt = (P.nent + E - 1) / E;
+    const uint32_t z0 = (uint32_t)((uint64_t)P.nhcol * tl / nt), z1 = (uint32_t)((uint64_t)P.nhcol * (tl + 1) / nt);
+    for (uint32_t i = tid; i < (z1 - z0) * K; i += TPB) y[(size_t)zrow[z0 + i / K] * ldy + i % K] = T(0);
+}
+
+// Adds the carries of the rows that cross workgroups of panel_kernel, a wave
+// per row: lanes over its workgroups and columns, then a butterfly.
+struct Cross {
+    uint32_t pid, row, b, e;  // problem, row, its first and last entry
+    int64_t yel;              // P.yoff + row (no pointer tables)
+    int32_t ldy;              // P.ldy (pointer tables)
+    uint32_t unit0;           // first unit of the problem
+};
+
+template <typename T, int K>
+__global__ __launch_bounds__(TPB) void panel_fixup_kernel(const Cross *__restrict__ cross, uint32_t n,
+                                                          const acc_t<T> *__restrict__ carry_val, Ptrs<T> io) {
+    using A = acc_t<T>;
+    constexpr uint32_t E = Panel<T, K>::E;
+    const uint32_t j = blockIdx.x * (TPB / WAVE) + threadIdx.x / WAVE;
+    if (j >= n) return;
+    const Cross C = cross[j];
+    const int lane = threadIdx.x % WAVE, q = lane % K;
+    A v = A(0);
+    for (uint32_t u = C.b / E + lane / K; u < C.e / E; u += WAVE / K) v = v + carry_val[(size_t)(C.unit0 + u) * K + q];
+    v = xor_sum<K, WAVE>(v);
+    if (lane < K) {
+        const gptr<T> yp = io.ytab ? gp((T *)io.ytab[C.pid] + io.q0) + (size_t)C.row * C.ldy : gp(io.yb) + C.yel * io.ldy;
+        yp[q] = to_val<T>((A)yp[q] + v);
     }
 }
 

@@ -15,6 +15,13 @@ static int launch_main(const Work &w, hipStream_t s, Ptrs<T> io) {
     using A = acc_t<T>;
     const dim3 grid(w.grid_cap && w.grid_cap < w.nunits ? w.grid_cap : w.nunits), block(TPB);
     A *cv = (A *)w.d_carry_val;
+    if (w.kind == WK_PANEL) {
+        constexpr uint32_t E = Panel<T, K>::E;
+        const uint32_t units = w.panel_nent ? (w.panel_nent + E - 1) / E : w.nunits;
+        hipLaunchKernelGGL((panel_kernel<T, K>), dim3(units), block, 0, s, w.d_prob, w.panel_nent ? nullptr : w.d_unit_pid,
+                           w.panel_nent ? nullptr : w.d_c0, io, cv);
+        return hipGetLastError() == hipSuccess ? SP_OK : SP_ERR_HIP;
+    }
     if constexpr (K > 8) {
         // wide chunks: row-granular kernels only (no carries, no LDS staging)
         if (w.kind == WK_CSR_VEC) {
@@ -309,6 +316,16 @@ static int launch_chunk(const Work &w, sp_ctx *ctx, Ptrs<T> io) {
         if (rc) return rc;
     }
     mark_dominant(ctx);
+    if (w.kind == WK_PANEL) {
+        using A = acc_t<T>;
+        const int i = __builtin_ctz(K);
+        if (w.ncross[i]) {
+            hipLaunchKernelGGL((panel_fixup_kernel<T, K>), dim3((w.ncross[i] + TPB / WAVE - 1) / (TPB / WAVE)), dim3(TPB), 0, s,
+                               w.d_cross[i], w.ncross[i], (const A *)w.d_carry_val, io);
+            if (hipGetLastError() != hipSuccess) return SP_ERR_HIP;
+        }
+        return SP_OK;
+    }
     if (w.d_runs) {  // CSR merge and wide tiles with their run list
         if (w.nruns) {
             using A = acc_t<T>;

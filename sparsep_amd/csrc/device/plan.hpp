@@ -38,6 +38,7 @@ struct PlanWork {
     Work work;
     std::vector<spd::Prob> h_probs;
     std::vector<uint32_t> h_unit_pid, h_c0, h_c1, h_c2, h_zpid, h_zrow;
+    std::vector<spd::Cross> h_cross;  // panels: the rows that cross workgroups at the widest panel
 };
 
 struct sp_plan : PlanWork {  // (the base: the main launch group)
@@ -51,7 +52,8 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
     uint32_t nparts = 0, nsub = 0, lanes = 0, ipt = 0, vert = 0, ntiles = 0;
     uint32_t launches = 1;
 
-    // wide tiles take one right-hand side: several run on this row-ordered group
+    // wide tiles take one right-hand side: several run on this group (even CSR rows: the row
+    // kernels; otherwise panels)
     std::unique_ptr<PlanWork> many;
     // the group that a call with k right-hand sides runs
     const PlanWork &group(int k) const {

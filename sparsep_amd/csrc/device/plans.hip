@@ -368,7 +368,7 @@ double row_lines(const uint32_t *colind, uint32_t nnz, size_t sv) {
 
 // Whether an automatic 1D CSR/COO plan takes wide tiles, and which.  Against the kernels that
 // the row-ordered group would take (us per SpMV, before -> wide):
-//   skewed rows and COO from 32K entries on: R-MAT 2^12 x 8 FP32 CSR 8.4 -> 6.5, 2^16 x 16
+//   skewed rows and COO from 2K entries on: R-MAT 2^12 x 8 FP32 CSR 8.4 -> 6.5, 2^16 x 16
 //     11.0 -> 8.2, 2^18 x 16 FP64 28.8 -> 22.7, 2^20 x 16 FP32 72.6 -> 62.1; COO 5-point stencil
 //     700^2 14.2 -> 9.6
 //   even rows: their single launch needs no fix-up, which decides small matrices (5-point
@@ -389,7 +389,7 @@ WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *co
     if (p->algo != SP_ALGO_AUTO || o.items_per_lane || o.lanes_per_row || o.nparts || o.nsub || o.lds_slice ||
         o.mem_cap_bytes)
         return {};
-    const uint32_t least = coo || skewed ? 32u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
+    const uint32_t least = coo || skewed ? 2u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
     if (nnz < least) return {};
     const bool scattered = row_lines(colind, nnz, sp_dtype_size(p->dtype)) > 0.3;
     if (acc_size(p->dtype) == 8) return scattered && nnz >= 2u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
@@ -397,8 +397,69 @@ WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *co
     return !scattered && nnz >= 1u << 20 ? WideShape{256, 16} : WideShape{512, 8};
 }
 
+// Makes a row-ordered CSR or COO group (one problem) the group for several right-hand sides with
+// uneven rows: panels over the same columns and values.
+int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
+    const size_t sa = acc_size(p->dtype);
+    Prob P = g.h_probs[0];
+    const uint32_t nnz = P.nent, nw = (uint32_t)(((uint64_t)nnz + 31) / 32), emin = spd::panel_entries(32, sa);
+    std::vector<uint32_t> word(2 * ((size_t)nw + 1), 0), rows, zrows;
+    std::vector<spd::Cross> cross;
+    for (uint32_t i = 0; i < P.nrows; i++) {
+        if (rowptr[i + 1] == rowptr[i]) {
+            zrows.push_back(i);
+            continue;
+        }
+        const uint32_t b = rowptr[i], e = rowptr[i + 1] - 1;
+        word[2 * (size_t)(e / 32)] |= 1u << (e % 32);
+        rows.push_back(i);
+        if (b / emin != e / emin) cross.push_back(spd::Cross{0, i, b, e, (int64_t)i, P.ldy, 0});
+    }
+    for (uint32_t w = 0, n = 0; w <= nw; w++) {  // (the closing pair: all rows)
+        word[2 * (size_t)w + 1] = n;
+        n += (uint32_t)__builtin_popcount(word[2 * (size_t)w]);
+    }
+    g = PlanWork{};
+    g.work.kind = WK_PANEL;
+    g.work.dtype = p->dtype;
+    g.work.nprob = g.work.nunits = 1;
+    g.work.panel_nent = nnz;
+    int rc;
+    void *d;
+    if ((rc = plan_upload(p, word.data(), word.size() * 4, &d))) return rc;
+    P.ptr = (const uint32_t *)d;
+    if ((rc = plan_upload(p, rows.data(), rows.size() * 4, &d))) return rc;
+    P.rind = (const uint32_t *)d;
+    if ((rc = plan_upload(p, zrows.data(), zrows.size() * 4, &d))) return rc;
+    P.hcol = (const uint32_t *)d;
+    P.nhcol = (uint32_t)zrows.size();
+    if ((rc = plan_upload(p, &P, sizeof(P), (void **)&g.work.d_prob))) return rc;
+    uint64_t carries = 0;
+    for (int i = 0; i < 6; i++) {
+        const uint32_t E = spd::panel_entries(1 << i, sa);
+        std::vector<spd::Cross> c;
+        for (const spd::Cross &C : cross)
+            if (C.b / E != C.e / E) c.push_back(C);
+        g.work.ncross[i] = (uint32_t)c.size();
+        if ((rc = plan_upload(p, c.data(), c.size() * sizeof(spd::Cross), (void **)&g.work.d_cross[i]))) return rc;
+        carries = std::max(carries, (((uint64_t)nnz + E - 1) / E) << i);
+    }
+    if ((rc = plan_alloc(p, carries * sa, &g.work.d_carry_val))) return rc;
+    g.h_probs = {P};
+    g.h_cross = std::move(cross);
+    return SP_OK;
+}
+
+// Whether panels replace the row-ordered group for several right-hand sides: not where the row
+// kernels serve even CSR rows, nor for COO floats, whose panels of columns have the bits of the
+// row-ordered COO tiles whatever the tile order.
+bool takes_panel(const sp_plan *p) {
+    const int kind = p->many->work.kind;
+    return kind == WK_CSR_MERGE || (kind == WK_COO_SEG && p->dtype != SP_F32 && p->dtype != SP_F64);
+}
+
 // Gives a plan whose row-ordered group is built (one problem) wide tiles for one right-hand
-// side; the row-ordered group stays for several.  SP_ERR_RANGE: not a matrix for wide tiles
+// side; its columns and values also serve several.  SP_ERR_RANGE: not a matrix for wide tiles
 // (columns of a tile too far apart, or one tile with most of the matrix's empty rows).
 int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
     const size_t sv = sp_dtype_size(p->dtype), sa = acc_size(p->dtype);
@@ -459,6 +520,7 @@ int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
     P.pbits = pb;
     p->many = std::make_unique<PlanWork>(std::move(*static_cast<PlanWork *>(p)));
     static_cast<PlanWork &>(*p) = PlanWork{};
+    if (takes_panel(p) && (rc = build_panel(p, *p->many, rowptr))) return rc;
     Builder b(p);
     b.add(P, cent, &crow, &carry);
     p->work.lanes = s.nt;

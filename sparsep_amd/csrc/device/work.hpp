@@ -12,7 +12,7 @@
 struct sp_ctx;
 
 enum WorkKind { WK_CSR_MERGE = 0, WK_CSR_VEC = 1, WK_COO_SEG = 2, WK_BCSR_VEC = 3, WK_BCOO_SEG = 4, WK_CSR_HOT = 5,
-               WK_BCSR_SEG = 6, WK_WIDE = 7 };
+               WK_BCSR_SEG = 6, WK_WIDE = 7, WK_PANEL = 8 };
 
 struct Work {
     int kind = WK_CSR_MERGE;
@@ -36,6 +36,9 @@ struct Work {
     bool slice = false;     // 2D CSR/COO tiles: one right-hand side gathers from an LDS copy of the tile's x slice
     spd::Run *d_runs = nullptr;  // CSR merge: row runs that cross tiles (fix-up list), nruns of them
     uint32_t nruns = 0;
+    uint32_t panel_nent = 0;     // panels of one problem: its entries (units follow from the width)
+    spd::Cross *d_cross[6] = {}; // panels: the rows that cross workgroups at widths 1, 2, 4 .. 32
+    uint32_t ncross[6] = {};
     bool atomic = false;         // COO/BCOO: rows crossing tiles merged by atomics (no carries)
     bool chunk = false;          // CSR merge / COO: every problem's arrays aligned to 4 entries and padded
                                  // past their end (library allocations), so tiles load 4-entry chunks
@@ -57,13 +60,14 @@ inline int max_rhs_chunk(const Work &w) {
     const bool wide8 = (w.dtype == SP_I64 || w.dtype == SP_F64) && w.R * w.C <= 16;
     switch (w.kind) {
     case WK_CSR_VEC: return 32;
+    case WK_PANEL: return 32;
     case WK_BCSR_VEC:
         if ((w.dtype == SP_F32 || w.dtype == SP_F64) && w.R == 4 && w.C == 4) return 32;  // matrix-core / vector-ALU kernels
         return wide8 ? 32 : w.R <= 2 ? 32 : w.R <= 4 ? 16 : 8;
     case WK_BCOO_SEG: return 1;
     case WK_BCSR_SEG: return 1;
     case WK_CSR_HOT: return 1;
-    case WK_WIDE: return 1;  // (plans with wide tiles keep a row-ordered work for several right-hand sides)
+    case WK_WIDE: return 1;  // (plans with wide tiles keep another group for several right-hand sides)
     default: return 8;
     }
 }
@@ -81,7 +85,7 @@ int run_work_t(const Work &w, sp_ctx *ctx, const void *xb, void *yb, const uintp
 // Whether a kind leaves carries of rows that cross units to the fix-up.
 inline bool has_carries(int kind) {
     return kind == WK_CSR_MERGE || kind == WK_COO_SEG || kind == WK_BCOO_SEG || kind == WK_CSR_HOT || kind == WK_BCSR_SEG ||
-           kind == WK_WIDE;
+           kind == WK_WIDE || kind == WK_PANEL;
 }
 extern template int run_work_t<int8_t>(const Work &, sp_ctx *, const void *, void *, const uintptr_t *,
                                        const uintptr_t *, int, int, int);

@@ -1,4 +1,4 @@
-"""Wide column-ordered tiles (automatic 1D CSR and COO plans): integers
+"""Wide column-ordered tiles and panels (automatic 1D CSR and COO plans): integers
 bit-exact against the oracle, floats within the gamma(len+2) bound of the
 long-double reference, at the edges of tiles, with rows crossing many tiles,
 empty rows anywhere, columns further apart than a key holds, other leading
@@ -78,6 +78,26 @@ def test_wide_even_rows(sp, ctx, dt, rows, per, band):
         assert_parity(dt, y, A, x, kern)
 
 
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16, 32, 43])
+@pytest.mark.parametrize("dt", [0, 1, 2, 3, 4, 5])
+def test_panel_parity(sp, ctx, dt, k):
+    """Panels of every width, whole 16-byte pieces of x or not, CSR and COO."""
+    name = ["hub", "empties", "one", "exact"][(dt + k) % 4]
+    n, m, row, col = _pattern(name, np.random.default_rng(k))
+    A = _coo(sp, dt, n, m, row, col)
+    for kern, ldx, ldy in (("CSR-nnz", k, k), ("COO-nnz", k + 1, k + 2)):
+        X = _x(sp, dt, (m, ldx))
+        plan = sp.Plan(ctx, kern, A)
+        xd = sp.DeviceArray.from_numpy(ctx, X)
+        yd = sp.DeviceArray(ctx, (n, ldy), X.dtype)
+        yd.fill_bytes(0x5A)
+        plan.spmm(k, xd.addr, ldx, yd.addr, ldy)
+        ctx.sync()
+        Y = yd.numpy()
+        assert_parity_multi(dt, np.ascontiguousarray(Y[:, :k]), A, np.ascontiguousarray(X[:, :k]), f"{kern}/{name}/k{k}")
+        assert np.all(Y[:, k:].view(np.uint8) == 0x5A)
+
+
 def test_wide_columns_too_far(sp, ctx):
     """Nearly every run would end early: the plan keeps row-ordered tiles."""
     rng = np.random.default_rng(2)
@@ -113,10 +133,10 @@ def test_wide_strides_and_knobs(sp, ctx):
 
 def test_wide_in_batches(sp, ctx):
     """Wide plans of both shapes in one batch, with one and several right-hand sides."""
-    mats, ks = [], [1, 1, 4, 1]
-    for i, name in enumerate(["hub", "empties", "hub", "one"]):
+    mats, ks = [], [1, 1, 4, 1, 4, 43]
+    for i, name in enumerate(["hub", "empties", "hub", "one", "exact", "one"]):
         mats.append(_coo(sp, 2, *_pattern(name, np.random.default_rng(i)), seed=i))
-    plans = [sp.Plan(ctx, k, A) for k, A in zip(["CSR-nnz", "COO-nnz", "CSR-nnz", "COO-row"], mats)]
+    plans = [sp.Plan(ctx, k, A) for k, A in zip(["CSR-nnz", "COO-nnz", "CSR-nnz", "COO-row", "COO-nnz", "CSR-row"], mats)]
     xs = [_x(sp, 2, (A.ncols, k)) for A, k in zip(mats, ks)]
     xd = [sp.DeviceArray.from_numpy(ctx, x) for x in xs]
     yd = [sp.DeviceArray(ctx, (A.nrows, k), np.int32) for A, k in zip(mats, ks)]
