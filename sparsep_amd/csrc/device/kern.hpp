@@ -48,7 +48,9 @@ struct Prob {
     uint32_t nhcol;        // hot-x CSR: number of staged ("hot") columns; wide tiles: entries per tile
     const uint32_t *hcol;  // hot-x CSR: the staged columns, slot order; wide tiles: base column per 64 words;
                            // panels: the rows without entries (nhcol of them)
-    void *xh;              // hot-x CSR: x at the staged columns, written before each launch
+    void *xh;              // hot-x CSR: x at the staged columns, written before each launch; wide
+                           // tiles with long gaps between rows: rows by number, then the gaps' rows
+    uint32_t nkept;        // wide tiles: rows outside long gaps
 };
 
 template <typename T> struct Ptrs {
@@ -598,9 +600,13 @@ __global__ __launch_bounds__(HOT_TPB) void csr_hot_kernel(const Prob *__restrict
 // sum in registers, a segmented scan of the open ends over lanes and then
 // waves, the row sums to LDS in row order, and from there to y: P.rind holds
 // for every row 1 + the number of its sum in the tile where the row ends, or 0
-// for a row without entries.  The open end of a tile is its carry; which row
+// for a row without entries.  Rows in gaps of more than WIDE_GAP are left out
+// there (a column stripe of a banded matrix has half of its rows in one) and
+// zeroed in even shares by all tiles.  The open end of a tile is its carry; which row
 // it belongs to is known to the plan (its run list).
 // ---------------------------------------------------------------------------
+constexpr uint32_t WIDE_GAP = 256;
+
 // Slot of row-order position pos: a thread's 16-byte pieces are exchanged by a
 // function of the thread, so that 16 neighbouring threads' reads of piece c
 // fall into different banks.  ce = values per piece, cpt = pieces per thread.
@@ -747,14 +753,30 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void wi
 
     // the rows that end in this tile and the empty ones among them, eight per thread at a time
     // (a tile of a graph's sparse end has several rows per entry)
-    for (uint32_t k0 = tid; k0 < nr; k0 += 8 * NT) {
-        uint32_t m[8];
+    auto output = [&](auto gaps_c) {
+        constexpr bool GAPS = decltype(gaps_c)::value;  // rows by number
+        const gptr<const uint32_t> __restrict__ rid = gp((const uint32_t *)P.xh);
+        for (uint32_t k0 = tid; k0 < nr; k0 += 8 * NT) {
+            uint32_t m[8], rw[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) m[i] = ldg(rmap + r0 + min(k0 + i * NT, nr - 1));
+            for (int i = 0; i < 8; i++) {
+                const uint32_t k = r0 + min(k0 + i * NT, nr - 1);
+                m[i] = ldg(rmap + k);
+                rw[i] = k;
+                if constexpr (GAPS) rw[i] = ldg(rid + k);
+            }
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (k0 + i * NT < nr) y[(size_t)(r0 + k0 + i * NT) * ldy] = m[i] ? to_val<T>(s_buf[m[i] - 1]) : T(0);
-    }
+            for (int i = 0; i < 8; i++)
+                if (k0 + i * NT < nr) y[(size_t)rw[i] * ldy] = m[i] ? to_val<T>(s_buf[m[i] - 1]) : T(0);
+        }
+        if constexpr (GAPS) {
+            const uint32_t nz = P.nrows - P.nkept, nt = (P.nent + P.nhcol - 1) / P.nhcol;
+            const uint32_t z1 = (uint32_t)((uint64_t)nz * (tl + 1) / nt);
+            for (uint32_t z = (uint32_t)((uint64_t)nz * tl / nt) + tid; z < z1; z += NT) y[(size_t)ldg(rid + P.nkept + z) * ldy] = T(0);
+        }
+    };
+    if (P.nkept == P.nrows) output(std::false_type{});
+    else output(std::true_type{});
 }
 
 // ---------------------------------------------------------------------------

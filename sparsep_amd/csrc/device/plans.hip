@@ -458,37 +458,53 @@ bool takes_panel(const sp_plan *p) {
     return kind == WK_CSR_MERGE || (kind == WK_COO_SEG && p->dtype != SP_F32 && p->dtype != SP_F64);
 }
 
-// Gives a plan whose row-ordered group is built (one problem) wide tiles for one right-hand
-// side; its columns and values also serve several.  SP_ERR_RANGE: not a matrix for wide tiles
-// (columns of a tile too far apart, or one tile with most of the matrix's empty rows).
-int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
+// One problem in wide tiles: its descriptor and the coordinates of its units.
+struct WidePart {
+    Prob P{};
+    std::vector<uint32_t> cent, crow, carry;  // entries, rows, row carried out
+};
+
+// Wide tiles of a problem whose row-ordered columns and values are on the device.
+// SP_ERR_RANGE: not a matrix for wide tiles (columns of a tile too far apart, or one tile with
+// most of the matrix's empty rows).
+int wide_part(sp_plan *p, const Prob &rows, const uint32_t *rowptr, WideShape s, WidePart &out) {
     const size_t sv = sp_dtype_size(p->dtype), sa = acc_size(p->dtype);
-    Prob P = p->h_probs[0];
+    Prob P = rows;
     const uint32_t words = s.nt * s.ipt, nnz = P.nent;
     uint32_t pb = 0;
     while ((1u << pb) < words) pb++;
     const uint32_t tile = P.ncols_elem <= (1ull << (32 - pb)) ? words : words - 256;  // entries per tile
     const uint32_t nt = (uint32_t)(((uint64_t)nnz + tile - 1) / tile);
     const uint64_t tot = (uint64_t)nt * words;
-    // the word of every thread, every row's sum, the first row of each tile's rows (those that end
-    // in it and the empty ones after each), the row it carries out
-    std::vector<uint32_t> word((size_t)nt * s.nt, 0), cent, crow, carry(nt + 1, spd::NONE);
-    std::vector<uint16_t> rmap(P.nrows, 0);
+    // the word of every thread, every kept row's sum, the first kept row of each tile's (those that
+    // end in it and the empty ones before the next), the row it carries out
+    std::vector<uint32_t> word((size_t)nt * s.nt, 0), &cent = out.cent, &crow = out.crow, &carry = out.carry;
+    std::vector<uint32_t> kept, gap;  // rows outside and inside long gaps
+    std::vector<uint16_t> rmap;
+    carry.assign((size_t)nt + 1, spd::NONE);
     crow.push_back(0);
-    for (uint32_t i = 0, ord = 0; i < P.nrows; i++) {
-        if (rowptr[i + 1] == rowptr[i]) continue;
+    for (uint32_t i = 0, next = 0, ord = 0; i <= P.nrows; i++) {
+        if (i < P.nrows && rowptr[i + 1] == rowptr[i]) continue;
+        for (const bool lng = i - next > spd::WIDE_GAP; next < i; next++) {
+            (lng ? gap : kept).push_back(next);
+            if (!lng) rmap.push_back(0);
+        }
+        if (i == P.nrows) break;
+        next = i + 1;
         const uint32_t e = rowptr[i + 1] - 1, t = e / tile, at = e % tile;
         while (crow.size() <= t) {  // row i is the first that ends in tile t
-            crow.push_back(i);
+            crow.push_back((uint32_t)kept.size());
             ord = 0;
         }
         uint32_t &w = word[(size_t)t * s.nt + at / s.ipt];
         w |= 1u << (at % s.ipt);
-        rmap[i] = (uint16_t)++ord;
+        kept.push_back(i);
+        rmap.push_back((uint16_t)++ord);
         for (uint32_t q = rowptr[i] / tile; q < t; q++) carry[q] = i;
     }
-    while (crow.size() <= nt) crow.push_back(P.nrows);
-    crow[nt] = P.nrows;
+    const uint32_t nkept = (uint32_t)kept.size();
+    while (crow.size() <= nt) crow.push_back(nkept);
+    crow[nt] = nkept;
     for (uint32_t t = 0; t < nt; t++) {
         if (crow[t + 1] - crow[t] > 16 * tile) return SP_ERR_RANGE;
         cent.push_back(t * tile);
@@ -518,19 +534,38 @@ int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
     P.hcol = (const uint32_t *)base;
     P.nhcol = tile;
     P.pbits = pb;
+    P.nkept = nkept;
+    if (!gap.empty()) {
+        kept.insert(kept.end(), gap.begin(), gap.end());
+        if ((rc = plan_upload(p, kept.data(), kept.size() * 4, &P.xh))) return rc;
+    }
+    out.P = P;
+    return SP_OK;
+}
+
+// Makes wide tiles the plan's group for one right-hand side; the group it has stays for several.
+int finish_wide(sp_plan *p, const std::vector<WidePart> &parts, WideShape s) {
     p->many = std::make_unique<PlanWork>(std::move(*static_cast<PlanWork *>(p)));
     static_cast<PlanWork &>(*p) = PlanWork{};
-    if (takes_panel(p) && (rc = build_panel(p, *p->many, rowptr))) return rc;
     Builder b(p);
-    b.add(P, cent, &crow, &carry);
+    for (const WidePart &w : parts) b.add(w.P, w.cent, &w.crow, &w.carry);
     p->work.lanes = s.nt;
     p->work.ipt = s.ipt;
     p->algo = SP_ALGO_SEGMENTED_SORTED;
     p->lanes = 0;
-    p->ipt = words / TPB;
-    p->ntiles = nt;
+    p->ipt = s.nt * s.ipt / TPB;
     p->nsub = s.nt;
     return b.finish(WK_WIDE, true, 1);
+}
+
+// Gives a 1D plan whose row-ordered group is built wide tiles for one right-hand side; its
+// columns and values also serve several.
+int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
+    std::vector<WidePart> part(1);
+    int rc = wide_part(p, p->h_probs[0], rowptr, s, part[0]);
+    if (rc || (rc = finish_wide(p, part, s))) return rc;
+    p->ntiles = p->work.nunits;
+    return takes_panel(p) ? build_panel(p, *p->many, rowptr) : SP_OK;
 }
 
 // Undoes a plan's groups (a wide layout that did not fit).
@@ -1051,7 +1086,7 @@ int run_plan(sp_plan *p, const void *x, void *y, int k, int ldx, int ldy) {
         p->d_ypart = d;
         p->ypart_bytes = need;
     }
-    Work w = p->work;
+    Work w = p->group(k).work;
     w.zero_rows = w.zero_all ? (uint64_t)p->vert * p->nrows : 0;
     int rc = run_work(w, p->ctx, x, p->d_ypart, nullptr, nullptr, k, ldx, k);
     if (rc) return rc;
@@ -1139,10 +1174,18 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
                           p->opts.count_values, &T);
     // row statistics for the CSR algorithm and the tile size choice
     uint32_t maxlen = 0;
+    WideShape wide;
+    std::vector<WidePart> wide_parts;
+    bool wide_zero = false;
     if (!rc && (tk.format == SP_FMT_CSR || tk.format == SP_FMT_COO)) {
         std::vector<uint32_t> cnt(n + 1, 0);
         for (uint32_t k = 0; k < A->nnz; k++) cnt[A->rowind[k]]++;
         for (uint32_t i = 0; i < n; i++) maxlen = std::max(maxlen, cnt[i]);
+        // Even rows take wide tiles as in 1D; skewed ones keep the kernels whose sums have the same
+        // bits as those over LDS slices of x.  (A plan's tiles are sorted one launch each: 16K
+        // entries per tile at least.)
+        if (A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64)
+            wide = wide_shape(p, tk.format == SP_FMT_COO, false, A->colind, n, A->nnz);
     }
     if (sorted) sp_free_coo(sorted);
     if (rc) return rc;
@@ -1189,6 +1232,7 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
                         c[j + 1] == c[j] + 1 && c[j + 2] == c[j] + 2 && c[j + 3] == c[j] + 3;
     }
     const bool padded = csr_chunk || coo_quads;
+    if (padded) wide = WideShape{};  // aligned four-column runs keep their four-value x loads
     std::vector<uint64_t> e0c;  // chunked layout: each tile's first entry in the uploaded arrays
     do {
         // upload the tiling's arrays once; tiles point into them
@@ -1425,6 +1469,35 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
             b.add(P, k0, kind == WK_CSR_MERGE ? &k1 : nullptr);
         }
         if (rc) break;
+        // Wide tiles for one right-hand side, as for 1D CSR/COO: stripes leave about half of a
+        // local matrix's rows empty in each, which cost a row map's word and no row of the row
+        // kernel.  (While the arrays on the device are row ordered.)
+        if (wide.nt) {
+            std::vector<uint32_t> rp;
+            for (uint32_t t = 0; t < nt && !rc; t++) {
+                const Prob &Q = b.probs[t];
+                if (Q.nent == 0) {
+                    wide_zero |= Q.nrows > 0;  // its rows of the partial buffer are zeroed first
+                    continue;
+                }
+                const uint32_t *hrp;
+                if (tk.format == SP_FMT_CSR) {
+                    hrp = T->drowptr + (size_t)t * (th + 1);
+                } else {
+                    rp.assign((size_t)Q.nrows + 1, 0);
+                    for (uint32_t k = 0; k < Q.nent; k++) rp[T->drowind[T->nnz_offset[t] + k] + 1]++;
+                    for (uint32_t i = 0; i < Q.nrows; i++) rp[i + 1] += rp[i];
+                    hrp = rp.data();
+                }
+                wide_parts.emplace_back();
+                rc = wide_part(p, Q, hrp, wide, wide_parts.back());
+            }
+            if (rc == SP_ERR_RANGE) {
+                rc = SP_OK;
+                wide_parts.clear();
+            }
+            if (rc) break;
+        }
         // Column-ordered tiles (as for 1D CSR/COO): every unit's entries sorted by local column,
         // with the row-order position in the low bits; the arrays uploaded above are replaced.
         if (col_order && !blk && T->nnz) {
@@ -1469,6 +1542,10 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
         if (atom) {
             p->work.atomic = true;
             p->launches = 1;
+        }
+        if (!rc && !wide_parts.empty()) {
+            rc = finish_wide(p, wide_parts, wide);
+            p->work.zero_all = wide_zero;
         }
         p->nsub = p->work.nunits;
     } while (0);

@@ -78,6 +78,28 @@ def test_wide_even_rows(sp, ctx, dt, rows, per, band):
         assert_parity(dt, y, A, x, kern)
 
 
+@pytest.mark.parametrize("kern", ["RBDCSR", "BDCSR", "DCSR", "RBDCOO", "DCOO"])
+@pytest.mark.parametrize("dt", [0, 4, 5])
+def test_wide_tilings(sp, ctx, dt, kern):
+    """2D tilings: long gaps of empty rows in every stripe, a stripe without entries, a wide panel."""
+    rng = np.random.default_rng(4)
+    n = 30011
+    row = np.repeat(np.arange(n), 33)
+    col = (row + rng.integers(0, 64, row.size)) % n
+    A = _coo(sp, dt, n, n, row, col)
+    B = _coo(sp, dt, n, 2 * n, row, col)  # the second of two stripes is empty
+    for M in (A, B):
+        x = _x(sp, dt, M.ncols)
+        y, plan = run(sp, ctx, kern, M, x)
+        assert plan.info()["algo"] == sp.ALGO_SEGMENTED_SORTED
+        assert_parity(dt, y, M, x, kern)
+        y, _ = run(sp, ctx, kern, M, x, plan=plan)
+        assert_parity(dt, y, M, x, kern)
+    X = _x(sp, dt, (n, 3))
+    Y, _ = run(sp, ctx, kern, A, X, k=3)
+    assert_parity_multi(dt, Y, A, X, kern)
+
+
 @pytest.mark.parametrize("k", [1, 2, 4, 8, 16, 32, 43])
 @pytest.mark.parametrize("dt", [0, 1, 2, 3, 4, 5])
 def test_panel_parity(sp, ctx, dt, k):
