@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <memory>
 #include <vector>
 
@@ -41,6 +42,16 @@ struct PlanWork {
     std::vector<spd::Cross> h_cross;  // panels: the rows that cross workgroups at the widest panel
 };
 
+// Vectors and state of a conjugate-gradient solve (solve.hip).
+struct CgBuf {
+    void *dev = nullptr, *note = nullptr;  // device memory, pinned host memory
+    void release() {
+        if (dev) (void)hipFree(dev);
+        if (note) (void)hipHostFree(note);
+        dev = note = nullptr;
+    }
+};
+
 struct sp_plan : PlanWork {  // (the base: the main launch group)
     sp_ctx *ctx = nullptr;
     int id = 0, dtype = 0, algo = 0;
@@ -69,6 +80,8 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
 
     std::vector<void *> allocs;
 
+    CgBuf cg;  // kept between solves, used by one at a time
+    std::atomic<bool> cg_busy{false};
 };
 
 // Allocation helpers (record in plan->allocs, respect mem_cap_bytes).

@@ -153,6 +153,7 @@ int plan_upload(sp_plan *p, const void *host, size_t bytes, void **out) {
 static void plan_free(sp_plan *p) {
     if (!p) return;
     for (void *d : p->allocs) (void)hipFree(d);
+    p->cg.release();
     delete p;
 }
 
