@@ -101,6 +101,185 @@ __global__ void dense_bwd_x(const float *__restrict__ dOut, const uint16_t *__re
     dIn[(size_t)b * I + i] = acc;
 }
 
+// Loss and gradient of one mini-batch in two kernels, for layer widths that are multiples of 8
+// (16-byte weight loads) and at most MAXW.  A mini-batch is 1 to 4 MFLOP: what costs is the chain
+// of launches and copies, not the arithmetic (batch 64 through the layer kernels above, eleven
+// launches and five copies: 157 us).
+//
+// mlp_sample: a workgroup takes ROWS samples through the forward pass, the loss gradient and the
+// input gradients, activations in LDS.  It reads the samples where the caller has them (pinned
+// host memory: once, 0.5 KB per sample) and leaves what the weight gradients need in device
+// memory.  mlp_weights: a workgroup takes 8 outputs x 64 inputs of one layer's weight gradient
+// over all samples (LDS tiles of 64 samples), or 256 of the loss terms; the gradient goes to
+// device memory (for Adam) and, when asked for, straight to pinned host memory.  Every sum runs
+// in the order of the layer kernels, so the results have the same bits.
+constexpr int ROWS = 2, SPT = 128, MAXW = 256;  // samples per workgroup, threads per sample
+
+struct MlpArgs {
+    int B, in, h1, h2, out;
+    const float *x, *t, *m;   // the batch (m may be null: all ones)
+    const float *p;           // FP32 parameters (biases)
+    const uint16_t *pb;       // BF16 weights
+    int off[6];
+    float *xc, *a1, *a2, *d1, *d2, *d3, *l;  // kept for the weight gradients (xc: copy of x, or null)
+    float *g, *hg, *part;     // gradient (device; host or null), loss partial sums
+    float inv_count;
+};
+
+// out[o] = act(W[o] . in + bias[o]) for one sample by SPT threads
+__device__ __forceinline__ void sample_dense(const float *s_in, int I, const uint16_t *__restrict__ W,
+                                             const float *__restrict__ bias, float *s_out, int O, bool relu, int lane) {
+    for (int o = lane; o < O; o += SPT) {
+        float acc = 0.f;
+#pragma unroll 4
+        for (int i = 0; i < I; i += 8) {
+            const uint4 w = *(const uint4 *)(W + (size_t)o * I + i);
+            const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                acc = __builtin_fmaf(s_in[i + 2 * k], __builtin_bit_cast(float, ww[k] << 16), acc);
+                acc = __builtin_fmaf(s_in[i + 2 * k + 1], __builtin_bit_cast(float, ww[k] & 0xFFFF0000u), acc);
+            }
+        }
+        const float v = acc + bias[o];
+        s_out[o] = (relu && v < 0.f) ? 0.f : v;
+    }
+}
+
+// dIn[i] = sum_o dOut[o] W[o][i] where the activation is positive
+__device__ __forceinline__ void sample_dense_bwd(const float *s_d, int O, const uint16_t *__restrict__ W, int I,
+                                                 const float *s_act, float *s_din, int lane) {
+    for (int i = lane; i < I; i += SPT) {
+        float acc = 0.f;
+#pragma unroll 16
+        for (int o = 0; o < O; o++) acc = __builtin_fmaf(s_d[o], bf2f(W[(size_t)o * I + i]), acc);
+        s_din[i] = s_act[i] <= 0.f ? 0.f : acc;
+    }
+}
+
+__global__ __launch_bounds__(ROWS * SPT) void mlp_sample(MlpArgs a) {
+    __shared__ __align__(16) float s_x[ROWS][MAXW], s_a1[ROWS][MAXW], s_a2[ROWS][MAXW], s_y[ROWS][MAXW];
+    __shared__ __align__(16) float s_d[ROWS][MAXW], s_e[ROWS][MAXW];
+    const int lane = threadIdx.x % SPT, r = threadIdx.x / SPT, b = blockIdx.x * ROWS + r;
+    const bool in = b < a.B;  // (a sample past the batch computes on zeros and stores nothing)
+    for (int i = lane; i < a.in; i += SPT) {
+        const float v = in ? a.x[(size_t)b * a.in + i] : 0.f;
+        s_x[r][i] = v;
+        if (in && a.xc) a.xc[(size_t)b * a.in + i] = v;
+    }
+    // the targets' way over the bus runs beside the forward pass
+    float t[MAXW / SPT], m[MAXW / SPT];
+#pragma unroll
+    for (int k = 0; k < MAXW / SPT; k++) {
+        const int o = lane + k * SPT;
+        const bool ok = in && o < a.out;
+        t[k] = ok ? a.t[(size_t)b * a.out + o] : 0.f;
+        m[k] = ok && a.m ? a.m[(size_t)b * a.out + o] : 1.f;
+    }
+    __syncthreads();
+    sample_dense(s_x[r], a.in, a.pb + a.off[0], a.p + a.off[1], s_a1[r], a.h1, true, lane);
+    __syncthreads();
+    sample_dense(s_a1[r], a.h1, a.pb + a.off[2], a.p + a.off[3], s_a2[r], a.h2, true, lane);
+    __syncthreads();
+    sample_dense(s_a2[r], a.h2, a.pb + a.off[4], a.p + a.off[5], s_y[r], a.out, false, lane);
+#pragma unroll
+    for (int k = 0; k < MAXW / SPT; k++) {  // (each thread takes the outputs that it has formed)
+        const int o = lane + k * SPT;
+        if (o < a.out) {
+            const float d = (s_y[r][o] - t[k]) * m[k];
+            const float dy = 2.f * d * m[k] * a.inv_count;
+            s_d[r][o] = dy;
+            if (in) {
+                a.d3[(size_t)b * a.out + o] = dy;
+                a.l[(size_t)b * a.out + o] = d * d;
+            }
+        }
+    }
+    __syncthreads();
+    sample_dense_bwd(s_d[r], a.out, a.pb + a.off[4], a.h2, s_a2[r], s_e[r], lane);
+    __syncthreads();
+    sample_dense_bwd(s_e[r], a.h2, a.pb + a.off[2], a.h1, s_a1[r], s_d[r], lane);
+    if (!in) return;
+    for (int i = lane; i < a.h1; i += SPT) {  // (each thread's own elements)
+        a.a1[(size_t)b * a.h1 + i] = s_a1[r][i];
+        a.d1[(size_t)b * a.h1 + i] = s_d[r][i];
+    }
+    for (int i = lane; i < a.h2; i += SPT) {
+        a.a2[(size_t)b * a.h2 + i] = s_a2[r][i];
+        a.d2[(size_t)b * a.h2 + i] = s_e[r][i];
+    }
+}
+
+constexpr int WO = 8, WI = 64, WB = 64;  // outputs, inputs and samples of a weight-gradient tile
+
+__host__ __device__ inline int weight_tiles(int I, int O) { return ((O + WO - 1) / WO) * ((I + WI - 1) / WI); }
+
+__global__ __launch_bounds__(256) void mlp_weights(MlpArgs a, const float *__restrict__ x) {
+    __shared__ float s_in[WB][WI], s_d[WB][WO];
+    const int tid = threadIdx.x;
+    int tile = blockIdx.x, I = a.in, O = a.h1, ow = a.off[0], ob = a.off[1];
+    const float *dOut = a.d1, *in = x;
+    const int n1 = weight_tiles(a.in, a.h1), n2 = weight_tiles(a.h1, a.h2), n3 = weight_tiles(a.h2, a.out);
+    if (tile >= n1 + n2 + n3) {  // loss terms
+        float *const s = &s_in[0][0];
+        const int i = (tile - n1 - n2 - n3) * 256 + tid;
+        s[tid] = i < a.B * a.out ? a.l[i] : 0.f;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if (tid < w) s[tid] += s[tid + w];
+            __syncthreads();
+        }
+        if (tid == 0) a.part[tile - n1 - n2 - n3] = s[0];
+        return;
+    }
+    if (tile >= n1 + n2) {
+        tile -= n1 + n2;
+        I = a.h2; O = a.out; ow = a.off[4]; ob = a.off[5]; dOut = a.d3; in = a.a2;
+    } else if (tile >= n1) {
+        tile -= n1;
+        I = a.h1; O = a.h2; ow = a.off[2]; ob = a.off[3]; dOut = a.d2; in = a.a1;
+    }
+    const int ti = (I + WI - 1) / WI, i0 = tile % ti * WI, o0 = tile / ti * WO;
+    const int i = tid % WI, og = tid / WI * 2;
+    float acc[2] = {0.f, 0.f}, accb = 0.f;
+    for (int b0 = 0; b0 < a.B; b0 += WB) {
+        const int nb = min(WB, a.B - b0);
+#pragma unroll
+        for (int k = 0; k < WB * WI / 256; k++) {
+            const int b = tid / WI + k * (256 / WI);
+            s_in[b][i] = b < nb && i0 + i < I ? in[(size_t)(b0 + b) * I + i0 + i] : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < WB * WO / 256; k++) {
+            const int b = tid / WO + k * (256 / WO), o = tid % WO;
+            s_d[b][o] = b < nb && o0 + o < O ? dOut[(size_t)(b0 + b) * O + o0 + o] : 0.f;
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int b = 0; b < nb; b++) {
+            const float v = s_in[b][i];
+            acc[0] = __builtin_fmaf(s_d[b][og], v, acc[0]);
+            acc[1] = __builtin_fmaf(s_d[b][og + 1], v, acc[1]);
+        }
+        if (i0 == 0 && tid < WO)
+            for (int b = 0; b < nb; b++) accb += s_d[b][tid];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int o = o0 + og + k;
+        if (o < O && i0 + i < I) {
+            const size_t at = (size_t)ow + (size_t)o * I + i0 + i;
+            a.g[at] = acc[k];
+            if (a.hg) a.hg[at] = acc[k];
+        }
+    }
+    if (i0 == 0 && tid < WO && o0 + tid < O) {
+        a.g[ob + o0 + tid] = accb;
+        if (a.hg) a.hg[ob + o0 + tid] = accb;
+    }
+}
+
 __global__ void adam_step(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
                           float *__restrict__ v, uint16_t *__restrict__ pb, int n, float lr, float b1, float b2,
                           float eps, float c1, float c2) {
@@ -135,21 +314,33 @@ struct sp_mlp {
     // activations for a batch
     int cap = 0;
     float *x = nullptr, *a1 = nullptr, *z1 = nullptr, *a2 = nullptr, *z2 = nullptr, *y = nullptr;
-    float *t = nullptr, *msk = nullptr, *d3 = nullptr, *d2 = nullptr, *d1 = nullptr, *part = nullptr;
+    float *t = nullptr, *msk = nullptr, *d3 = nullptr, *d2 = nullptr, *d1 = nullptr, *part = nullptr, *l = nullptr;
+    // pinned host memory for a batch: x, t and mask in; gradient and loss partial sums out
+    float *hx = nullptr, *hg = nullptr;
+    // widths that the two-kernel path takes (16-byte weight loads at every row)
+    bool two() const {
+        return in % 8 == 0 && h1 % 8 == 0 && h2 % 8 == 0 && in <= MAXW && h1 <= MAXW && h2 <= MAXW && out <= MAXW;
+    }
 };
 
 static int mlp_alloc(float **p, size_t n) { return hipMalloc((void **)p, (n ? n : 1) * sizeof(float)) == hipSuccess ? SP_OK : SP_ERR_NOMEM; }
 
 static int mlp_reserve(sp_mlp *m, int B) {
     if (B <= m->cap) return SP_OK;
-    float **bufs[] = {&m->x, &m->a1, &m->z1, &m->a2, &m->z2, &m->y, &m->t, &m->msk, &m->d3, &m->d2, &m->d1, &m->part};
+    float **bufs[] = {&m->x, &m->a1, &m->z1, &m->a2, &m->z2, &m->y, &m->t, &m->msk, &m->d3, &m->d2, &m->d1, &m->part, &m->l};
+    m->cap = 0;
     for (float **b : bufs)
         if (*b) { (void)hipFree(*b); *b = nullptr; }
+    for (float **b : {&m->hx, &m->hg})
+        if (*b) { (void)hipHostFree(*b); *b = nullptr; }
     const size_t n[] = {(size_t)B * m->in, (size_t)B * m->h1, (size_t)B * m->h1, (size_t)B * m->h2, (size_t)B * m->h2,
                         (size_t)B * m->out, (size_t)B * m->out, (size_t)B * m->out, (size_t)B * m->out,
-                        (size_t)B * m->h2, (size_t)B * m->h1, (size_t)B * m->out / 256 + 2};
-    for (int i = 0; i < 12; i++)
+                        (size_t)B * m->h2, (size_t)B * m->h1, (size_t)B * m->out / 256 + 2, (size_t)B * m->out};
+    for (int i = 0; i < 13; i++)
         if (mlp_alloc(bufs[i], n[i])) return SP_ERR_NOMEM;
+    if (m->two() && (hipHostMalloc((void **)&m->hx, (size_t)B * (m->in + 2 * m->out) * 4) != hipSuccess ||
+                     hipHostMalloc((void **)&m->hg, ((size_t)m->np + n[11]) * 4) != hipSuccess))
+        return SP_ERR_NOMEM;
     m->cap = B;
     return SP_OK;
 }
@@ -188,9 +379,11 @@ extern "C" int sp_mlp_create(sp_ctx *ctx, int in, int h1, int h2, int out, uint6
 
 extern "C" int sp_mlp_destroy(sp_mlp *m) {
     if (!m) return SP_ERR_ARG;
-    float *bufs[] = {m->p, m->g, m->m, m->v, m->x, m->a1, m->z1, m->a2, m->z2, m->y, m->t, m->msk, m->d3, m->d2, m->d1, m->part};
+    float *bufs[] = {m->p, m->g, m->m, m->v, m->x, m->a1, m->z1, m->a2, m->z2, m->y, m->t, m->msk, m->d3, m->d2, m->d1, m->part, m->l};
     for (float *b : bufs)
         if (b) (void)hipFree(b);
+    for (float *b : {m->hx, m->hg})
+        if (b) (void)hipHostFree(b);
     if (m->pb) (void)hipFree(m->pb);
     delete m;
     return SP_OK;
@@ -235,8 +428,33 @@ extern "C" int sp_mlp_predict(sp_mlp *m, const float *X, int B, float *Y) {
     return SP_OK;
 }
 
+static float mean_loss(const float *part, int nb, int ny) {
+    double l = 0;
+    for (int i = 0; i < nb; i++) l += part[i];
+    return (float)(l / ny);
+}
+
+// Loss and gradient of the batch at x, t, msk (device or pinned host memory; msk may be null) in
+// two kernels; waits for them.  The gradient stays in m->g and is copied to `grad` if given.
+static int loss_grad_two(sp_mlp *m, int B, const float *x, const float *t, const float *msk, float *loss, float *grad) {
+    hipStream_t s = m->ctx->stream;
+    const int ny = B * m->out, nb = (ny + 255) / 256;
+    MlpArgs a{B, m->in, m->h1, m->h2, m->out, x, t, msk, m->p, m->pb, {}, x == m->x ? nullptr : m->x, m->a1, m->a2,
+              m->d1, m->d2, m->d3, m->l, m->g, grad ? m->hg : nullptr, m->hg + m->np, 1.f / (float)ny};
+    for (int i = 0; i < 6; i++) a.off[i] = m->off[i];
+    const int tiles = weight_tiles(m->in, m->h1) + weight_tiles(m->h1, m->h2) + weight_tiles(m->h2, m->out);
+    hipLaunchKernelGGL(mlp_sample, dim3((B + ROWS - 1) / ROWS), dim3(ROWS * SPT), 0, s, a);
+    hipLaunchKernelGGL(mlp_weights, dim3(tiles + nb), dim3(256), 0, s, a, (const float *)m->x);
+    if (hipGetLastError() != hipSuccess) return SP_ERR_HIP;
+    SP_HIP_TRY(hipStreamSynchronize(s));
+    if (loss) *loss = mean_loss(m->hg + m->np, nb, ny);
+    if (grad) memcpy(grad, m->hg, (size_t)m->np * 4);
+    return SP_OK;
+}
+
 // Forward + masked-MSE backward for one batch already in m->x / m->t / m->msk.
 static int loss_grad_dev(sp_mlp *m, int B, float *loss) {
+    if (m->two()) return loss_grad_two(m, B, m->x, m->t, m->msk, loss, nullptr);
     hipStream_t s = m->ctx->stream;
     int rc = forward_dev(m, B);
     if (rc) return rc;
@@ -257,9 +475,7 @@ static int loss_grad_dev(sp_mlp *m, int B, float *loss) {
         std::vector<float> part(nb);
         SP_HIP_TRY(hipMemcpyAsync(part.data(), m->part, (size_t)nb * 4, hipMemcpyDeviceToHost, s));
         SP_HIP_TRY(hipStreamSynchronize(s));
-        double l = 0;
-        for (float v : part) l += v;
-        *loss = (float)(l / ny);
+        *loss = mean_loss(part.data(), nb, ny);
     }
     return SP_OK;
 }
@@ -270,6 +486,13 @@ extern "C" int sp_mlp_loss_grad(sp_mlp *m, const float *X, const float *T, const
     int rc = mlp_reserve(m, B);
     if (rc) return rc;
     hipStream_t s = m->ctx->stream;
+    if (m->two()) {  // the kernels read the batch from pinned memory (every call ends with a wait)
+        float *const hx = m->hx, *const ht = hx + (size_t)B * m->in, *const hm = ht + (size_t)B * m->out;
+        memcpy(hx, X, (size_t)B * m->in * 4);
+        memcpy(ht, T, (size_t)B * m->out * 4);
+        if (M) memcpy(hm, M, (size_t)B * m->out * 4);
+        return loss_grad_two(m, B, hx, ht, M ? hm : nullptr, loss, grad);
+    }
     SP_HIP_TRY(hipMemcpyAsync(m->x, X, (size_t)B * m->in * 4, hipMemcpyHostToDevice, s));
     SP_HIP_TRY(hipMemcpyAsync(m->t, T, (size_t)B * m->out * 4, hipMemcpyHostToDevice, s));
     if (M) SP_HIP_TRY(hipMemcpyAsync(m->msk, M, (size_t)B * m->out * 4, hipMemcpyHostToDevice, s));
