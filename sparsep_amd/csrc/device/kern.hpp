@@ -1767,35 +1767,21 @@ __global__ __launch_bounds__(TPB) void rows_rhs_kernel(const Prob *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// BCSR 4 x 4 blocks times 8 or 16 right-hand sides on the matrix cores: the
-// block-row product of the reference (spmv/1D/BCSR-nnz/dpu/task.c:337-370)
+// BCSR 4 x 4 FP64 blocks times 8 or 16 right-hand sides on the matrix cores:
+// the block-row product of the reference (spmv/1D/BCSR-nnz/dpu/task.c:337-370)
 // as a dense 4 x 4 x K contraction per block.  A wave takes a block row; its
-// block columns are read 64 at a time, one per lane, and handed out by
+// block columns are read 32 at a time, one per lane, and handed out by
 // shuffles.  (32 right-hand sides go to bcsr4_valu_kernel, which is faster on
-// the 27-point stencil: FP32 331-345 against 514 us, FP64 633-637 against
-// 727 us.)
+// the 27-point stencil: 633-637 against 727 us; FP32: bcsr4_mfma_kernel.)
 //
-// FP32, v_mfma_f32_4x4x1_16b_f32: 16 independent 4x4x1 products per
-// instruction; product m = lane / 4 gets A[i] from lane 4m + i and B[j] from
-// lane 4m + j, and lane 4m + j holds D[v][j] in its register v.  Lane
-// l = K*g + 4*b + j takes matrix block g of the step (G = 64 / K blocks per
-// step), right-hand side column 4b + j, and matrix row j: A = block row j,
-// column c; B = x row (4 J + c), column 4b + j.  Four instructions (c = 0..3)
-// form the block's 4 x K contribution; the G partial sums are added across
-// lanes at the end of the row.  A lane reads its block row (A values) as
-// one 16-byte piece and its four B values element by element: the 4K-byte
-// rows of x come in whole, coalesced, with K lanes per row.  (Staging the
-// block values in LDS and reading x in 16-byte pieces with a DPP transpose
-// across each quad measured slower on the 27-point stencil.)
-//
-// FP64, v_mfma_f64_4x4x4_4b_f64: 4 independent 4x4x4 products per
-// instruction; product m takes A[i][k] from lane 16k + 4m + i and B[k][j]
-// from lane 16k + 4m + j, and lane 16i + 4m + j holds D[i][j].  Lane
-// l = 16h + 4m + o supplies block[o][h] (A, from the block values staged in
-// LDS 32 blocks at a time in 16-byte chunks) and x row (4 J + h) (B); the
-// columns that B's j = o stands for are a relabelling of the right-hand
-// sides: 16: one instruction per block, columns 4m + o; 8: two blocks per
-// instruction (products 0-1 and 2-3), columns 4(m%2) + o.
+// v_mfma_f64_4x4x4_4b_f64: 4 independent 4x4x4 products per instruction;
+// product m takes A[i][k] from lane 16k + 4m + i and B[k][j] from lane 16k +
+// 4m + j, and lane 16i + 4m + j holds D[i][j].  Lane l = 16h + 4m + o supplies
+// block[o][h] (A, from the block values staged in LDS 32 blocks at a time in
+// 16-byte chunks) and x row (4 J + h) (B); the columns that B's j = o stands
+// for are a relabelling of the right-hand sides: 16: one instruction per
+// block, columns 4m + o; 8: two blocks per instruction (products 0-1 and 2-3),
+// columns 4(m%2) + o.
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
@@ -1807,10 +1793,10 @@ __global__ __launch_bounds__(TPB) void bcsr_mfma_kernel(const Prob *__restrict__
                                                         const uint32_t *__restrict__ urow, Ptrs<T> io,
                                                         uint32_t nunits) {
     static_assert(K == 8 || K == 16, "8 or 16 right-hand sides per pass");
-    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "FP32 or FP64");
+    static_assert(__is_same(T, double), "FP64 blocks");
     constexpr int NW = TPB / WAVE;
-    constexpr int NB64 = 32;  // FP64: blocks per LDS batch (4 KB of values per wave)
-    __shared__ __align__(16) double s_val[sizeof(T) == 8 ? NW : 1][sizeof(T) == 8 ? NB64 * 16 : 1];
+    constexpr int NB64 = 32;  // blocks per LDS batch (4 KB of values per wave)
+    __shared__ __align__(16) double s_val[NW][NB64 * 16];
     const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
     for (uint32_t u = blockIdx.x; u < nunits; u += gridDim.x) {
     const uint32_t pid = unit_pid[u];
@@ -1824,7 +1810,6 @@ __global__ __launch_bounds__(TPB) void bcsr_mfma_kernel(const Prob *__restrict__
     const uint32_t ncols = P.ncols_elem;
     // This wave's block rows r0 + wid + NW t: their block ranges in one load (64 rows
     // a round), and the next row's first block columns loaded while a row runs.
-    constexpr uint32_t NBATCH = sizeof(T) == 4 ? WAVE : NB64;  // blocks per batch
     for (uint32_t R0 = r0 + wid; R0 < r1; R0 += NW * WAVE) {
     const uint32_t nrw = min((uint32_t)WAVE, (r1 - R0 + NW - 1) / NW);
     const uint32_t Il = R0 + NW * (uint32_t)lane;
@@ -1832,7 +1817,7 @@ __global__ __launch_bounds__(TPB) void bcsr_mfma_kernel(const Prob *__restrict__
     auto first_cols = [&](uint32_t t) {  // row t's first batch of block columns, one per lane
         const uint32_t bb = (uint32_t)__builtin_amdgcn_readlane((int)bl, (int)t);
         const uint32_t ee = (uint32_t)__builtin_amdgcn_readlane((int)el, (int)t);
-        return (uint32_t)lane < min(NBATCH, ee - bb) ? ldg(cip + bb + lane) : 0u;
+        return (uint32_t)lane < min((uint32_t)NB64, ee - bb) ? ldg(cip + bb + lane) : 0u;
     };
     uint32_t Jn = first_cols(0);
     for (uint32_t t = 0; t < nrw; t++) {
@@ -1841,96 +1826,186 @@ __global__ __launch_bounds__(TPB) void bcsr_mfma_kernel(const Prob *__restrict__
         const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)el, (int)t);
         const uint32_t Jfirst = Jn;
         if (t + 1 < nrw) Jn = first_cols(t + 1);
-        if constexpr (sizeof(T) == 4) {
-            constexpr int G = WAVE / K;  // matrix blocks per step
-            constexpr int U = 8 / G;     // steps whose loads go out together
-            const int g = lane / K, q = lane % K, j = lane % 4;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            // blocks in batches of 64: one coalesced load of their block columns,
-            // handed to the lanes that need them by a shuffle
-            for (uint32_t base = b; base < e; base += WAVE) {
-                const uint32_t nb = min((uint32_t)WAVE, e - base);
-                const uint32_t Jl = base == b ? Jfirst : ((uint32_t)lane < nb ? ldg(cip + base + lane) : 0u);
-                for (uint32_t t0 = 0; t0 < nb; t0 += G * U) {
-                    T a[U][4], xb[U][4];
-                    bool act[U];
-                    uint32_t J[U];
+        constexpr int BPS = K == 8 ? 2 : 1;  // matrix blocks per instruction
+        constexpr int U = 4 / BPS;           // steps whose loads go out together
+        double *const sv = s_val[wid];
+        const int h = lane / 16, m = (lane / 4) % 4, o = lane % 4;
+        const int gblk = BPS == 2 ? m / 2 : 0;  // block of this product within the step
+        // right-hand side column of this lane (a relabelling, see above)
+        const int colq = K == 16 ? 4 * m + o : 4 * (m % 2) + o;
+        double acc = 0.0;
+        for (uint32_t base = b; base < e; base += NB64) {
+            const uint32_t nb = min((uint32_t)NB64, e - base);
+            // the batch's values to LDS in 16-byte chunks, its block columns to lanes
+            __builtin_amdgcn_wave_barrier();
+            for (uint32_t c = lane; c < nb * 8; c += WAVE)
+                *(u32x4 *)(sv + c * 2) = __builtin_nontemporal_load((gptr<const u32x4>)(bv + (size_t)base * 16) + c);
+            const uint32_t Jl = base == b ? Jfirst : ((uint32_t)lane < nb ? ldg(cip + base + lane) : 0u);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (uint32_t t0 = 0; t0 < nb; t0 += BPS * U) {
+                double xv[U];
+                bool act[U];
+                uint32_t sidx[U];
 #pragma unroll
-                    for (int w = 0; w < U; w++) {
-                        const uint32_t sl = t0 + w * G + g;
-                        act[w] = sl < nb;
-                        const uint32_t sc = act[w] ? sl : 0u;  // a valid block; its product is dropped
-                        J[w] = (uint32_t)__shfl((int)Jl, (int)sc, WAVE);
-                        ldg_n<T, 4>(bv + (size_t)(base + sc) * 16 + j * 4, a[w]);  // matrix row j of the block
+                for (int w = 0; w < U; w++) {
+                    const uint32_t sl = t0 + w * BPS + gblk;
+                    act[w] = sl < nb;
+                    sidx[w] = act[w] ? sl : 0u;
+                    const uint32_t row = (uint32_t)__shfl((int)Jl, (int)sidx[w], WAVE) * 4 + h;
+                    const bool ok = act[w] && row < ncols;
+                    xv[w] = ok ? (double)x[(size_t)row * ldx + colq] : 0.0;
+                }
+#pragma unroll
+                for (int w = 0; w < U; w++) {
+                    const double av = act[w] ? sv[sidx[w] * 16 + o * 4 + h] : 0.0;
+                    acc = __builtin_amdgcn_mfma_f64_4x4x4f64(av, xv[w], acc, 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();  // the next batch overwrites the staged values
+        }
+        const uint32_t row = I * 4 + h;
+        if constexpr (BPS == 2) acc += lane_xor<8>(acc);  // the other block of the step: m ^ 2
+        if ((BPS == 1 || gblk == 0) && row < P.nrows_elem) y[(size_t)row * ldy + colq] = (T)acc;
+    }
+    }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// BCSR 4 x 4 FP32 blocks times 8 or 16 right-hand sides on the matrix cores
+// (the block-row product of spmv/1D/BCSR-nnz/dpu/task.c:337-370 over a 4 x K
+// panel of x per block).  v_mfma_f32_4x4x1_16b_f32 is 16 independent 4 x 4 x 1
+// products: product m takes A[i] from lane 4m + i and B[j] from lane 4m + j,
+// and lane 4m + j keeps D[v][j] in its register v.  Which right-hand side
+// column a lane's B stands for is free, so a lane takes V = K / 4 consecutive
+// columns and the instruction runs once per column q of them: lane 4 g + r
+// holds block g of the step (16 blocks) and columns V r .. V r + V - 1.  Its A
+// is row r of the block, one 16-byte load straight from the values, its B the
+// four x rows' pieces of 4 V bytes, and 4 V instructions take 16 blocks.  The
+// block slots' sums are joined by a scattered butterfly at the end of the row.
+// One column per lane and 4-byte loads of x, as the instruction's layout
+// suggests, takes more load instructions per block: 27-point stencil 48^3 x 4,
+// 8 columns 91 -> 74 us, 16 columns 122 -> 102 us; 20^3 x 4 16 -> 11 and
+// 19 -> 14 us.  (32 columns, 8 lanes per block: 151 us against 138 us for the
+// vector-ALU kernel below; both wait for x rows from the L2.)
+// ---------------------------------------------------------------------------
+template <int K>
+__global__ __launch_bounds__(TPB) void bcsr4_mfma_kernel(const Prob *__restrict__ probs,
+                                                         const uint32_t *__restrict__ unit_pid,
+                                                         const uint32_t *__restrict__ urow, Ptrs<float> io,
+                                                         uint32_t nunits) {
+    static_assert(K == 8 || K == 16, "8 or 16 right-hand sides per pass");
+    constexpr int V = K / 4, LPB = K / V, G = WAVE / LPB;  // columns per lane, lanes per block, blocks per step
+    constexpr int NW = TPB / WAVE;
+    typedef float FV __attribute__((ext_vector_type(V)));
+    const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
+    const int g = lane / LPB, r = lane % LPB;
+    for (uint32_t u = blockIdx.x; u < nunits; u += gridDim.x) {
+    const uint32_t pid = unit_pid[u];
+    const Prob P = probs[pid];
+    const gptr<const float> __restrict__ x = gp(io.x(pid, P));
+    const gptr<float> __restrict__ y = gp(io.y(pid, P));
+    const gptr<const uint32_t> __restrict__ rp = gp(P.ptr), cip = gp(P.cind);
+    const gptr<const float> __restrict__ bv = gp((const float *)P.val);
+    const int ldx = io.lx(P), ldy = io.ly(P);
+    const uint32_t r0 = urow[u + pid], r1 = urow[u + pid + 1];
+    const uint32_t ncols = P.ncols_elem;
+    auto rows = [&](auto whole_c) {
+    constexpr bool WHOLE = decltype(whole_c)::value;  // whole x pieces and whole block columns
+    // this wave's block rows r0 + wid + NW t: their block ranges in one load (64 rows a
+    // round), and the next row's first block columns loaded while a row runs
+    for (uint32_t R0 = r0 + wid; R0 < r1; R0 += NW * WAVE) {
+    const uint32_t nrw = min((uint32_t)WAVE, (r1 - R0 + NW - 1) / NW);
+    const uint32_t Il = R0 + NW * (uint32_t)lane;
+    const uint32_t bl = (uint32_t)lane < nrw ? rp[Il] : 0u, el = (uint32_t)lane < nrw ? rp[Il + 1] : 0u;
+    auto first_cols = [&](uint32_t t) {  // row t's first batch of block columns, one per lane
+        const uint32_t bb = (uint32_t)__builtin_amdgcn_readlane((int)bl, (int)t);
+        const uint32_t ee = (uint32_t)__builtin_amdgcn_readlane((int)el, (int)t);
+        return (uint32_t)lane < min((uint32_t)WAVE, ee - bb) ? ldg(cip + bb + lane) : 0u;
+    };
+    uint32_t Jn = first_cols(0);
+    for (uint32_t t = 0; t < nrw; t++) {
+        const uint32_t I = R0 + NW * t;
+        const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)bl, (int)t);
+        const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)el, (int)t);
+        const uint32_t Jfirst = Jn;
+        if (t + 1 < nrw) Jn = first_cols(t + 1);
+        f32x4 acc[V];
+#pragma unroll
+        for (int q = 0; q < V; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (uint32_t base = b; base < e; base += WAVE) {
+            const uint32_t nb = min((uint32_t)WAVE, e - base);
+            const uint32_t Jl = base == b ? Jfirst : ((uint32_t)lane < nb ? ldg(cip + base + lane) : 0u);
+            // (Two steps' loads in flight measured slower, 84 against 74 us at 8 columns: 87 VGPRs.)
+            auto step = [&](uint32_t t0, auto tail_c) {
+                constexpr bool TAIL = decltype(tail_c)::value;  // empty slots multiply zeros by zeros
+                const uint32_t sl = t0 + g;
+                const bool act = !TAIL || sl < nb;
+                const uint32_t sc = act ? sl : 0u;
+                const uint32_t J = (uint32_t)__shfl((int)Jl, (int)sc, WAVE);
+                float a[4];
+                FV xv[4];
+                ldg_n<float, 4>(bv + (size_t)(base + sc) * 16 + (lane % 4) * 4, a);
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const uint32_t col = J * 4 + c;
+                    if constexpr (WHOLE) {
+                        xv[c] = *(gptr<const FV>)(x + (size_t)col * ldx + V * r);
+                    } else {
+                        const bool ok = col < ncols;
+                        const gptr<const float> px = x + (size_t)(ok ? col : 0u) * ldx + V * r;
+#pragma unroll
+                        for (int q = 0; q < V; q++) xv[c][q] = ok ? px[q] : 0.f;
                     }
-#pragma unroll
-                    for (int w = 0; w < U; w++)
-#pragma unroll
-                        for (int c = 0; c < 4; c++) {
-                            const uint32_t col = J[w] * 4 + c;
-                            xb[w][c] = (act[w] && col < ncols) ? x[(size_t)col * ldx + q] : T(0);
-                        }
-#pragma unroll
-                    for (int w = 0; w < U; w++)
-#pragma unroll
-                        for (int c = 0; c < 4; c++)
-                            acc = __builtin_amdgcn_mfma_f32_4x4x1f32(act[w] ? a[w][c] : T(0), xb[w][c], acc, 0, 0, 0);
                 }
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int q = 0; q < V; q++)
+                        acc[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(act ? a[c] : 0.f, act ? xv[c][q] : 0.f, acc[q], 0, 0, 0);
+            };
+            uint32_t t0 = 0;
+            for (; t0 + G <= nb; t0 += G) step(t0, std::false_type{});
+            if (t0 < nb) step(t0, std::true_type{});
+        }
+        // sums over the block slots, scattered: each exchange hands over half of the sums a lane
+        // keeps, block rows by lane bits 5 and 4, then columns by bits 3 and 2
+        const bool hb = lane & 32, mb = lane & 16, lb = lane & 8, kb = lane & 4;
+        float h[2][V], d[V];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int q = 0; q < V; q++) {
+                const float keep = hb ? acc[q][i + 2] : acc[q][i], send = hb ? acc[q][i] : acc[q][i + 2];
+                h[i][q] = keep + lane_xor<32>(send);
             }
 #pragma unroll
-            for (int v = 0; v < 4; v++) acc[v] = xor_sum<K, WAVE>(acc[v]);
-            if (g == 0) {
+        for (int q = 0; q < V; q++) {
+            const float keep = mb ? h[1][q] : h[0][q], send = mb ? h[0][q] : h[1][q];
+            d[q] = keep + lane_xor<16>(send);
+        }
+        float o[V / 2];
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const uint32_t row = I * 4 + v;
-                    if (row < P.nrows_elem) y[(size_t)row * ldy + q] = acc[v];
-                }
-            }
+        for (int q = 0; q < V / 2; q++) {
+            const float keep = lb ? d[q + V / 2] : d[q], send = lb ? d[q] : d[q + V / 2];
+            o[q] = keep + lane_xor<8>(send);
+        }
+        uint32_t col = V * r + (lb ? V / 2 : 0);
+        const uint32_t row = I * 4 + (mb ? 1 : 0) + (hb ? 2 : 0);
+        if constexpr (K == 16) {
+            const float keep = kb ? o[1] : o[0], send = kb ? o[0] : o[1];
+            const float v = keep + lane_xor<4>(send);
+            if (row < P.nrows_elem) y[(size_t)row * ldy + col + (kb ? 1 : 0)] = v;
         } else {
-            constexpr int BPS = K == 8 ? 2 : 1;  // matrix blocks per instruction
-            constexpr int U = 4 / BPS;           // steps whose loads go out together
-            double *const sv = s_val[wid];
-            const int h = lane / 16, m = (lane / 4) % 4, o = lane % 4;
-            const int gblk = BPS == 2 ? m / 2 : 0;  // block of this product within the step
-            // right-hand side column of this lane (a relabelling, see above)
-            const int colq = K == 16 ? 4 * m + o : 4 * (m % 2) + o;
-            double acc = 0.0;
-            for (uint32_t base = b; base < e; base += NB64) {
-                const uint32_t nb = min((uint32_t)NB64, e - base);
-                // the batch's values to LDS in 16-byte chunks, its block columns to lanes
-                __builtin_amdgcn_wave_barrier();
-                for (uint32_t c = lane; c < nb * 8; c += WAVE)
-                    *(u32x4 *)(sv + c * 2) = __builtin_nontemporal_load((gptr<const u32x4>)(bv + (size_t)base * 16) + c);
-                const uint32_t Jl = base == b ? Jfirst : ((uint32_t)lane < nb ? ldg(cip + base + lane) : 0u);
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                for (uint32_t t0 = 0; t0 < nb; t0 += BPS * U) {
-                    double xv[U];
-                    bool act[U];
-                    uint32_t sidx[U];
-#pragma unroll
-                    for (int w = 0; w < U; w++) {
-                        const uint32_t sl = t0 + w * BPS + gblk;
-                        act[w] = sl < nb;
-                        sidx[w] = act[w] ? sl : 0u;
-                        const uint32_t row = (uint32_t)__shfl((int)Jl, (int)sidx[w], WAVE) * 4 + h;
-                        const bool ok = act[w] && row < ncols;
-                        xv[w] = ok ? (double)x[(size_t)row * ldx + colq] : 0.0;
-                    }
-#pragma unroll
-                    for (int w = 0; w < U; w++) {
-                        const double av = act[w] ? sv[sidx[w] * 16 + o * 4 + h] : 0.0;
-                        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(av, xv[w], acc, 0, 0, 0);
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();  // the next batch overwrites the staged values
-            }
-            const uint32_t row = I * 4 + h;
-            if constexpr (BPS == 2) acc += lane_xor<8>(acc);  // the other block of the step: m ^ 2
-            if ((BPS == 1 || gblk == 0) && row < P.nrows_elem) y[(size_t)row * ldy + colq] = (T)acc;
+            const float v = o[0] + lane_xor<4>(o[0]);
+            if (row < P.nrows_elem && !kb) y[(size_t)row * ldy + col] = v;
         }
     }
     }
+    };
+    if ((uintptr_t)io.x(pid, P) % sizeof(FV) == 0 && ldx % V == 0 && ncols % 4 == 0) rows(std::true_type{});
+    else rows(std::false_type{});
     }
 }
 

@@ -39,9 +39,11 @@ static int launch_main(const Work &w, hipStream_t s, Ptrs<T> io) {
         }
         if (w.kind == WK_BCSR_VEC) {
             if constexpr (__is_same(T, float) || __is_same(T, double)) {
-                if (w.R == 4 && w.C == 4) {  // 4 x 4 blocks: the matrix-core kernel (32 columns: vector ALUs)
+                if (w.R == 4 && w.C == 4) {  // 4 x 4 blocks: the matrix-core kernels (32 columns: vector ALUs)
                     if constexpr (K == 32)
                         hipLaunchKernelGGL((bcsr4_valu_kernel<T, 32>), grid, block, 0, s, w.d_prob, w.d_unit_pid, w.d_c0, io, w.nunits);
+                    else if constexpr (__is_same(T, float))
+                        hipLaunchKernelGGL((bcsr4_mfma_kernel<K>), grid, block, 0, s, w.d_prob, w.d_unit_pid, w.d_c0, io, w.nunits);
                     else
                         hipLaunchKernelGGL((bcsr_mfma_kernel<T, K>), grid, block, 0, s, w.d_prob, w.d_unit_pid, w.d_c0, io, w.nunits);
                     return hipGetLastError() == hipSuccess ? SP_OK : SP_ERR_HIP;
@@ -224,7 +226,10 @@ static int launch_main(const Work &w, hipStream_t s, Ptrs<T> io) {
     case WK_BCSR_VEC: {
         if constexpr (K == 8 && (__is_same(T, float) || __is_same(T, double))) {
             if (w.R == 4 && w.C == 4) {  // 4 x 4 blocks: the matrix-core kernel
-                hipLaunchKernelGGL((bcsr_mfma_kernel<T, 8>), grid, block, 0, s, w.d_prob, w.d_unit_pid, w.d_c0, io, w.nunits);
+                if constexpr (__is_same(T, float))
+                    hipLaunchKernelGGL((bcsr4_mfma_kernel<8>), grid, block, 0, s, w.d_prob, w.d_unit_pid, w.d_c0, io, w.nunits);
+                else
+                    hipLaunchKernelGGL((bcsr_mfma_kernel<T, 8>), grid, block, 0, s, w.d_prob, w.d_unit_pid, w.d_c0, io, w.nunits);
                 break;
             }
         }
