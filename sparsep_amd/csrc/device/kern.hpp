@@ -605,7 +605,7 @@ __global__ __launch_bounds__(HOT_TPB) void csr_hot_kernel(const Prob *__restrict
 // zeroed in even shares by all tiles.  The open end of a tile is its carry; which row
 // it belongs to is known to the plan (its run list).
 // ---------------------------------------------------------------------------
-constexpr uint32_t WIDE_GAP = 256;
+constexpr uint32_t WIDE_GAP = 4096;
 
 // Slot of row-order position pos: a thread's 16-byte pieces are exchanged by a
 // function of the thread, so that 16 neighbouring threads' reads of piece c

@@ -1006,6 +1006,25 @@ int build_bcsr_plan(sp_plan *p, const sp_bcsr *B) {
 // ---------------------------------------------------------------------------
 // BCOO (ids 7, 8)
 // ---------------------------------------------------------------------------
+// Even block rows of a BCOO matrix in the coalesced BCSR kernels: the same blocks with block-row
+// pointers in place of row indices, 16 block rows per unit, one launch and no carries.
+static int bcoo_rows(sp_plan *p, Prob P, const std::vector<uint32_t> &ptr) {
+    int rc;
+    void *d;
+    if ((rc = plan_upload(p, ptr.data(), ptr.size() * 4, &d))) return rc;
+    P.ptr = (const uint32_t *)d;
+    P.rind = nullptr;
+    std::vector<uint32_t> units;
+    for (uint32_t I = 0; I < P.nrows; I += 16) units.push_back(I);
+    units.push_back(P.nrows);
+    p->work.lanes = 0;
+    p->work.R = p->opts.row_block_size;
+    p->work.C = p->opts.col_block_size;
+    Builder b(p);
+    b.add(P, units, nullptr);
+    return b.finish(WK_BCSR_VEC, false, 1);
+}
+
 int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
     const size_t sv = sp_dtype_size(B->dtype);
     const uint32_t R = B->row_block_size, C = B->col_block_size;
@@ -1015,8 +1034,6 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
     Prob P{};
     int rc;
     void *d;
-    if ((rc = plan_upload(p, B->browind, nb * 4, &d))) return rc;
-    P.rind = (const uint32_t *)d;
     if ((rc = plan_upload(p, B->bcolind, nb * 4, &d))) return rc;
     P.cind = (const uint32_t *)d;
     if ((rc = plan_upload(p, B->bval, nb * rc2 * sv, &d))) return rc;
@@ -1025,6 +1042,35 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
     P.nent = (uint32_t)nb;
     P.nrows_elem = B->nrows;
     P.ncols_elem = B->ncols;
+    // Automatic plans, no knob asked for, with even block rows of a shape the coalesced BCSR
+    // kernel takes: several right-hand sides run as block rows (the block-balanced kernel takes
+    // one per pass), and so does one where that is faster (27-point stencil, 4 x 4 blocks, us
+    // block balanced -> block rows: FP64 9^3 11.0 -> 5.3, 37^3 51.0 -> 34.6, 52^3 133 -> 97; FP32
+    // 16^3 10.3 -> 6.9, 24^3 12.5 -> 10.1, 37^3 23.1 -> 23.4, 52^3 53.2 -> 57.8; INT8 24^3
+    // 10.1 -> 7.3): 8-byte values, and others up to a million blocks.
+    const sp_opts &o = p->opts;
+    if (p->algo == SP_ALGO_AUTO && nb && !o.nparts && !o.nsub && !o.lanes_per_row && !o.items_per_lane && !o.lds_slice &&
+        !o.mem_cap_bytes) {
+        std::vector<uint32_t> ptr((size_t)P.nrows + 1, 0);
+        for (uint64_t k = 0; k < nb; k++) ptr[B->browind[k] + 1]++;
+        const uint32_t maxlen = *std::max_element(ptr.begin(), ptr.end());
+        const double avg = (double)nb / P.nrows;
+        for (uint32_t I = 0; I < P.nrows; I++) ptr[I + 1] += ptr[I];
+        if (maxlen <= 4 * avg + 64 && coal_ok(B->dtype, R, C, avg)) {
+            if ((rc = bcoo_rows(p, P, ptr))) return rc;
+            if (sv == 8 || nb <= 1u << 20) {
+                p->algo = SP_ALGO_VECTOR;
+                p->lanes = 64;
+                p->nparts = 1;
+                p->nsub = p->work.nunits;
+                return SP_OK;
+            }
+            p->many = std::make_unique<PlanWork>(std::move(*static_cast<PlanWork *>(p)));
+            static_cast<PlanWork &>(*p) = PlanWork{};
+        }
+    }
+    if ((rc = plan_upload(p, B->browind, nb * 4, &d))) return rc;
+    P.rind = (const uint32_t *)d;
     const bool atom = p->algo == SP_ALGO_SEGMENTED_ATOMIC;
     p->algo = atom ? SP_ALGO_SEGMENTED_ATOMIC : SP_ALGO_SEGMENTED;
     p->work.R = R;
@@ -1184,7 +1230,10 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
         // Even rows take wide tiles as in 1D; skewed ones keep the kernels whose sums have the same
         // bits as those over LDS slices of x.  (A plan's tiles are sorted one launch each: 16K
         // entries per tile at least.)
-        if (A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64)
+        // CSR from 1M entries: a fix-up more than the row kernel's two launches (RBDCSR, 15000 x 33
+        // uniform FP32 9.3 against 12.0 us, banded 76952 x 33 INT32 18.2 -> 13.8 us).
+        if (A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64 &&
+            (tk.format == SP_FMT_COO || A->nnz >= 1u << 20))
             wide = wide_shape(p, tk.format == SP_FMT_COO, false, A->colind, n, A->nnz);
     }
     if (sorted) sp_free_coo(sorted);
@@ -1472,14 +1521,14 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
         // Wide tiles for one right-hand side, as for 1D CSR/COO: stripes leave about half of a
         // local matrix's rows empty in each, which cost a row map's word and no row of the row
         // kernel.  (While the arrays on the device are row ordered.)
-        if (wide.nt) {
+        // An empty tile's rows need the partial buffer zeroed first, as COO tilings do anyway; CSR
+        // ones keep the row kernel then (DCSR, banded 76952 x 33 INT32: 21.1 against 25.3 us).
+        for (const Prob &Q : b.probs) wide_zero |= Q.nent == 0 && Q.nrows > 0;
+        if (wide.nt && !(wide_zero && tk.format == SP_FMT_CSR)) {
             std::vector<uint32_t> rp;
             for (uint32_t t = 0; t < nt && !rc; t++) {
                 const Prob &Q = b.probs[t];
-                if (Q.nent == 0) {
-                    wide_zero |= Q.nrows > 0;  // its rows of the partial buffer are zeroed first
-                    continue;
-                }
+                if (Q.nent == 0) continue;
                 const uint32_t *hrp;
                 if (tk.format == SP_FMT_CSR) {
                     hrp = T->drowptr + (size_t)t * (th + 1);
