@@ -366,6 +366,29 @@ double row_lines(const uint32_t *colind, uint32_t nnz, size_t sv) {
     return (double)lines / (64.0 * windows);
 }
 
+// Every knob that picks a kernel left alone, and no memory cap (which keeps one copy).
+bool no_knobs(const sp_opts &o) {
+    return !o.items_per_lane && !o.lanes_per_row && !o.nparts && !o.nsub && !o.lds_slice && !o.mem_cap_bytes;
+}
+
+// Widths (bit i: 2^i right-hand sides) at which even CSR rows run as panels and not in the row
+// kernels (us, rows -> panel): rows of 16 to 64 entries with 4- and 8-byte values while a row of x
+// is at most 64 bytes (250000 x 33 banded INT32: 2 columns 38.2 -> 21.2, 8 columns 49.4 -> 46.7;
+// 200000 x 33 uniform: 8 columns 80 -> 61.5; 60000 x 33 banded INT64 8 columns 36.4 -> 25.0),
+// wider ones only for small matrices (32 columns: 10000 x 33 25.6 -> 11.2, 250000 x 33 99 -> 144);
+// shorter rows where the row kernel spreads a wave over the columns of one row (x rows of 64
+// bytes and more; 5-point stencil 500^2: 16 columns 75.4 -> 22.7, INT64 8 columns 113 -> 22.1, but
+// 8 columns INT32 12.5 -> 15.5); longer rows never (27-point stencil: 18.4 -> 30.8).
+uint32_t panel_widths(double avg, uint32_t nnz, size_t sv) {
+    uint32_t mask = 0;
+    for (uint32_t i = 1; i <= 5; i++) {
+        const size_t bytes = sv << i;
+        const bool use = avg < 16 ? bytes >= 64 : avg <= 64 && sv >= 4 && (bytes <= 64 || nnz <= 1u << 20);
+        mask |= (uint32_t)use << i;
+    }
+    return mask;
+}
+
 // Whether an automatic 1D CSR/COO plan takes wide tiles, and which.  Against the kernels that
 // the row-ordered group would take (us per SpMV, before -> wide):
 //   skewed rows and COO from 2K entries on: R-MAT 2^12 x 8 FP32 CSR 8.4 -> 6.5, 2^16 x 16
@@ -385,10 +408,7 @@ double row_lines(const uint32_t *colind, uint32_t nnz, size_t sv) {
 // 8 per thread (20.1 against 24.3).
 WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
     const sp_opts &o = p->opts;
-    // any knob asked for keeps its kernel; a memory cap keeps one copy of the matrix
-    if (p->algo != SP_ALGO_AUTO || o.items_per_lane || o.lanes_per_row || o.nparts || o.nsub || o.lds_slice ||
-        o.mem_cap_bytes)
-        return {};
+    if (p->algo != SP_ALGO_AUTO || !no_knobs(o)) return {};
     const uint32_t least = coo || skewed ? 2u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
     if (nnz < least) return {};
     const bool scattered = row_lines(colind, nnz, sp_dtype_size(p->dtype)) > 0.3;
@@ -749,11 +769,17 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     const int algo = p->algo;
     WideShape s;
     int rc = build_csr_group(p, A, &s);
-    if (rc || !s.nt) return rc;
-    rc = add_wide(p, A->rowptr, s);
-    if (rc != SP_ERR_RANGE) return rc;
-    drop_groups(p, opts, algo);
-    return build_csr_group(p, A, nullptr);
+    if (!rc && s.nt && (rc = add_wide(p, A->rowptr, s)) == SP_ERR_RANGE) {
+        drop_groups(p, opts, algo);
+        rc = build_csr_group(p, A, nullptr);
+    }
+    // even rows (their group is the row kernels' either way): panels at some widths
+    const PlanWork &rows = p->many ? *p->many : *p;
+    if (rc || algo != SP_ALGO_AUTO || !no_knobs(opts) || rows.work.kind != WK_CSR_VEC || A->nnz < 16u << 10) return rc;
+    p->panel_widths = panel_widths((double)A->nnz / A->nrows, A->nnz, sp_dtype_size(A->dtype));
+    if (!p->panel_widths) return SP_OK;
+    p->panel = std::make_unique<PlanWork>(rows);
+    return build_panel(p, *p->panel, A->rowptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1049,8 +1075,7 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
     // 16^3 10.3 -> 6.9, 24^3 12.5 -> 10.1, 37^3 23.1 -> 23.4, 52^3 53.2 -> 57.8; INT8 24^3
     // 10.1 -> 7.3): 8-byte values, and others up to a million blocks.
     const sp_opts &o = p->opts;
-    if (p->algo == SP_ALGO_AUTO && nb && !o.nparts && !o.nsub && !o.lanes_per_row && !o.items_per_lane && !o.lds_slice &&
-        !o.mem_cap_bytes) {
+    if (p->algo == SP_ALGO_AUTO && nb && no_knobs(o)) {
         std::vector<uint32_t> ptr((size_t)P.nrows + 1, 0);
         for (uint64_t k = 0; k < nb; k++) ptr[B->browind[k] + 1]++;
         const uint32_t maxlen = *std::max_element(ptr.begin(), ptr.end());
