@@ -35,6 +35,9 @@ std::vector<spd::Run> crossing_runs(int kind, const std::vector<Prob> &probs, co
 
 namespace {
 
+// Bytes that an array of n bytes takes inside a shared allocation: aligned, with 32 readable past its end.
+size_t piece(size_t n) { return (n + 32 + 255) & ~(size_t)255; }
+
 size_t acc_size(int dt) { return (dt == SP_I64 || dt == SP_F64) ? 8 : 4; }
 
 struct Builder {
@@ -74,7 +77,8 @@ struct Builder {
         if ((rc = plan_upload(p, unit_pid.data(), unit_pid.size() * 4, (void **)&w.d_unit_pid))) return rc;
         if ((rc = plan_upload(p, c0.data(), c0.size() * 4, (void **)&w.d_c0))) return rc;
         if (!c1.empty() && (rc = plan_upload(p, c1.data(), c1.size() * 4, (void **)&w.d_c1))) return rc;
-        if (!c2.empty() && (rc = plan_upload(p, c2.data(), c2.size() * 4, (void **)&w.d_c2))) return rc;
+        // (wide tiles: c2 and the carried rows stay with the host, in the run list)
+        if (!c2.empty() && kind != WK_WIDE && (rc = plan_upload(p, c2.data(), c2.size() * 4, (void **)&w.d_c2))) return rc;
         w.nzero = (uint32_t)zrow.size();
         if (w.nzero) {
             if ((rc = plan_upload(p, zpid.data(), zpid.size() * 4, (void **)&w.d_zpid))) return rc;
@@ -85,7 +89,7 @@ struct Builder {
             // atomic merges write no carries (batches allocate their own)
             if (p->algo != SP_ALGO_SEGMENTED_ATOMIC) {
                 const size_t n = (size_t)std::max<uint32_t>(w.nunits, 1) * slots;
-                if ((rc = plan_alloc(p, n * 4, (void **)&w.d_carry_row))) return rc;
+                if (kind != WK_WIDE && (rc = plan_alloc(p, n * 4, (void **)&w.d_carry_row))) return rc;
                 if ((rc = plan_alloc(p, n * w.carry_k * acc_size(p->dtype), &w.d_carry_val))) return rc;
             }
         }
@@ -410,7 +414,7 @@ WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *co
     const sp_opts &o = p->opts;
     if (p->algo != SP_ALGO_AUTO || !no_knobs(o)) return {};
     const uint32_t least = coo || skewed ? 2u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
-    if (nnz < least) return {};
+    if (nnz < least || nnz > 0xF0000000u) return {};  // (entry numbers plus a tile stay below 2^32)
     const bool scattered = row_lines(colind, nnz, sp_dtype_size(p->dtype)) > 0.3;
     if (acc_size(p->dtype) == 8) return scattered && nnz >= 2u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
     if (scattered && nnz >= 3u << 20) return {1024, 16};
@@ -444,27 +448,42 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
     g.work.dtype = p->dtype;
     g.work.nprob = g.work.nunits = 1;
     g.work.panel_nent = nnz;
-    int rc;
-    void *d;
-    if ((rc = plan_upload(p, word.data(), word.size() * 4, &d))) return rc;
-    P.ptr = (const uint32_t *)d;
-    if ((rc = plan_upload(p, rows.data(), rows.size() * 4, &d))) return rc;
-    P.rind = (const uint32_t *)d;
-    if ((rc = plan_upload(p, zrows.data(), zrows.size() * 4, &d))) return rc;
-    P.hcol = (const uint32_t *)d;
-    P.nhcol = (uint32_t)zrows.size();
-    if ((rc = plan_upload(p, &P, sizeof(P), (void **)&g.work.d_prob))) return rc;
+    // one block: words, rows, rows without entries, the crossing rows of every width, descriptor
+    std::vector<spd::Cross> lists[6];
     uint64_t carries = 0;
+    size_t o_rows = piece(word.size() * 4), o_zrows = o_rows + piece(rows.size() * 4);
+    size_t o_list[7] = {o_zrows + piece(zrows.size() * 4)};
     for (int i = 0; i < 6; i++) {
         const uint32_t E = spd::panel_entries(1 << i, sa);
-        std::vector<spd::Cross> c;
         for (const spd::Cross &C : cross)
-            if (C.b / E != C.e / E) c.push_back(C);
-        g.work.ncross[i] = (uint32_t)c.size();
-        if ((rc = plan_upload(p, c.data(), c.size() * sizeof(spd::Cross), (void **)&g.work.d_cross[i]))) return rc;
+            if (C.b / E != C.e / E) lists[i].push_back(C);
+        g.work.ncross[i] = (uint32_t)lists[i].size();
+        o_list[i + 1] = o_list[i] + piece(lists[i].size() * sizeof(spd::Cross));
         carries = std::max(carries, (((uint64_t)nnz + E - 1) / E) << i);
     }
-    if ((rc = plan_alloc(p, carries * sa, &g.work.d_carry_val))) return rc;
+    int rc;
+    void *d;
+    if ((rc = plan_alloc(p, o_list[6] + sizeof(Prob), &d)) || (rc = plan_alloc(p, carries * sa, &g.work.d_carry_val)))
+        return rc;
+    char *const dev = (char *)d;
+    P.ptr = (const uint32_t *)dev;
+    P.rind = (const uint32_t *)(dev + o_rows);
+    P.hcol = (const uint32_t *)(dev + o_zrows);
+    P.nhcol = (uint32_t)zrows.size();
+    std::vector<char> host(o_list[6] + sizeof(Prob), 0);
+    auto put = [&](size_t at, const void *src, size_t n) {
+        if (n) memcpy(host.data() + at, src, n);
+    };
+    put(0, word.data(), word.size() * 4);
+    put(o_rows, rows.data(), rows.size() * 4);
+    put(o_zrows, zrows.data(), zrows.size() * 4);
+    for (int i = 0; i < 6; i++) {
+        put(o_list[i], lists[i].data(), lists[i].size() * sizeof(spd::Cross));
+        g.work.d_cross[i] = (spd::Cross *)(dev + o_list[i]);
+    }
+    put(o_list[6], &P, sizeof(P));
+    g.work.d_prob = (Prob *)(dev + o_list[6]);
+    SP_HIP_TRY(hipMemcpy(d, host.data(), host.size(), hipMemcpyHostToDevice));
     g.h_probs = {P};
     g.h_cross = std::move(cross);
     return SP_OK;
@@ -536,13 +555,17 @@ int wide_part(sp_plan *p, const Prob &rows, const uint32_t *rowptr, WideShape s,
         }
     }
     cent.push_back(nnz);
+    // two allocations: what the sort writes (keys, values, bases, flag) and what the host has
+    // (words, row map); each piece aligned, with the slack that plan_alloc gives an array
     int rc;
-    void *key, *val, *base, *drmap, *dword, *flag;
-    if ((rc = plan_alloc(p, tot * 4, &key)) || (rc = plan_alloc(p, tot * sv, &val)) ||
-        (rc = plan_alloc(p, tot / 64 * 4, &base)) || (rc = plan_alloc(p, 4, &flag)) ||
-        (rc = plan_upload(p, rmap.data(), rmap.size() * 2, &drmap)) ||
-        (rc = plan_upload(p, word.data(), word.size() * 4, &dword)))
-        return rc;
+    const size_t o_val = piece(tot * 4), o_base = o_val + piece(tot * sv), o_flag = o_base + piece(tot / 64 * 4);
+    std::vector<char> host(piece(word.size() * 4) + rmap.size() * 2);
+    memcpy(host.data(), word.data(), word.size() * 4);
+    if (!rmap.empty()) memcpy(host.data() + piece(word.size() * 4), rmap.data(), rmap.size() * 2);
+    void *sorted, *tables;
+    if ((rc = plan_alloc(p, o_flag + 4, &sorted)) || (rc = plan_upload(p, host.data(), host.size(), &tables))) return rc;
+    char *const key = (char *)sorted, *const val = key + o_val, *const base = key + o_base, *const flag = key + o_flag;
+    char *const dword = (char *)tables, *const drmap = dword + piece(word.size() * 4);
     // on the null stream, as the uploads before it
     if ((rc = launch_wide_sort(nullptr, P.cind, P.val, sv, nnz, tile, words, pb, s.ipt, sa, (uint32_t *)key, val,
                                (uint32_t *)base, (uint32_t *)flag)))
@@ -775,7 +798,9 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     }
     // even rows (their group is the row kernels' either way): panels at some widths
     const PlanWork &rows = p->many ? *p->many : *p;
-    if (rc || algo != SP_ALGO_AUTO || !no_knobs(opts) || rows.work.kind != WK_CSR_VEC || A->nnz < 16u << 10) return rc;
+    if (rc || algo != SP_ALGO_AUTO || !no_knobs(opts) || rows.work.kind != WK_CSR_VEC || A->nnz < 16u << 10 ||
+        A->nnz > 0xF0000000u)
+        return rc;
     p->panel_widths = panel_widths((double)A->nnz / A->nrows, A->nnz, sp_dtype_size(A->dtype));
     if (!p->panel_widths) return SP_OK;
     p->panel = std::make_unique<PlanWork>(rows);

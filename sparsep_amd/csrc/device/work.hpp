@@ -21,8 +21,7 @@ struct Work {
     spd::Prob *d_prob = nullptr;
     uint32_t *d_unit_pid = nullptr;
     uint32_t *d_c0 = nullptr, *d_c1 = nullptr;  // coordinates, index unit + pid
-    uint32_t *d_c2 = nullptr;                   // hot-x CSR: staged entries per tile; wide tiles: row
-                                                // carried out (NONE: none); index unit + pid
+    uint32_t *d_c2 = nullptr;                   // hot-x CSR: staged entries per tile, index unit + pid
     uint32_t hcol_max = 0;                      // hot-x CSR: largest staged-column count of the problems
     uint32_t ipt = 8, lanes = 1, R = 1, C = 1;  // (wide tiles: lanes = threads per workgroup)
     uint32_t *d_carry_row = nullptr;
