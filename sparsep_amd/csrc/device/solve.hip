@@ -15,13 +15,13 @@ constexpr int RB = 256;      // reduction block
 constexpr int RGRID = 1024;  // partial sums per dot product
 constexpr int AHEAD = 2;     // iterations queued beyond the last one known to be done
 
-// What the kernels of a solve share.  Two slots of each scalar alternate between iterations, so
-// that a kernel's blocks, which all form the same scalar from the partial sums, never read one
-// that another block of the same kernel writes.
+// What the kernels of a solve share.  The kernels of iteration it read slot it % 2 of rr and stop;
+// cg_turn, the last of them, writes the other slot.  So no thread reads a word that the same kernel
+// writes, and all threads of a kernel take the same side of a test of stop (barriers lie behind it).
 struct CgState {
-    double rr[2];  // r.r at the start of iteration it (slot it % 2)
+    double rr[2];  // r.r at the start of iteration it
     double bb, pq;
-    int stop;      // 0 running, 1 ended (converged or maxit), 2 not positive definite
+    int stop[2];   // at the start of iteration it: 0 running, 1 ended (converged or maxit), 2 not positive definite
 };
 
 // Where the host reads a solve's progress while it runs (pinned host memory).
@@ -99,17 +99,18 @@ __global__ __launch_bounds__(RB) void cg_begin(const double *__restrict__ part_b
     if (threadIdx.x == 0) {
         st->bb = bb;
         st->rr[0] = rr;
-        st->stop = maxit <= 0 || converged(rr, bb, rtol);
-        tell(note, 0, st->stop, rr, bb);
+        const int stop = maxit <= 0 || converged(rr, bb, rtol);
+        st->stop[0] = stop;
+        tell(note, 0, stop, rr, bb);
     }
 }
 
 // partial sums of p.q
 template <typename T>
 __global__ __launch_bounds__(RB) void cg_dot(const T *__restrict__ a, const T *__restrict__ b, uint64_t n,
-                                             double *__restrict__ part, const CgState *__restrict__ st) {
+                                             double *__restrict__ part, const CgState *__restrict__ st, int it) {
     __shared__ double s[RB];
-    if (st->stop) return;
+    if (st->stop[it & 1]) return;
     double acc = 0.0;
     for (uint64_t i = (uint64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * RB)
         acc += (double)a[i] * (double)b[i];
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(RB) void cg_step(T *__restrict__ x, T *__restrict__
                                               const T *__restrict__ q, uint64_t n, const double *__restrict__ part_pq,
                                               double *__restrict__ part_r, CgState *__restrict__ st, int it) {
     __shared__ double s[RB];
-    if (st->stop) return;
+    if (st->stop[it & 1]) return;
     const double pq = sum_partials(part_pq, s);
     if (blockIdx.x == 0 && threadIdx.x == 0) st->pq = pq;  // (read by cg_turn)
     if (!(pq > 0)) return;  // not positive definite: cg_turn stops the solve
@@ -139,18 +140,23 @@ __global__ __launch_bounds__(RB) void cg_step(T *__restrict__ x, T *__restrict__
     if (threadIdx.x == 0) part_r[blockIdx.x] = acc;
 }
 
-// beta = new r.r / old r.r; p = r + beta p; block 0 counts the iteration.  (A block that starts
-// after block 0 has stopped the solve leaves p as it is; nothing reads p then.)
+// beta = new r.r / old r.r; p = r + beta p; block 0 counts the iteration and hands the state on to
+// the next one's slot, also when the solve has stopped.
 template <typename T>
 __global__ __launch_bounds__(RB) void cg_turn(T *__restrict__ p, const T *__restrict__ r, uint64_t n,
                                               const double *__restrict__ part_r, CgState *__restrict__ st,
                                               CgNote *__restrict__ note, double rtol, int it, int maxit) {
     __shared__ double s[RB];
-    if (st->stop) return;
+    const int ended = st->stop[it & 1];
+    int *const next = &st->stop[(it + 1) & 1];
+    if (ended) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *next = ended;
+        return;
+    }
     const double pq = st->pq, rr = st->rr[it & 1];
     if (!(pq > 0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            st->stop = 2;
+            *next = 2;
             tell(note, it, 2, rr, st->bb);
         }
         return;
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(RB) void cg_turn(T *__restrict__ p, const T *__rest
         const double bb = st->bb;
         const int stop = it + 1 >= maxit || converged(rr1, bb, rtol);
         st->rr[(it + 1) & 1] = rr1;
-        if (stop) st->stop = 1;
+        *next = stop;
         tell(note, it + 1, stop, rr1, bb);
     }
     const T beta = (T)(rr1 / rr);
@@ -220,7 +226,7 @@ int cg_t(sp_plan *A, const T *b, T *x, int maxit, double rtol, int *iters, doubl
         if (it >= AHEAD && !await_note(note, it - AHEAD, s)) { rc = SP_ERR_HIP; break; }
         if (__atomic_load_n(&note->stop, __ATOMIC_ACQUIRE)) break;
         if ((rc = sp_spmv(A, p, q))) break;
-        hipLaunchKernelGGL(cg_dot<T>, g, t, 0, s, p, q, n, part_pq, st);
+        hipLaunchKernelGGL(cg_dot<T>, g, t, 0, s, p, q, n, part_pq, st, it);
         hipLaunchKernelGGL(cg_step<T>, g, t, 0, s, x, r, p, q, n, part_pq, part_r, st, it);
         hipLaunchKernelGGL(cg_turn<T>, g, t, 0, s, p, r, n, part_r, st, note, rtol, it, maxit);
         if (hipGetLastError() != hipSuccess) rc = SP_ERR_HIP;
