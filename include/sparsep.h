@@ -15,9 +15,12 @@
  * Conventions: every function returns 0 (SP_OK) or a negative sp_status;
  * nothing aborts.  The caller owns host matrices and vectors; a plan owns
  * its device copy of the matrix; a context owns its stream.  A context is
- * not thread-safe: use one per host thread.  Values are untyped pointers
- * tagged by sp_dtype; integers use two's-complement wraparound exactly as
- * C `val_dt` arithmetic does under gcc (support/utils.h:13-34).
+ * not thread-safe: use one per host thread.  The exceptions are sp_spmv,
+ * sp_spmm and sp_cg, which several threads may call at the same time, also
+ * on one plan: each product enters the context's stream as a whole.  Values
+ * are untyped pointers tagged by sp_dtype; integers use two's-complement
+ * wraparound exactly as C `val_dt` arithmetic does under gcc
+ * (support/utils.h:13-34).
  */
 #ifndef SPARSEP_H
 #define SPARSEP_H
@@ -515,8 +518,9 @@ int sp_plan_get_info(const sp_plan *plan, sp_plan_info *info);
  * Replaces x push + dpu_launch + y pull + host merge
  * (spmv/1D/CSR-row/host/app.c:257-287, spmv/2D/DCSR/host/app.c:340-351).
  * A plan keeps per-call device state (carry slots, partial vectors, the
- * staged x of hot-x plans), so calls on one plan are ordered on its
- * context's stream; run two plans to overlap work on two streams. */
+ * staged x of hot-x plans), so calls on one plan, of one thread or of
+ * several, are ordered on its context's stream; run two plans to overlap
+ * work on two streams. */
 int sp_spmv(sp_plan *plan, const void *x, void *y);
 
 /* Y = A X for k right-hand sides; X is ncols x k row-major with leading

@@ -7,6 +7,7 @@
 
 #include <atomic>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "sparsep.h"
@@ -83,6 +84,11 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
     uint32_t ypart_k = 0;     // right-hand sides ypart currently holds
 
     std::vector<void *> allocs;
+
+    // Held while a call's launches are enqueued: carries, staged x and ypart belong to the plan, so
+    // a second thread's launches must not fall between a tile kernel and the fix-up that reads its
+    // carries.  The stream orders the calls after that.
+    std::mutex run_lock;
 
     CgBuf cg;  // kept between solves, used by one at a time
     std::atomic<bool> cg_busy{false};

@@ -1172,6 +1172,7 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
 // ---------------------------------------------------------------------------
 int run_plan(sp_plan *p, const void *x, void *y, int k, int ldx, int ldy) {
     if (p->nrows == 0) return SP_OK;
+    const std::lock_guard<std::mutex> hold(p->run_lock);
     if (!p->tiled) return run_work(p->group(k).work, p->ctx, x, y, nullptr, nullptr, k, ldx, ldy);
     // 2D: partial rows per stripe into ypart, then the stripe-order reduction.
     const uint64_t need = (uint64_t)p->vert * p->nrows * (uint64_t)k * sp_dtype_size(p->dtype);
