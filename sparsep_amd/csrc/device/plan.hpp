@@ -83,7 +83,11 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
     uint64_t ypart_bytes = 0;
     uint32_t ypart_k = 0;     // right-hand sides ypart currently holds
 
-    std::vector<void *> allocs;
+    struct Alloc {
+        void *dev;
+        uint64_t bytes;
+    };
+    std::vector<Alloc> allocs;
 
     // Held while a call's launches are enqueued: carries, staged x and ypart belong to the plan, so
     // a second thread's launches must not fall between a tile kernel and the fix-up that reads its
@@ -94,7 +98,9 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
     std::atomic<bool> cg_busy{false};
 };
 
-// Allocation helpers (record in plan->allocs, respect mem_cap_bytes).
+// Allocation helpers (record in plan->allocs, respect mem_cap_bytes); plan_release frees the
+// allocations from number `from` up to `to`.
+void plan_release(sp_plan *p, size_t from, size_t to);
 int plan_alloc(sp_plan *p, size_t bytes, void **out);
 int plan_upload(sp_plan *p, const void *host, size_t bytes, void **out);
 

@@ -422,7 +422,7 @@ WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *co
 }
 
 // Makes a row-ordered CSR or COO group (one problem) the group for several right-hand sides with
-// uneven rows: panels over the same columns and values.
+// uneven rows: panels over the same columns and values.  The group stays as it is on an error.
 int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
     const size_t sa = acc_size(p->dtype);
     Prob P = g.h_probs[0];
@@ -443,11 +443,11 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
         word[2 * (size_t)w + 1] = n;
         n += (uint32_t)__builtin_popcount(word[2 * (size_t)w]);
     }
-    g = PlanWork{};
-    g.work.kind = WK_PANEL;
-    g.work.dtype = p->dtype;
-    g.work.nprob = g.work.nunits = 1;
-    g.work.panel_nent = nnz;
+    PlanWork n;
+    n.work.kind = WK_PANEL;
+    n.work.dtype = p->dtype;
+    n.work.nprob = n.work.nunits = 1;
+    n.work.panel_nent = nnz;
     // one block: words, rows, rows without entries, the crossing rows of every width, descriptor
     std::vector<spd::Cross> lists[6];
     uint64_t carries = 0;
@@ -457,14 +457,18 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
         const uint32_t E = spd::panel_entries(1 << i, sa);
         for (const spd::Cross &C : cross)
             if (C.b / E != C.e / E) lists[i].push_back(C);
-        g.work.ncross[i] = (uint32_t)lists[i].size();
+        n.work.ncross[i] = (uint32_t)lists[i].size();
         o_list[i + 1] = o_list[i] + piece(lists[i].size() * sizeof(spd::Cross));
         carries = std::max(carries, (((uint64_t)nnz + E - 1) / E) << i);
     }
-    int rc;
     void *d;
-    if ((rc = plan_alloc(p, o_list[6] + sizeof(Prob), &d)) || (rc = plan_alloc(p, carries * sa, &g.work.d_carry_val)))
+    const size_t mark = p->allocs.size();
+    int rc = plan_alloc(p, o_list[6] + sizeof(Prob), &d);
+    if (!rc) rc = plan_alloc(p, carries * sa, &n.work.d_carry_val);
+    if (rc) {
+        plan_release(p, mark, p->allocs.size());
         return rc;
+    }
     char *const dev = (char *)d;
     P.ptr = (const uint32_t *)dev;
     P.rind = (const uint32_t *)(dev + o_rows);
@@ -479,13 +483,14 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
     put(o_zrows, zrows.data(), zrows.size() * 4);
     for (int i = 0; i < 6; i++) {
         put(o_list[i], lists[i].data(), lists[i].size() * sizeof(spd::Cross));
-        g.work.d_cross[i] = (spd::Cross *)(dev + o_list[i]);
+        n.work.d_cross[i] = (spd::Cross *)(dev + o_list[i]);
     }
     put(o_list[6], &P, sizeof(P));
-    g.work.d_prob = (Prob *)(dev + o_list[6]);
+    n.work.d_prob = (Prob *)(dev + o_list[6]);
     SP_HIP_TRY(hipMemcpy(d, host.data(), host.size(), hipMemcpyHostToDevice));
-    g.h_probs = {P};
-    g.h_cross = std::move(cross);
+    n.h_probs = {P};
+    n.h_cross = std::move(cross);
+    g = std::move(n);
     return SP_OK;
 }
 
@@ -601,6 +606,11 @@ int finish_wide(sp_plan *p, const std::vector<WidePart> &parts, WideShape s) {
     return b.finish(WK_WIDE, true, 1);
 }
 
+// Wide tiles and panels are second layouts of a matrix that is on the device already: a plan goes
+// without one that its columns or the device's memory have no room for.
+bool unfit(int rc) { return rc == SP_ERR_RANGE || rc == SP_ERR_NOMEM; }
+int optional(int rc) { return unfit(rc) ? SP_OK : rc; }
+
 // Gives a 1D plan whose row-ordered group is built wide tiles for one right-hand side; its
 // columns and values also serve several.
 int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
@@ -608,16 +618,16 @@ int add_wide(sp_plan *p, const uint32_t *rowptr, WideShape s) {
     int rc = wide_part(p, p->h_probs[0], rowptr, s, part[0]);
     if (rc || (rc = finish_wide(p, part, s))) return rc;
     p->ntiles = p->work.nunits;
-    return takes_panel(p) ? build_panel(p, *p->many, rowptr) : SP_OK;
+    return takes_panel(p) ? optional(build_panel(p, *p->many, rowptr)) : SP_OK;
 }
 
 // Undoes a plan's groups (a wide layout that did not fit).
 void drop_groups(sp_plan *p, const sp_opts &opts, int algo) {
-    for (void *d : p->allocs) (void)hipFree(d);
-    p->allocs.clear();
-    p->device_bytes = 0;
+    plan_release(p, 0, p->allocs.size());
     p->many.reset();
     static_cast<PlanWork &>(*p) = PlanWork{};
+    p->d_ypart = nullptr;
+    p->ypart_bytes = 0;
     p->opts = opts;
     p->algo = algo;
 }
@@ -792,7 +802,7 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     const int algo = p->algo;
     WideShape s;
     int rc = build_csr_group(p, A, &s);
-    if (!rc && s.nt && (rc = add_wide(p, A->rowptr, s)) == SP_ERR_RANGE) {
+    if (!rc && s.nt && unfit(rc = add_wide(p, A->rowptr, s))) {
         drop_groups(p, opts, algo);
         rc = build_csr_group(p, A, nullptr);
     }
@@ -804,7 +814,11 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     p->panel_widths = panel_widths((double)A->nnz / A->nrows, A->nnz, sp_dtype_size(A->dtype));
     if (!p->panel_widths) return SP_OK;
     p->panel = std::make_unique<PlanWork>(rows);
-    return build_panel(p, *p->panel, A->rowptr);
+    if ((rc = build_panel(p, *p->panel, A->rowptr))) {
+        p->panel.reset();
+        p->panel_widths = 0;
+    }
+    return optional(rc);
 }
 
 // ---------------------------------------------------------------------------
@@ -948,7 +962,7 @@ int build_coo_plan(sp_plan *p, const sp_coo *A) {
     int rc = build_coo_group(p, A, &s, rowptr);
     if (rc || !s.nt) return rc;
     rc = add_wide(p, rowptr.data(), s);
-    if (rc != SP_ERR_RANGE) return rc;
+    if (!unfit(rc)) return rc;
     drop_groups(p, opts, algo);
     return build_coo_group(p, A, nullptr, rowptr);
 }
@@ -1076,7 +1090,11 @@ static int bcoo_rows(sp_plan *p, Prob P, const std::vector<uint32_t> &ptr) {
     return b.finish(WK_BCSR_VEC, false, 1);
 }
 
-int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
+// `rows` (in): whether block rows may serve several right-hand sides beside the block-balanced
+// group; out: whether they do.
+static int build_bcoo_group(sp_plan *p, const sp_bcoo *B, bool &rows) {
+    const bool may = rows;
+    rows = false;
     const size_t sv = sp_dtype_size(B->dtype);
     const uint32_t R = B->row_block_size, C = B->col_block_size;
     const size_t rc2 = (size_t)R * C;
@@ -1106,9 +1124,11 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
         const uint32_t maxlen = *std::max_element(ptr.begin(), ptr.end());
         const double avg = (double)nb / P.nrows;
         for (uint32_t I = 0; I < P.nrows; I++) ptr[I + 1] += ptr[I];
-        if (maxlen <= 4 * avg + 64 && coal_ok(B->dtype, R, C, avg)) {
+        const bool alone = sv == 8 || nb <= 1u << 20;
+        if (maxlen <= 4 * avg + 64 && coal_ok(B->dtype, R, C, avg) && (alone || may)) {
+            rows = !alone;
             if ((rc = bcoo_rows(p, P, ptr))) return rc;
-            if (sv == 8 || nb <= 1u << 20) {
+            if (alone) {
                 p->algo = SP_ALGO_VECTOR;
                 p->lanes = 64;
                 p->nparts = 1;
@@ -1165,6 +1185,17 @@ int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
     b.add(P, units, nullptr);
     if ((rc = b.finish(WK_BCOO_SEG, true, R))) return rc;
     return atom ? atomic_prezero(p, B->browind, units, R, B->nrows, b.zrow) : SP_OK;
+}
+
+int build_bcoo_plan(sp_plan *p, const sp_bcoo *B) {
+    const sp_opts opts = p->opts;
+    const int algo = p->algo;
+    bool rows = true;
+    int rc = build_bcoo_group(p, B, rows);
+    if (rc != SP_ERR_NOMEM || !rows) return rc;
+    drop_groups(p, opts, algo);
+    rows = false;
+    return build_bcoo_group(p, B, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -1238,7 +1269,10 @@ TiledKind tiled_kind(int id) {
 
 }  // namespace
 
-int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
+// `tried`: whether wide tiles may be taken; returns whether they were tried.
+static int build_tiles(sp_plan *p, const sp_coo *A0, bool &tried) {
+    const bool may = tried;
+    tried = false;
     const TiledKind tk = tiled_kind(p->id);
     const uint32_t n = A0->nrows;
     const size_t sv = sp_dtype_size(A0->dtype);
@@ -1283,7 +1317,7 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
         // entries per tile at least.)
         // CSR from 1M entries: a fix-up more than the row kernel's two launches (RBDCSR, 15000 x 33
         // uniform FP32 9.3 against 12.0 us, banded 76952 x 33 INT32 18.2 -> 13.8 us).
-        if (A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64 &&
+        if (may && A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64 &&
             (tk.format == SP_FMT_COO || A->nnz >= 1u << 20))
             wide = wide_shape(p, tk.format == SP_FMT_COO, false, A->colind, n, A->nnz);
     }
@@ -1575,7 +1609,8 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
         // An empty tile's rows need the partial buffer zeroed first, as COO tilings do anyway; CSR
         // ones keep the row kernel then (DCSR, banded 76952 x 33 INT32: 21.1 against 25.3 us).
         for (const Prob &Q : b.probs) wide_zero |= Q.nent == 0 && Q.nrows > 0;
-        if (wide.nt && !(wide_zero && tk.format == SP_FMT_CSR)) {
+        tried = wide.nt && !(wide_zero && tk.format == SP_FMT_CSR);
+        if (tried) {
             std::vector<uint32_t> rp;
             for (uint32_t t = 0; t < nt && !rc; t++) {
                 const Prob &Q = b.probs[t];
@@ -1646,9 +1681,24 @@ int build_tiled_plan(sp_plan *p, const sp_coo *A0) {
         if (!rc && !wide_parts.empty()) {
             rc = finish_wide(p, wide_parts, wide);
             p->work.zero_all = wide_zero;
+            // with the partial rows of one right-hand side, so that a plan which has no room for
+            // them beside its wide tiles goes without the tiles
+            const uint64_t part = (uint64_t)vert * n * sv;
+            if (!rc && !(rc = plan_alloc(p, part, &p->d_ypart))) p->ypart_bytes = part;
         }
         p->nsub = p->work.nunits;
     } while (0);
     sp_free_tiled(T);
     return rc;
+}
+
+int build_tiled_plan(sp_plan *p, const sp_coo *A) {
+    const sp_opts opts = p->opts;
+    const int algo = p->algo;
+    bool wide = true;
+    int rc = build_tiles(p, A, wide);
+    if (rc != SP_ERR_NOMEM || !wide) return rc;
+    drop_groups(p, opts, algo);
+    wide = false;
+    return build_tiles(p, A, wide);
 }

@@ -136,11 +136,22 @@ int plan_alloc(sp_plan *p, size_t bytes, void **out) {
     bytes = (bytes + 32 + 255) & ~(size_t)255;
     if (p->opts.mem_cap_bytes && p->device_bytes + bytes > p->opts.mem_cap_bytes) return SP_ERR_NOMEM;
     void *d = nullptr;
-    if (hipMalloc(&d, bytes) != hipSuccess) return SP_ERR_NOMEM;
-    p->allocs.push_back(d);
+    if (hipMalloc(&d, bytes) != hipSuccess) {
+        (void)hipGetLastError();  // reported here; the next launch's check is not to find it
+        return SP_ERR_NOMEM;
+    }
+    p->allocs.push_back({d, bytes});
     p->device_bytes += bytes;
     *out = d;
     return SP_OK;
+}
+
+void plan_release(sp_plan *p, size_t from, size_t to) {
+    for (size_t i = from; i < to; i++) {
+        (void)hipFree(p->allocs[i].dev);
+        p->device_bytes -= p->allocs[i].bytes;
+    }
+    p->allocs.erase(p->allocs.begin() + from, p->allocs.begin() + to);
 }
 
 int plan_upload(sp_plan *p, const void *host, size_t bytes, void **out) {
@@ -152,7 +163,7 @@ int plan_upload(sp_plan *p, const void *host, size_t bytes, void **out) {
 
 static void plan_free(sp_plan *p) {
     if (!p) return;
-    for (void *d : p->allocs) (void)hipFree(d);
+    plan_release(p, 0, p->allocs.size());
     p->cg.release();
     delete p;
 }

@@ -1,0 +1,90 @@
+"""Device memory of plans, on a device that is simulated in host memory
+(fake_device.c): a second layout that has no room is left out, so a matrix that
+fits once gets its plan, and a plan frees what it does not keep."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PLANS = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_limit.argtypes = [ctypes.c_size_t]
+fake.fake_live.restype = ctypes.c_size_t
+import numpy as np
+import sparsep_amd.api as sp
+NONE = 2 ** 64 - 1
+kern, matrix, dt, k = sys.argv[2], sys.argv[3], int(sys.argv[4]), int(sys.argv[5])
+ctx = sp.Context(0)
+if matrix == "rmat":
+    A = sp.gen_rmat(13, 100000, dtype=dt, seed=1)
+elif matrix == "even":
+    A = sp.gen_banded(40000, 32, 20, 40, dtype=dt, seed=2)
+else:
+    A = sp.gen_stencil27(34, 4, True, dt, seed=3)
+x, y = 64, 64  # (kernels do not run)
+
+
+def product(plan):
+    if k == 1:
+        plan.spmv(x, y)
+    else:
+        plan.spmm(k, x, k, y, k)
+
+
+base = fake.fake_live()
+plan = sp.Plan(ctx, kern, A, sp.opts(mem_cap_bytes=1 << 40))  # (a cap: one layout)
+product(plan)
+need = fake.fake_live() - base
+once = plan.info()
+del plan
+plan = sp.Plan(ctx, kern, A)
+product(plan)
+full = fake.fake_live() - base
+assert full == plan.info()["device_bytes"], (full, plan.info())
+both = plan.info()
+del plan
+assert fake.fake_live() == base
+print("need", need, "full", full, "algo", once["algo"], both["algo"], flush=True)
+assert full > need
+for part in range(9):
+    limit = base + need + (full - need) * part // 8
+    fake.fake_limit(limit)
+    plan = sp.Plan(ctx, kern, A)
+    product(plan)
+    i = plan.info()
+    assert fake.fake_live() - base == i["device_bytes"] <= limit - base
+    if part == 0:
+        assert (i["algo"], i["launches"]) == (once["algo"], once["launches"])
+    if part == 8:
+        assert (i["algo"], i["launches"]) == (both["algo"], both["launches"])
+    del plan
+    fake.fake_limit(NONE)
+    assert fake.fake_live() == base
+print("ok")
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if not shutil.which("gcc") or not os.path.exists("/opt/rocm/include/hip/hip_runtime_api.h"):
+        pytest.skip("no C compiler or no HIP headers")
+    so = str(tmp_path_factory.mktemp("fake") / "fake_device.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "fake_device.c"), "-o", so], check=True)
+    return so
+
+
+@pytest.mark.parametrize("kern,matrix,dt,k", [
+    ("CSR-nnz", "rmat", 4, 1), ("CSR-nnz", "rmat", 3, 8), ("CSR-row", "even", 4, 1), ("CSR-row", "even", 2, 4),
+    ("COO-nnz", "rmat", 5, 1), ("COO-nnz", "rmat", 0, 32), ("COO-row", "even", 4, 2),
+    ("RBDCSR", "even", 4, 1), ("BDCOO", "even", 5, 1), ("DCOO", "even", 2, 3),
+    ("BCOO-nnz", "blocks", 4, 1), ("BCOO-block", "blocks", 2, 8)])
+def test_second_layouts_only_where_they_fit(fake, kern, matrix, dt, k):
+    r = subprocess.run([sys.executable, "-c", PLANS, fake, kern, matrix, str(dt), str(k)], cwd=os.path.dirname(HERE),
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
