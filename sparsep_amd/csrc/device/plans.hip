@@ -1609,6 +1609,7 @@ static int build_tiles(sp_plan *p, const sp_coo *A0, bool &tried) {
         // An empty tile's rows need the partial buffer zeroed first, as COO tilings do anyway; CSR
         // ones keep the row kernel then (DCSR, banded 76952 x 33 INT32: 21.1 against 25.3 us).
         for (const Prob &Q : b.probs) wide_zero |= Q.nent == 0 && Q.nrows > 0;
+        const size_t mark = p->allocs.size();
         tried = wide.nt && !(wide_zero && tk.format == SP_FMT_CSR);
         if (tried) {
             std::vector<uint32_t> rp;
@@ -1630,6 +1631,7 @@ static int build_tiles(sp_plan *p, const sp_coo *A0, bool &tried) {
             if (rc == SP_ERR_RANGE) {
                 rc = SP_OK;
                 wide_parts.clear();
+                plan_release(p, mark, p->allocs.size());
             }
             if (rc) break;
         }
