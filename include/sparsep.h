@@ -507,7 +507,8 @@ typedef struct sp_plan_info {
     uint32_t nrows, ncols, nnz;
     uint64_t num_blocks;
     uint64_t algo_bytes;      /* algorithmic HBM bytes of one SpMV        */
-    uint64_t device_bytes;    /* device memory owned by the plan          */
+    uint64_t device_bytes;    /* device memory owned by the plan, with the *
+                               * vectors that it keeps after a solve      */
     uint32_t nparts, nsub, lanes_per_row, items_per_lane, vert, ntiles;
     uint32_t row_block_size, col_block_size;
     uint32_t launches;        /* kernels per SpMV                          */

@@ -96,6 +96,7 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
 
     CgBuf cg;  // kept between solves, used by one at a time
     std::atomic<bool> cg_busy{false};
+    std::atomic<uint64_t> cg_bytes{0};  // device memory of cg
 };
 
 // Allocation helpers (record in plan->allocs, respect mem_cap_bytes); plan_release frees the

@@ -308,7 +308,7 @@ extern "C" int sp_plan_get_info(const sp_plan *p, sp_plan_info *i) {
     i->nnz = p->nnz;
     i->num_blocks = p->nb;
     i->algo_bytes = p->algo_bytes;
-    i->device_bytes = p->device_bytes;
+    i->device_bytes = p->device_bytes + p->cg_bytes.load();
     i->nparts = p->nparts;
     i->nsub = p->nsub;
     i->lanes_per_row = p->lanes;

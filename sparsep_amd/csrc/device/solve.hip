@@ -202,9 +202,11 @@ int cg_t(sp_plan *A, const T *b, T *x, int maxit, double rtol, int *iters, doubl
     };
     if (!buf->dev && (hipMalloc(&buf->dev, bytes) != hipSuccess ||
                       hipHostMalloc(&buf->note, sizeof(CgNote)) != hipSuccess)) {
+        (void)hipGetLastError();  // reported here
         buf->release();
         return done(SP_ERR_NOMEM);
     }
+    if (kept) A->cg_bytes.store(bytes);
     char *d = (char *)buf->dev;
     T *r = (T *)d, *p = (T *)(d + vec), *q = (T *)(d + 2 * vec);
     double *part_pq = (double *)(d + 3 * vec), *part_r = part_pq + RGRID, *part_b = part_r + RGRID;

@@ -55,6 +55,32 @@ assert full == plan.info()["device_bytes"], (full, plan.info())
 both = plan.info()
 del plan
 assert fake.fake_live() == base
+if k == 1 and dt >= 4 and A.nrows == A.ncols:  # a solve's vectors are kept, and counted
+    plan = sp.Plan(ctx, kern, A)
+    product(plan)
+    for _ in range(2):
+        try:
+            plan.cg(x, y, maxit=3)
+        except sp._lib.SparsePError:
+            pass
+        kept = fake.fake_live() - base - full
+        assert kept >= 3 * A.nrows * sp.NP_DTYPE[dt]().itemsize
+        assert fake.fake_live() - base == plan.info()["device_bytes"]
+    del plan
+    assert fake.fake_live() == base
+    plan = sp.Plan(ctx, kern, A)
+    product(plan)
+    fake.fake_limit(fake.fake_live())
+    for _ in range(2):  # no room for them: an error of its own, and the plan still multiplies
+        try:
+            plan.cg(x, y, maxit=3)
+            raise SystemExit("a solve without memory")
+        except sp._lib.SparsePError as e:
+            assert e.rc == -2
+        product(plan)
+    assert plan.info()["device_bytes"] == full
+    del plan
+    fake.fake_limit(NONE)
 print("need", need, "full", full, "algo", once["algo"], both["algo"], flush=True)
 assert matrix == "gaps" or full > need
 for part in range(9):
