@@ -315,8 +315,11 @@ struct sp_mlp {
     int cap = 0;
     float *x = nullptr, *a1 = nullptr, *z1 = nullptr, *a2 = nullptr, *z2 = nullptr, *y = nullptr;
     float *t = nullptr, *msk = nullptr, *d3 = nullptr, *d2 = nullptr, *d1 = nullptr, *part = nullptr, *l = nullptr;
-    // pinned host memory for a batch: x, t and mask in; gradient and loss partial sums out
+    // pinned host memory of the two-kernel path: x, t and mask of a batch in (calls that hand over
+    // a batch: hcap samples); gradient and loss partial sums out (ncap floats)
     float *hx = nullptr, *hg = nullptr;
+    int hcap = 0;
+    size_t ncap = 0;
     // widths that the two-kernel path takes (16-byte weight loads at every row)
     bool two() const {
         return in % 8 == 0 && h1 % 8 == 0 && h2 % 8 == 0 && in <= MAXW && h1 <= MAXW && h2 <= MAXW && out <= MAXW;
@@ -331,17 +334,36 @@ static int mlp_reserve(sp_mlp *m, int B) {
     m->cap = 0;
     for (float **b : bufs)
         if (*b) { (void)hipFree(*b); *b = nullptr; }
-    for (float **b : {&m->hx, &m->hg})
-        if (*b) { (void)hipHostFree(*b); *b = nullptr; }
     const size_t n[] = {(size_t)B * m->in, (size_t)B * m->h1, (size_t)B * m->h1, (size_t)B * m->h2, (size_t)B * m->h2,
                         (size_t)B * m->out, (size_t)B * m->out, (size_t)B * m->out, (size_t)B * m->out,
                         (size_t)B * m->h2, (size_t)B * m->h1, (size_t)B * m->out / 256 + 2, (size_t)B * m->out};
     for (int i = 0; i < 13; i++)
         if (mlp_alloc(bufs[i], n[i])) return SP_ERR_NOMEM;
-    if (m->two() && (hipHostMalloc((void **)&m->hx, (size_t)B * (m->in + 2 * m->out) * 4) != hipSuccess ||
-                     hipHostMalloc((void **)&m->hg, ((size_t)m->np + n[11]) * 4) != hipSuccess))
-        return SP_ERR_NOMEM;
     m->cap = B;
+    return SP_OK;
+}
+
+// Pinned memory is slow to make: only gradients ask for it, and prediction for none.
+static int mlp_pin(float **p, size_t n) {
+    if (*p) (void)hipHostFree(*p);
+    *p = nullptr;
+    if (hipHostMalloc((void **)p, n * sizeof(float)) == hipSuccess) return SP_OK;
+    (void)hipGetLastError();  // reported here
+    return SP_ERR_NOMEM;
+}
+static int mlp_pin_in(sp_mlp *m, int B) {
+    if (B <= m->hcap) return SP_OK;
+    m->hcap = 0;
+    if (int rc = mlp_pin(&m->hx, (size_t)B * (m->in + 2 * m->out))) return rc;
+    m->hcap = B;
+    return SP_OK;
+}
+static int mlp_pin_out(sp_mlp *m, int B) {
+    const size_t n = (size_t)m->np + (size_t)B * m->out / 256 + 2;
+    if (n <= m->ncap) return SP_OK;
+    m->ncap = 0;
+    if (int rc = mlp_pin(&m->hg, n)) return rc;
+    m->ncap = n;
     return SP_OK;
 }
 
@@ -437,6 +459,7 @@ static float mean_loss(const float *part, int nb, int ny) {
 // Loss and gradient of the batch at x, t, msk (device or pinned host memory; msk may be null) in
 // two kernels; waits for them.  The gradient stays in m->g and is copied to `grad` if given.
 static int loss_grad_two(sp_mlp *m, int B, const float *x, const float *t, const float *msk, float *loss, float *grad) {
+    if (int rc = mlp_pin_out(m, B)) return rc;
     hipStream_t s = m->ctx->stream;
     const int ny = B * m->out, nb = (ny + 255) / 256;
     MlpArgs a{B, m->in, m->h1, m->h2, m->out, x, t, msk, m->p, m->pb, {}, x == m->x ? nullptr : m->x, m->a1, m->a2,
@@ -487,6 +510,7 @@ extern "C" int sp_mlp_loss_grad(sp_mlp *m, const float *X, const float *T, const
     if (rc) return rc;
     hipStream_t s = m->ctx->stream;
     if (m->two()) {  // the kernels read the batch from pinned memory (every call ends with a wait)
+        if ((rc = mlp_pin_in(m, B))) return rc;
         float *const hx = m->hx, *const ht = hx + (size_t)B * m->in, *const hm = ht + (size_t)B * m->out;
         memcpy(hx, X, (size_t)B * m->in * 4);
         memcpy(ht, T, (size_t)B * m->out * 4);

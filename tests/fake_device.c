@@ -4,31 +4,34 @@
 #include <stdlib.h>
 #include <string.h>
 
-static size_t limit = (size_t)-1, live;
+static size_t limit = (size_t)-1, live, pinned;
 static hipError_t last;
 
 void fake_limit(size_t bytes) { limit = bytes; }
 size_t fake_live(void) { return live; }
+size_t fake_pinned(void) { return pinned; }
 
-hipError_t hipMalloc(void **p, size_t n) {
-    if (n > limit || live > limit - n) return last = hipErrorOutOfMemory;
+static hipError_t take(void **p, size_t n, size_t *sum, size_t most) {
+    if (n > most || *sum > most - n) return last = hipErrorOutOfMemory;
     size_t *b = calloc(1, n + 64);
     if (!b) return last = hipErrorOutOfMemory;
     *b = n;
-    live += n;
+    *sum += n;
     *p = (char *)b + 64;
     return hipSuccess;
 }
-hipError_t hipFree(void *p) {
+static hipError_t give(void *p, size_t *sum) {
     if (p) {
         size_t *b = (size_t *)((char *)p - 64);
-        live -= *b;
+        *sum -= *b;
         free(b);
     }
     return hipSuccess;
 }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned f) { return (*p = calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) { return take(p, n, &live, limit); }
+hipError_t hipFree(void *p) { return give(p, &live); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned f) { return take(p, n, &pinned, (size_t)-1); }
+hipError_t hipHostFree(void *p) { return give(p, &pinned); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t t) { memcpy(d, s, n); return hipSuccess; }
 hipError_t hipMemset(void *d, int v, size_t n) { memset(d, v, n); return hipSuccess; }

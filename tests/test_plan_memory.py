@@ -113,6 +113,38 @@ def fake(tmp_path_factory):
     return so
 
 
+MLP = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_pinned.restype = ctypes.c_size_t
+import numpy as np
+import sparsep_amd.api as sp
+mlp = sp.Mlp(sp.Context(0), (64, 128, 128, 25))
+X, T = np.zeros((4000, 64), np.float32), np.zeros((4000, 25), np.float32)
+mlp.predict(X)
+assert fake.fake_pinned() == 0, "prediction pins host memory"
+mlp.train(X, T, epochs=1, batch=64)
+out = fake.fake_pinned()
+assert 0 < out <= 4 * (mlp.nparams + 64 * 25 // 256 + 2), "training needs room for a gradient and its loss"
+mlp.loss_grad(X[:64], T[:64])
+both = fake.fake_pinned()
+assert both == out + 64 * (64 + 2 * 25) * 4
+mlp.predict(X)
+mlp.loss_grad(X[:1], T[:1])
+assert fake.fake_pinned() == both
+mlp.loss_grad(X, T)
+del mlp
+assert fake.fake_pinned() == 0
+print("ok")
+"""
+
+
+def test_selector_pins_only_for_gradients(fake):
+    r = subprocess.run([sys.executable, "-c", MLP, fake], cwd=os.path.dirname(HERE), capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
+
+
 @pytest.mark.parametrize("kern,matrix,dt,k", [
     ("CSR-nnz", "rmat", 4, 1), ("CSR-nnz", "rmat", 3, 8), ("CSR-row", "even", 4, 1), ("CSR-row", "even", 2, 4),
     ("COO-nnz", "rmat", 5, 1), ("COO-nnz", "rmat", 0, 32), ("COO-row", "even", 4, 2),
