@@ -645,8 +645,9 @@ template <int N, typename A> __device__ __forceinline__ A open_scan(A v, uint64_
 // Running sums of p, starting anew after each position whose bit is set in `ends`.  FP32 adds in
 // double precision and rounds each sum once, where sums in a row would round N - 1 times.  (Relative
 // error and time of an FP32 product, sums in single -> double precision: R-MAT 2^20 9.9e-8 ->
-// 7.2e-8, 64.1 -> 64.6 us; RBDCSR banded 199999 x 33 8.5e-8 -> 5.3e-8, 20.0 -> 20.2 us.  The merge
-// tiles and row kernels that these plans ran before: 9.0e-8 and 6.5e-8.)
+// 7.2e-8, 64.1 -> 64.6 us; RBDCSR banded 199999 x 33 8.5e-8 -> 5.3e-8, 20.0 -> 20.2 us;
+// panels, R-MAT 2^18 times 8 columns 9.6e-8 -> 6.8e-8, 36.1 -> 36.2 us.  The merge tiles and row
+// kernels that these plans ran before: 9.0e-8, 6.5e-8 and 8.2e-8.)
 template <int N, typename A> __device__ __forceinline__ void run_sums(A (&p)[N], uint32_t ends) {
     using S = std::conditional_t<std::is_same<A, float>::value, double, A>;
     S s = (S)p[0];
@@ -905,8 +906,7 @@ __global__ __launch_bounds__(TPB) void panel_kernel(const Prob *__restrict__ pro
     A p[GE];
 #pragma unroll
     for (int s = 0; s < GE; s++) p[s] = s_buf[PN::slot(g * GE + s) * K + q];
-#pragma unroll
-    for (int s = 1; s < GE; s++) p[s] = (mask >> (s - 1) & 1) ? p[s] : p[s - 1] + p[s];
+    run_sums<GE>(p, mask);
     A v = (mask >> (GE - 1) & 1) ? A(0) : p[GE - 1];
     const uint64_t ends = __ballot(mask != 0), upto = ends & ((2ull << lane) - 1);
     const int from = upto ? (63 - __builtin_clzll(upto)) / K * K + q : 0;  // lane of the last group with an end

@@ -34,3 +34,18 @@ def test_wide_rounding(sp, ctx, kern, n, length, stride):
     y, plan = run(sp, ctx, kern, A, np.ones(A.ncols, np.float32))
     assert plan.info()["algo"] == sp.ALGO_SEGMENTED_SORTED
     assert np.abs(y.astype(np.float64) - want).max() <= 8 * U
+
+
+@pytest.mark.parametrize("k", [2, 8, 32])
+@pytest.mark.parametrize("skewed", [True, False])
+def test_panel_rounding(sp, ctx, k, skewed):
+    """Groups of 16 entries.  Additions that meet the 1: rounding a group's sum (once), five levels
+    over the groups of a wave, three waves before, the row's own group, the workgroups before."""
+    A, want = _rows(sp, 9001, 33, 1)
+    if skewed:  # a row of many entries, each of value 0
+        extra = np.arange(A.ncols, dtype=np.uint32)
+        A = sp.Coo.from_arrays(A.nrows + 1, A.ncols, np.concatenate([A.rowind, np.full(A.ncols, A.nrows, np.uint32)]),
+                               np.concatenate([A.colind, extra]), np.concatenate([A.values, np.zeros(A.ncols, np.float32)]))
+    Y, _ = run(sp, ctx, "CSR-nnz", A, np.ones((A.ncols, k), np.float32), k=k)
+    err = np.abs(Y[:9001].astype(np.float64) - want)
+    assert err.max() <= 11 * U and not Y[9001:].any()
