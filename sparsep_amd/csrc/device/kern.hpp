@@ -642,18 +642,33 @@ template <int N, typename A> __device__ __forceinline__ A open_scan(A v, uint64_
     return v;
 }
 
-// Running sums of p, starting anew after each position whose bit is set in `ends`.  FP32 adds in
-// double precision and rounds each sum once, where sums in a row would round N - 1 times.  (Relative
-// error and time of an FP32 product, sums in single -> double precision: R-MAT 2^20 9.9e-8 ->
-// 7.2e-8, 64.1 -> 64.6 us; RBDCSR banded 199999 x 33 8.5e-8 -> 5.3e-8, 20.0 -> 20.2 us;
-// panels, R-MAT 2^18 times 8 columns 9.6e-8 -> 6.8e-8, 36.1 -> 36.2 us.  The merge tiles and row
-// kernels that these plans ran before: 9.0e-8, 6.5e-8 and 8.2e-8.)
+// Running sums of p, starting anew after each position whose bit is set in `ends`.  N sums in a row
+// would round N - 1 times; here each is rounded about once: FP32 adds in double precision, FP64
+// gives what an addition rounds off to the next one (Kahan's summation; an overflow must not reach
+// it).  Relative error against the kernels that the plans ran before, in single additions and now:
+//   FP32  R-MAT 2^20 9.0e-8, 9.9e-8, 7.2e-8 (64.1 -> 64.6 us); RBDCSR banded 199999 x 33 6.5e-8,
+//         8.5e-8, 5.3e-8 (20.0 -> 20.2 us); R-MAT 2^18 times 8 columns 8.2e-8, 9.6e-8, 6.8e-8
+//         (36.1 -> 36.2 us)
+//   FP64  banded 100001 x 33 1.20e-16, 1.43e-16, 1.17e-16 (13.8 -> 14.0 us), times 8 columns
+//         1.20e-16, 1.42e-16, 1.18e-16 (36.0 -> 38.3 us); R-MAT 2^18 COO 1.55e-16, 1.70e-16,
+//         1.45e-16 (23.4 us both)
+// (log2(N) rounds of additions over doubling reaches left FP64 at 1.32e-16: the row kernels'
+// products are not rounded; two-sums gave 1.10e-16 at 40.5 us for 8 columns.)
 template <int N, typename A> __device__ __forceinline__ void run_sums(A (&p)[N], uint32_t ends) {
     using S = std::conditional_t<std::is_same<A, float>::value, double, A>;
     S s = (S)p[0];
+    [[maybe_unused]] S c = S(0);
 #pragma unroll
     for (int q = 1; q < N; q++) {
-        s = (ends >> (q - 1) & 1) ? (S)p[q] : s + (S)p[q];
+        const bool anew = ends >> (q - 1) & 1;
+        const S v = (S)p[q];
+        if constexpr (std::is_same<A, double>::value) {
+            const S w = v - c, t = s + w, r = (t - s) - w;
+            c = anew || !__builtin_isfinite(r) ? S(0) : r;
+            s = anew ? v : t;
+        } else {
+            s = anew ? v : s + v;
+        }
         p[q] = (A)s;
     }
 }

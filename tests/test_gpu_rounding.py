@@ -49,3 +49,17 @@ def test_panel_rounding(sp, ctx, k, skewed):
     Y, _ = run(sp, ctx, "CSR-nnz", A, np.ones((A.ncols, k), np.float32), k=k)
     err = np.abs(Y[:9001].astype(np.float64) - want)
     assert err.max() <= 11 * U and not Y[9001:].any()
+
+
+@pytest.mark.parametrize("kern,k", [("CSR-nnz", 1), ("COO-row", 1), ("CSR-row", 8), ("CSR-row", 16)])
+def test_fp64_rounding(sp, ctx, kern, k):
+    """Rows of nine entries in threads or groups of eight: additions that meet the 1 are the rounding
+    of its thread's sum, the other thread's and the tile's before."""
+    n, u = 180000, 2.0 ** -53
+    rng = np.random.default_rng(9)
+    col = np.arange(n)[:, None] + np.arange(9)
+    val = np.full((n, 9), u)
+    val[np.arange(n), rng.integers(0, 9, n)] = 1.0
+    A = sp.Coo.from_arrays(n, n + 8, np.repeat(np.arange(n, dtype=np.uint32), 9), col.ravel().astype(np.uint32), val.ravel())
+    Y, _ = run(sp, ctx, kern, A, np.ones((n + 8, k) if k > 1 else n + 8), k=k)
+    assert np.abs((Y - 1.0) - 8 * u).max() <= 3 * u
