@@ -649,9 +649,9 @@ template <int N, typename A> __device__ __forceinline__ A open_scan(A v, uint64_
 //   FP32  R-MAT 2^20 9.0e-8, 9.9e-8, 7.2e-8 (64.1 -> 64.6 us); RBDCSR banded 199999 x 33 6.5e-8,
 //         8.5e-8, 5.3e-8 (20.0 -> 20.2 us); R-MAT 2^18 times 8 columns 8.2e-8, 9.6e-8, 6.8e-8
 //         (36.1 -> 36.2 us)
-//   FP64  banded 100001 x 33 1.20e-16, 1.43e-16, 1.17e-16 (13.8 -> 14.0 us), times 8 columns
+//   FP64  banded 100001 x 33 1.20e-16, 1.43e-16, 1.17e-16 (13.7 -> 14.0 us), times 8 columns
 //         1.20e-16, 1.42e-16, 1.18e-16 (36.0 -> 38.3 us); R-MAT 2^18 COO 1.55e-16, 1.70e-16,
-//         1.45e-16 (23.4 us both)
+//         1.45e-16 (22.9 -> 23.4 us)
 // (log2(N) rounds of additions over doubling reaches left FP64 at 1.32e-16: the row kernels'
 // products are not rounded; two-sums gave 1.10e-16 at 40.5 us for 8 columns.)
 template <int N, typename A> __device__ __forceinline__ void run_sums(A (&p)[N], uint32_t ends) {

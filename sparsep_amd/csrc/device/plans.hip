@@ -1071,6 +1071,18 @@ int build_bcsr_plan(sp_plan *p, const sp_bcsr *B) {
 // ---------------------------------------------------------------------------
 // BCOO (ids 7, 8)
 // ---------------------------------------------------------------------------
+// The widest pass of block rows whose floating-point sums are no less accurate than the
+// block-balanced kernel's; 0: none.  (Relative error against long double, block balanced -> block
+// rows, 27-point stencil 20^3 x 4: FP32 4 x 4 blocks 8 and 16 columns 7.6e-8 -> 7.5e-8, 32 columns
+// 7.5e-8 -> 8.3e-8; FP64 4 x 4 4 columns 1.42e-16 -> 1.40e-16, 8 columns 2.5e-16, 16 columns 3.5e-16;
+// FP64 2 x 2, 2 x 4 and 4 x 2 8 columns 1.44e-16 -> 1.39e-16, 16 columns 1.9e-16; 8 x 8 one column
+// FP32 7.5e-8 -> 8.6e-8, FP64 1.42e-16 -> 1.61e-16.)
+static int bcoo_row_width(int dtype, uint32_t R, uint32_t C) {
+    if (dtype != SP_F32 && dtype != SP_F64) return 32;
+    if (R * C > 16) return 0;
+    return R * C < 16 ? (dtype == SP_F32 ? 32 : 8) : dtype == SP_F32 ? 16 : 4;
+}
+
 // Even block rows of a BCOO matrix in the coalesced BCSR kernels: the same blocks with block-row
 // pointers in place of row indices, 16 block rows per unit, one launch and no carries.
 static int bcoo_rows(sp_plan *p, Prob P, const std::vector<uint32_t> &ptr) {
@@ -1085,6 +1097,7 @@ static int bcoo_rows(sp_plan *p, Prob P, const std::vector<uint32_t> &ptr) {
     p->work.lanes = 0;
     p->work.R = p->opts.row_block_size;
     p->work.C = p->opts.col_block_size;
+    p->work.kmax = bcoo_row_width(p->dtype, p->work.R, p->work.C);
     Builder b(p);
     b.add(P, units, nullptr);
     return b.finish(WK_BCSR_VEC, false, 1);
@@ -1125,7 +1138,7 @@ static int build_bcoo_group(sp_plan *p, const sp_bcoo *B, bool &rows) {
         const double avg = (double)nb / P.nrows;
         for (uint32_t I = 0; I < P.nrows; I++) ptr[I + 1] += ptr[I];
         const bool alone = sv == 8 || nb <= 1u << 20;
-        if (maxlen <= 4 * avg + 64 && coal_ok(B->dtype, R, C, avg) && (alone || may)) {
+        if (maxlen <= 4 * avg + 64 && coal_ok(B->dtype, R, C, avg) && bcoo_row_width(B->dtype, R, C) && (alone || may)) {
             rows = !alone;
             if ((rc = bcoo_rows(p, P, ptr))) return rc;
             if (alone) {

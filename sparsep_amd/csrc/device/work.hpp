@@ -35,6 +35,7 @@ struct Work {
     bool slice = false;     // 2D CSR/COO tiles: one right-hand side gathers from an LDS copy of the tile's x slice
     spd::Run *d_runs = nullptr;  // CSR merge: row runs that cross tiles (fix-up list), nruns of them
     uint32_t nruns = 0;
+    int kmax = 32;               // widest pass (a plan may ask for less than the kernels take)
     uint32_t panel_nent = 0;     // panels of one problem: its entries (units follow from the width)
     spd::Cross *d_cross[6] = {}; // panels: the rows that cross workgroups at widths 1, 2, 4 .. 32
     uint32_t ncross[6] = {};
@@ -57,12 +58,14 @@ struct Work {
 // keep K partial sums per carry slot.
 inline int max_rhs_chunk(const Work &w) {
     const bool wide8 = (w.dtype == SP_I64 || w.dtype == SP_F64) && w.R * w.C <= 16;
+    const bool valu32 = (w.dtype == SP_F32 || w.dtype == SP_F64) && w.R == 4 && w.C == 4;  // matrix-core / vector-ALU kernels
     switch (w.kind) {
     case WK_CSR_VEC: return 32;
     case WK_PANEL: return 32;
-    case WK_BCSR_VEC:
-        if ((w.dtype == SP_F32 || w.dtype == SP_F64) && w.R == 4 && w.C == 4) return 32;  // matrix-core / vector-ALU kernels
-        return wide8 ? 32 : w.R <= 2 ? 32 : w.R <= 4 ? 16 : 8;
+    case WK_BCSR_VEC: {
+        const int most = valu32 || wide8 || w.R <= 2 ? 32 : w.R <= 4 ? 16 : 8;
+        return w.kmax < most ? w.kmax : most;
+    }
     case WK_BCOO_SEG: return 1;
     case WK_BCSR_SEG: return 1;
     case WK_CSR_HOT: return 1;

@@ -63,3 +63,29 @@ def test_fp64_rounding(sp, ctx, kern, k):
     A = sp.Coo.from_arrays(n, n + 8, np.repeat(np.arange(n, dtype=np.uint32), 9), col.ravel().astype(np.uint32), val.ravel())
     Y, _ = run(sp, ctx, kern, A, np.ones((n + 8, k) if k > 1 else n + 8), k=k)
     assert np.abs((Y - 1.0) - 8 * u).max() <= 3 * u
+
+
+@pytest.mark.parametrize("dt", [4, 5])
+@pytest.mark.parametrize("rc,ks", [((4, 4), (1, 8, 16, 32, 43)), ((2, 2), (1, 16)), ((2, 4), (1, 16, 32)),
+                                   ((4, 2), (1, 32)), ((8, 8), (1, 2, 16))])
+def test_bcoo_rounding(sp, ctx, dt, rc, ks):
+    """Default BCOO plans, whatever kernel serves a width, are as accurate as the block-balanced kernel
+    (algo=2): root mean square errors of 23000 sums or more, known to about 0.5%, within 2%."""
+    A = sp.gen_stencil27(18, 4, True, dt, seed=3)
+    rng = np.random.default_rng(4)
+    t = sp.NP_DTYPE[dt]
+    val = rng.uniform(-1, 1, A.nnz).astype(t)
+    row, col = A.rowind.copy(), A.colind.copy()
+    A = sp.Coo.from_arrays(A.nrows, A.ncols, row, col, val)
+    starts = np.flatnonzero(np.r_[True, row[1:] != row[:-1]])
+    o = {"row_block_size": rc[0], "col_block_size": rc[1]}
+    plan, balanced = sp.Plan(ctx, "BCOO-nnz", A, sp.opts(**o)), sp.Plan(ctx, "BCOO-nnz", A, sp.opts(algo=2, **o))
+    for k in ks:
+        X = rng.uniform(-1, 1, (A.ncols, k) if k > 1 else A.ncols).astype(t)
+        Y = [run(sp, ctx, "BCOO-nnz", A, X, k=k, plan=p)[0].reshape(A.nrows, k) for p in (plan, balanced)]
+        X = X.reshape(A.ncols, k)
+        err = np.zeros(2)
+        for q in {0, 1, k // 2, k - 1} & set(range(k)):
+            want = np.add.reduceat(val.astype(np.longdouble) * X[col, q].astype(np.longdouble), starts)
+            err += [float(((y[:, q] - want) ** 2).mean()) for y in Y]
+        assert err[0] <= 1.02 ** 2 * err[1], (k, np.sqrt(err))
