@@ -1126,10 +1126,15 @@ static int build_bcoo_group(sp_plan *p, const sp_bcoo *B, bool &rows) {
     P.ncols_elem = B->ncols;
     // Automatic plans, no knob asked for, with even block rows of a shape the coalesced BCSR
     // kernel takes: several right-hand sides run as block rows (the block-balanced kernel takes
-    // one per pass), and so does one where that is faster (27-point stencil, 4 x 4 blocks, us
-    // block balanced -> block rows: FP64 9^3 11.0 -> 5.3, 37^3 51.0 -> 34.6, 52^3 133 -> 97; FP32
-    // 16^3 10.3 -> 6.9, 24^3 12.5 -> 10.1, 37^3 23.1 -> 23.4, 52^3 53.2 -> 57.8; INT8 24^3
-    // 10.1 -> 7.3): 8-byte values, and others up to a million blocks.
+    // one per pass), and so does one where that is faster (27-point stencil, us block balanced ->
+    // block rows):
+    //   8-byte values in blocks of 8 or 16 at any size: FP64 4 x 4 9^3 11.0 -> 5.3, 37^3 51.0 ->
+    //     34.6, 52^3 133 -> 97; 2 x 4 22^3 18.7 -> 10.5, 36^3 38.5 -> 36.0; 4 x 2 40^3 52.7 -> 45.0
+    //   8-byte 2 x 2 blocks up to 1.7M: 16^3 9.3 -> 5.7, 25^3 (1.69M) 18.7 -> 15.2, but 26^3
+    //     (1.90M) 19.9 -> 21.6, 33^3 32.6 -> 35.9
+    //   4-byte values up to 900K: FP32 4 x 4 16^3 9.0 -> 4.8, 24^3 12.6 -> 9.7, 32^3 (0.88M) 17.1 ->
+    //     13.1, but 33^3 (0.97M) 17.4 -> 18.1, 52^3 53.2 -> 57.8; 2 x 4 25^3 (0.84M) 12.3 -> 9.9,
+    //     but 26^3 (0.95M) 12.7 -> 14.0
     const sp_opts &o = p->opts;
     if (p->algo == SP_ALGO_AUTO && nb && no_knobs(o)) {
         std::vector<uint32_t> ptr((size_t)P.nrows + 1, 0);
@@ -1137,7 +1142,7 @@ static int build_bcoo_group(sp_plan *p, const sp_bcoo *B, bool &rows) {
         const uint32_t maxlen = *std::max_element(ptr.begin(), ptr.end());
         const double avg = (double)nb / P.nrows;
         for (uint32_t I = 0; I < P.nrows; I++) ptr[I + 1] += ptr[I];
-        const bool alone = sv == 8 || nb <= 1u << 20;
+        const bool alone = sv < 8 ? nb <= 900000 : R * C >= 8 || nb <= 1700000;
         if (maxlen <= 4 * avg + 64 && coal_ok(B->dtype, R, C, avg) && bcoo_row_width(B->dtype, R, C) && (alone || may)) {
             rows = !alone;
             if ((rc = bcoo_rows(p, P, ptr))) return rc;

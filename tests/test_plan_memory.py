@@ -113,6 +113,28 @@ def fake(tmp_path_factory):
     return so
 
 
+BCOO_ROUTES = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import sparsep_amd.api as sp
+ctx = sp.Context(0)
+for dt, g, rc, algo in [(sp.F32, 32, (4, 4), sp.ALGO_VECTOR), (sp.F32, 33, (4, 4), sp.ALGO_SEGMENTED),
+                        (sp.I32, 25, (2, 4), sp.ALGO_VECTOR), (sp.I32, 26, (2, 4), sp.ALGO_SEGMENTED),
+                        (sp.F64, 25, (2, 2), sp.ALGO_VECTOR), (sp.F64, 26, (2, 2), sp.ALGO_SEGMENTED),
+                        (sp.F64, 33, (4, 4), sp.ALGO_VECTOR), (sp.F64, 33, (4, 2), sp.ALGO_VECTOR)]:
+    A = sp.gen_stencil27(g, 4, True, dt, seed=3)
+    i = sp.Plan(ctx, "BCOO-nnz", A, sp.opts(row_block_size=rc[0], col_block_size=rc[1])).info()
+    assert i["algo"] == algo, (dt, g, rc, i)
+print("ok")
+"""
+
+
+def test_bcoo_block_rows_where_they_are_faster(fake):
+    r = subprocess.run([sys.executable, "-c", BCOO_ROUTES, fake], cwd=os.path.dirname(HERE), capture_output=True,
+                       text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
+
+
 MLP = r"""
 import ctypes, sys
 fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
