@@ -407,7 +407,8 @@ uint32_t panel_widths(double avg, uint32_t nnz, size_t sv) {
 // Shape: scattered columns (over 0.3 lines per entry in row order; R-MAT 0.84, banded and
 // stencils up to 0.2) want the widest tile once it leaves enough of them (R-MAT 2^20: 74.8 with
 // 4096 entries, 66.4 with 8192, 62.1 with 16384; uniform INT8 9.9M entries: 29.5, 22.9, 23.0;
-// but 2.9M entries INT16: 13.8 with 4096, 16.4 with 16384); local ones 16 entries per thread in
+// but 2.9M entries INT16: 13.8 with 4096, 16.4 with 16384; FP64 3 in every row 2.4M: 30.1 with 2048,
+// 37.0 with 8192, 3.5M 39.9 with 8192, 46.1 in the row kernel); local ones 16 entries per thread in
 // the smallest workgroup (199999 x 33 FP32: 14.2 with 256 threads, 16.4 with 1024), 8-byte sums
 // 8 per thread (20.1 against 24.3).
 WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
@@ -416,7 +417,7 @@ WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *co
     const uint32_t least = coo || skewed ? 2u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
     if (nnz < least || nnz > 0xF0000000u) return {};  // (entry numbers plus a tile stay below 2^32)
     const bool scattered = row_lines(colind, nnz, sp_dtype_size(p->dtype)) > 0.3;
-    if (acc_size(p->dtype) == 8) return scattered && nnz >= 2u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
+    if (acc_size(p->dtype) == 8) return scattered && nnz >= 3u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
     if (scattered && nnz >= 3u << 20) return {1024, 16};
     return !scattered && nnz >= 1u << 20 ? WideShape{256, 16} : WideShape{512, 8};
 }

@@ -135,6 +135,29 @@ def test_bcoo_block_rows_where_they_are_faster(fake):
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
 
 
+TILES = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+import sparsep_amd.api as sp
+ctx = sp.Context(0)
+for dt, nnz, small in [(sp.F64, 2800000, True), (sp.F64, 3200000, False), (sp.F32, 2800000, True), (sp.F32, 3200000, False)]:
+    n = nnz // 20
+    row = np.repeat(np.arange(n, dtype=np.uint32), 20)
+    col = np.sort(np.random.default_rng(1).integers(0, n, (n, 20)), axis=1).ravel().astype(np.uint32)
+    i = sp.Plan(ctx, "COO-nnz", sp.Coo.from_arrays(n, n, row, col, np.ones(row.size, sp.NP_DTYPE[dt]))).info()
+    assert i["algo"] == sp.ALGO_SEGMENTED_SORTED and (i["ntiles"] > 600) == small, (dt, nnz, i)
+print("ok")
+"""
+
+
+def test_wide_tile_sizes(fake):
+    """Scattered columns: small tiles up to 3M entries, for either size of sums."""
+    r = subprocess.run([sys.executable, "-c", TILES, fake], cwd=os.path.dirname(HERE), capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
+
+
 MLP = r"""
 import ctypes, sys
 fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
