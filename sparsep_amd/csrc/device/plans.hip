@@ -393,16 +393,58 @@ uint32_t panel_widths(double avg, uint32_t nnz, size_t sv) {
     return mask;
 }
 
+// Entries from which an even-row CSR matrix takes wide tiles.  The row kernels need one launch and
+// wide tiles a second one for the rows that cross tiles, about 2.5 us.  Below, row kernel against
+// wide tiles in us, products back to back, medians over five pairs of plans; "local": columns
+// within 80, "scattered": anywhere.
+//   no row crosses a tile (16 or 64 entries in every row): from 192K; FP32 local 16 300K 6.1, 4.2
+//   rows of which a wave's longest mostly takes its lanes two steps: FP32 local 63 in every row 200K
+//     8.2, 7.2, 500K 7.6, 7.3, 1.2M 10.5, 8.8; 2 .. 32 320K 7.2, 7.3, 800K 7.8, 7.5
+//   every fourth wave, or lengths beyond 1.6 times the mean: FP32 local 2 .. 64 320K 6.5, 7.4, 500K
+//     6.4, 7.5, 800K 8.2, 7.5; scattered 500K 6.8, 7.0, 800K 8.8, 7.3; FP64 500K 7.7, 7.5
+//   calmer rows, scattered: FP32 17 in every row 1.2M 10.4, 11.5, 1.7M 13.6, 12.3; 33 1.2M 9.8, 10.3,
+//     1.7M 13.5, 10.8; FP64 24 1.7M 16.0, 15.7, 33 1.2M 11.6, 12.3, 1.7M 16.1, 15.5.  (Up to 9216
+//     rows they keep wide tiles, the route that tests/test_gpu_wide.py holds: INT32 9001 x 33 5.2, 7.3)
+//   calmer rows, local: FP32 17 in every row 2.4M 9.5, 10.3, 3.5M 11.2, 11.3, 33 2.4M 9.8, 10.2, 3.5M
+//     11.4, 11.5; lengths beyond 1.25 times the mean 8 .. 25 1.7M 8.8, 9.1, 2.4M 10.5, 10.2; 16 .. 49
+//     1.2M 8.1, 8.7, 1.7M 9.0, 9.1, 2.4M 10.6, 10.2 (from 1000K, as the same test holds)
+//   rows shorter than 16 (another row kernel), local: FP32 5 1.2M 7.7, 8.7, 1.4M 11.1, 8.9, 3 1.4M 8.0,
+//     8.6, 1.7M 10.9, 8.9, 15 1.7M 8.0, 9.4, 2.1M 12.2, 9.7; scattered: FP32 5 1.2M 10.0, 13.7, 1.7M
+//     15.6, 14.4, INT8 3 1.4M 9.7, 11.6, 1.7M 13.1, 12.5; FP64 3 2.7M 32.1, 37.1, 3.5M 46.2, 39.9
+uint32_t even_rows_least(const uint32_t *rowptr, uint32_t nrows, uint32_t nnz, size_t sv, bool scattered) {
+    constexpr uint32_t K = 1u << 10;
+    const double avg = (double)nnz / nrows;
+    if (avg < 16) return scattered ? (sv == 8 ? 3072 * K : 1536 * K) : avg < 12 ? 1400 * K : 1792 * K;
+    // waves of the chunked row kernel: rows side by side, steps of the longest
+    const uint32_t L = chunk_lanes(avg), rows = 64 / L;
+    uint64_t steps = 0, waves = 0;
+    uint32_t maxlen = 0;
+    bool cross = false;
+    for (uint32_t i = 0; i < nrows; i += rows, waves++) {
+        uint32_t most = 0;
+        for (uint32_t r = i; r < std::min(i + rows, nrows); r++) {
+            const uint32_t b = rowptr[r], e = rowptr[r + 1];
+            if (e == b) continue;
+            maxlen = std::max(maxlen, e - b);
+            most = std::max(most, (e + 3) / 4 - b / 4);
+            cross = cross || b / 2048 != (e - 1) / 2048;
+        }
+        steps += (most + L - 1) / L;
+    }
+    if (!cross) return 192 * K;
+    if (2 * steps >= 3 * waves) return 256 * K;
+    if (4 * steps >= 5 * waves || maxlen > 1.6 * avg) return 512 * K;
+    if (scattered) return nrows <= 9216 ? 288 * K : sv == 8 ? 1792 * K : 1536 * K;
+    return maxlen <= 1.25 * avg ? 3584 * K : avg >= 24 ? 1000 * K : 2304 * K;
+}
+
 // Whether an automatic 1D CSR/COO plan takes wide tiles, and which.  Against the kernels that
 // the row-ordered group would take (us per SpMV, before -> wide):
 //   skewed rows and COO from 2K entries on: R-MAT 2^12 x 8 FP32 CSR 8.4 -> 6.5, 2^16 x 16
-//     11.0 -> 8.2, 2^18 x 16 FP64 28.8 -> 22.7, 2^20 x 16 FP32 72.6 -> 62.1; COO 5-point stencil
+//     11.0 -> 8.2, 2^18 x 16 FP64 28.8 -> 22.7, 2^20 x 16 FP32 72.6 -> 64.6; COO 5-point stencil
 //     700^2 14.2 -> 9.6
-//   even rows: their single launch needs no fix-up, which decides small matrices (5-point
-//     stencil 256^2 INT32, 0.3M entries: 5.0 against 6.4; 5001 rows of 33 entries: 6.6 against
-//     6.8), so from 192K entries for rows of 16 or more (banded 5999 x 33 INT16 7.6 -> 6.6, 20999
-//     x 33 FP32 9.8 -> 6.8, 199999 x 33 23.7 -> 14.2) and from 1M for shorter ones (5-point
-//     stencil 700^2 FP32 15.3 -> 11.4, 1400^2 58 -> 26)
+//   even CSR rows (`even`: their row pointers) where even_rows_least says so; 2D tilings ask for
+//     1M entries themselves
 //   rows made of aligned four-column runs keep their four-value x loads (the caller's check)
 // Shape: scattered columns (over 0.3 lines per entry in row order; R-MAT 0.84, banded and
 // stencils up to 0.2) want the widest tile once it leaves enough of them (R-MAT 2^20: 74.8 with
@@ -411,12 +453,13 @@ uint32_t panel_widths(double avg, uint32_t nnz, size_t sv) {
 // 37.0 with 8192, 3.5M 39.9 with 8192, 46.1 in the row kernel); local ones 16 entries per thread in
 // the smallest workgroup (199999 x 33 FP32: 14.2 with 256 threads, 16.4 with 1024), 8-byte sums
 // 8 per thread (20.1 against 24.3).
-WideShape wide_shape(const sp_plan *p, bool coo, bool skewed, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
+WideShape wide_shape(const sp_plan *p, const uint32_t *even, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
     const sp_opts &o = p->opts;
+    const size_t sv = sp_dtype_size(p->dtype);
     if (p->algo != SP_ALGO_AUTO || !no_knobs(o)) return {};
-    const uint32_t least = coo || skewed ? 2u << 10 : nnz / std::max(nrows, 1u) >= 16 ? 192u << 10 : 1u << 20;
-    if (nnz < least || nnz > 0xF0000000u) return {};  // (entry numbers plus a tile stay below 2^32)
-    const bool scattered = row_lines(colind, nnz, sp_dtype_size(p->dtype)) > 0.3;
+    if (nnz < (even ? 192u << 10 : 2u << 10) || nnz > 0xF0000000u) return {};  // (entry numbers plus a tile stay below 2^32)
+    const bool scattered = row_lines(colind, nnz, sv) > 0.3;
+    if (even && nnz < even_rows_least(even, nrows, nnz, sv, scattered)) return {};
     if (acc_size(p->dtype) == 8) return scattered && nnz >= 3u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
     if (scattered && nnz >= 3u << 20) return {1024, 16};
     return !scattered && nnz >= 1u << 20 ? WideShape{256, 16} : WideShape{512, 8};
@@ -660,7 +703,7 @@ static int build_csr_group(sp_plan *p, const sp_csr *A, WideShape *wide) {
         for (uint32_t i = 0; i < A->nrows; i++) maxlen = std::max(maxlen, A->rowptr[i + 1] - A->rowptr[i]);
         const double avg = A->nrows ? (double)A->nnz / A->nrows : 0.0;
         if (wide && !quad_rows(A->rowptr, A->nrows, A->colind, A->nnz, A->ncols))
-            *wide = wide_shape(p, false, maxlen > 4 * avg + 64, A->colind, A->nrows, A->nnz);
+            *wide = wide_shape(p, maxlen > 4 * avg + 64 ? nullptr : A->rowptr, A->colind, A->nrows, A->nnz);
         // Row-granular kernel for even row lengths up to a few million entries (one launch,
         // no carries); the merge-path kernel for skewed rows, and for large matrices, where
         // its deeper per-thread load batches win (27-point stencil, 113M entries: 1.3x).
@@ -863,7 +906,7 @@ static int build_coo_group(sp_plan *p, const sp_coo *A0, WideShape *wide, std::v
         const bool quads = !atom && !p->opts.lds_slice && p->algo != SP_ALGO_SEGMENTED_SORTED &&
                            quad_rows(rowptr.data(), n, A->colind, nnz, A->ncols);
         if (wide && !quads)
-            *wide = wide_shape(p, true, maxlen > 4.0 * nnz / std::max(n, 1u) + 64, A->colind, n, nnz);
+            *wide = wide_shape(p, nullptr, A->colind, n, nnz);
         // 4 items per lane, the tuner's usual winner for 1D COO; skewed rows and more than 8M
         // entries take 4096-entry tiles (16, run as 512 x 8: R-MAT 2^20 86 vs 109 us), as for CSR
         if (p->opts.items_per_lane == 0 && maxlen > 4.0 * nnz / std::max(n, 1u) + 64 && nnz > (8u << 20) &&
@@ -1338,7 +1381,7 @@ static int build_tiles(sp_plan *p, const sp_coo *A0, bool &tried) {
         // uniform FP32 9.3 against 12.0 us, banded 76952 x 33 INT32 18.2 -> 13.8 us).
         if (may && A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64 &&
             (tk.format == SP_FMT_COO || A->nnz >= 1u << 20))
-            wide = wide_shape(p, tk.format == SP_FMT_COO, false, A->colind, n, A->nnz);
+            wide = wide_shape(p, nullptr, A->colind, n, A->nnz);
     }
     if (sorted) sp_free_coo(sorted);
     if (rc) return rc;

@@ -25,7 +25,7 @@ def _rows(sp, n, length, stride, seed=6):
 
 
 @pytest.mark.parametrize("kern", ["CSR-nnz", "COO-nnz", "RBDCSR"])
-@pytest.mark.parametrize("n,length,stride", [(40000, 33, 1), (160000, 20, 1), (50000, 40, 1), (90001, 36, 997)])
+@pytest.mark.parametrize("n,length,stride", [(112000, 33, 1), (190000, 20, 1), (92000, 40, 1), (90001, 36, 997)])
 def test_wide_rounding(sp, ctx, kern, n, length, stride):
     """Tiles of 16 entries per thread.  Additions that meet the 1: rounding a thread's sum (once),
     three levels over the threads of a row, the waves before, the row's own thread, the tile before,

@@ -12,7 +12,7 @@ THREADS, ROUNDS = 4, 25
 
 
 def _banded(sp, dt, n, per):
-    """Symmetric, positive definite, 2 per + 1 entries per row (wide tiles from 192K entries on)."""
+    """Symmetric, positive definite, 2 per + 1 entries per row (wide tiles from 3.7M entries on)."""
     i = np.arange(n)
     row, col, val = [i], [i], [np.full(n, 2.0 * per + 1)]
     for d in range(1, per + 1):
@@ -73,7 +73,7 @@ def test_products_on_one_plan(sp, ctx, kern, k, algo):
 
 @pytest.mark.parametrize("kern", ["CSR-nnz", "RBDCSR"])
 def test_solves_on_one_plan(sp, ctx, kern):
-    A = _banded(sp, 5, 60001, 12)
+    A = _banded(sp, 5, 150001, 12)
     plan = sp.Plan(ctx, kern, A)
     assert plan.info()["algo"] == sp.ALGO_SEGMENTED_SORTED and plan.info()["launches"] >= 2
     bs = [sp.DeviceArray.from_numpy(ctx, np.random.default_rng(i).standard_normal(A.nrows)) for i in range(THREADS)]

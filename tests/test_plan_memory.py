@@ -158,6 +158,52 @@ def test_wide_tile_sizes(fake):
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
 
 
+CSR_ROUTES = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+import sparsep_amd.api as sp
+ctx = sp.Context(0)
+
+
+def matrix(lens, local, dt):
+    rng = np.random.default_rng(1)
+    n = len(lens)
+    m = n + 80 if local else n
+    row = np.repeat(np.arange(n), lens)
+    key = np.sort(row * m + (row + rng.integers(0, 80, row.size) if local else rng.integers(0, m, row.size)))
+    return sp.Coo.from_arrays(n, m, (key // m).astype(np.uint32), (key % m).astype(np.uint32),
+                              np.ones(key.size, sp.NP_DTYPE[dt]))
+
+
+def spread(lo, hi, n):
+    return np.random.default_rng(2).integers(lo, hi + 1, n)
+
+
+ROWS, WIDE = sp.ALGO_VECTOR, sp.ALGO_SEGMENTED_SORTED
+for lens, local, dt, algo in [
+        (np.full(100000, 17), True, sp.F32, ROWS), (np.full(290000, 17), True, sp.F32, WIDE),
+        (np.full(60000, 27), True, sp.F64, ROWS), (np.full(20000, 16), True, sp.F32, WIDE),
+        (np.full(30000, 33), False, sp.F32, ROWS), (np.full(60000, 33), False, sp.F32, WIDE),
+        (np.full(100000, 17), False, sp.F64, ROWS), (np.full(120000, 17), False, sp.F64, WIDE),
+        (np.full(4000, 63), True, sp.I8, ROWS), (np.full(5000, 63), True, sp.I8, WIDE),
+        (spread(2, 64, 10000), True, sp.F32, ROWS), (spread(2, 64, 20000), True, sp.F32, WIDE),
+        (np.full(250000, 5), True, sp.F32, ROWS), (np.full(300000, 5), True, sp.F32, WIDE),
+        (np.full(110000, 15), True, sp.F32, ROWS), (np.full(130000, 15), True, sp.F32, WIDE),
+        (np.full(160000, 8), False, sp.F32, ROWS), (np.full(220000, 8), False, sp.F32, WIDE),
+        (np.full(300000, 8), False, sp.F64, ROWS)]:
+    i = sp.Plan(ctx, "CSR-nnz", matrix(lens, local, dt)).info()
+    assert i["algo"] == algo, (lens[:4], len(lens), local, dt, i)
+print("ok")
+"""
+
+
+def test_even_rows_take_wide_tiles_where_they_are_faster(fake):
+    r = subprocess.run([sys.executable, "-c", CSR_ROUTES, fake], cwd=os.path.dirname(HERE), capture_output=True,
+                       text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
+
+
 MLP = r"""
 import ctypes, sys
 fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
