@@ -1377,10 +1377,14 @@ static int build_tiles(sp_plan *p, const sp_coo *A0, bool &tried) {
         // Even rows take wide tiles as in 1D; skewed ones keep the kernels whose sums have the same
         // bits as those over LDS slices of x.  (A plan's tiles are sorted one launch each: 16K
         // entries per tile at least.)
-        // CSR from 1M entries: a fix-up more than the row kernel's two launches (RBDCSR, 15000 x 33
-        // uniform FP32 9.3 against 12.0 us, banded 76952 x 33 INT32 18.2 -> 13.8 us).
-        if (may && A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4.0 * A->nnz / std::max(n, 1u) + 64 &&
-            (tk.format == SP_FMT_COO || A->nnz >= 1u << 20))
+        // CSR: a fix-up more than the row kernel's two launches, from 1M entries (RBDCSR, 15000 x 33
+        // uniform FP32 9.3 against 12.0 us, banded 76952 x 33 INT32 18.2 -> 13.8 us); short local
+        // rows of one length from 2.5M (FP32 5 in every row 1.06M 12.2 -> 13.4, 1.5M 12.6 -> 13.7,
+        // 2.5M 15.6 -> 15.6, 4M 21.5 -> 19.8; scattered 1.5M 17.8 -> 15.8).
+        const double avg = (double)A->nnz / std::max(n, 1u);
+        const bool brief = avg < 16 && maxlen <= 1.25 * avg && row_lines(A->colind, A->nnz, sv) <= 0.3;
+        if (may && A->nnz / std::max(T->ntiles, 1u) >= 16u << 10 && maxlen <= 4 * avg + 64 &&
+            (tk.format == SP_FMT_COO || A->nnz >= (brief ? 2500u : 1024u) << 10))
             wide = wide_shape(p, nullptr, A->colind, n, A->nnz);
     }
     if (sorted) sp_free_coo(sorted);

@@ -194,6 +194,10 @@ for lens, local, dt, algo in [
         (np.full(300000, 8), False, sp.F64, ROWS)]:
     i = sp.Plan(ctx, "CSR-nnz", matrix(lens, local, dt)).info()
     assert i["algo"] == algo, (lens[:4], len(lens), local, dt, i)
+for lens, local, algo in [(np.full(300000, 5), True, ROWS), (np.full(530000, 5), True, WIDE),
+                          (np.full(300000, 5), False, WIDE), (np.full(70000, 17), True, WIDE)]:
+    i = sp.Plan(ctx, "RBDCSR", matrix(lens, local, sp.F32)).info()
+    assert i["algo"] == algo, ("RBDCSR", lens[:4], len(lens), local, i)
 print("ok")
 """
 
