@@ -375,19 +375,65 @@ bool no_knobs(const sp_opts &o) {
     return !o.items_per_lane && !o.lanes_per_row && !o.nparts && !o.nsub && !o.lds_slice && !o.mem_cap_bytes;
 }
 
+// What the row kernels make of even CSR rows.
+struct EvenRows {
+    double avg;
+    uint32_t maxlen = 0;
+    bool cross = false;  // some row crosses a multiple of 2048 entries, where wide tiles end
+    // steps that a wave of the chunked row kernel takes (rows side by side, those of its longest)
+    uint64_t steps = 0, waves = 0;
+    bool two_steps(double share) const { return steps >= (1 + share) * waves; }
+    // lengths differ little, or mostly within one step
+    bool calm() const { return avg < 16 ? maxlen <= 1.25 * avg : !two_steps(0.25) && maxlen <= 1.6 * avg; }
+    EvenRows(const uint32_t *rowptr, uint32_t nrows) : avg((double)rowptr[nrows] / nrows) {
+        const uint32_t L = chunk_lanes(avg), rows = 64 / L;
+        for (uint32_t i = 0; i < nrows; i += rows, waves++) {
+            uint32_t most = 0;
+            for (uint32_t r = i; r < std::min(i + rows, nrows); r++) {
+                const uint32_t b = rowptr[r], e = rowptr[r + 1];
+                if (e == b) continue;
+                maxlen = std::max(maxlen, e - b);
+                most = std::max(most, (e + 3) / 4 - b / 4);
+                cross = cross || b / 2048 != (e - 1) / 2048;
+            }
+            steps += (most + L - 1) / L;
+        }
+    }
+};
+
 // Widths (bit i: 2^i right-hand sides) at which even CSR rows run as panels and not in the row
-// kernels (us, rows -> panel): rows of 16 to 64 entries with 4- and 8-byte values while a row of x
-// is at most 64 bytes (250000 x 33 banded INT32: 2 columns 38.2 -> 21.2, 8 columns 49.4 -> 46.7;
-// 200000 x 33 uniform: 8 columns 80 -> 61.5; 60000 x 33 banded INT64 8 columns 36.4 -> 25.0),
-// wider ones only for small matrices (32 columns: 10000 x 33 25.6 -> 11.2, 250000 x 33 99 -> 144);
-// shorter rows where the row kernel spreads a wave over the columns of one row (x rows of 64
-// bytes and more; 5-point stencil 500^2: 16 columns 75.4 -> 22.7, INT64 8 columns 113 -> 22.1, but
-// 8 columns INT32 12.5 -> 15.5); longer rows never (27-point stencil: 18.4 -> 30.8).
-uint32_t panel_widths(double avg, uint32_t nnz, size_t sv) {
+// kernels.  Panels take two launches, the row kernels one.  (us, row kernel, panels; medians over
+// pairs of plans; "local": columns within 80, "scattered": anywhere.)
+//   rows of 16 to 64 entries with 4- and 8-byte values, x rows of 64 bytes: FP32 16 columns local
+//     17 in every row 100K 27.0, 8.2, 4M 68.9, 42.6; calm local rows above 40 up to 2.5M (63 in
+//     every row 2M 24.1, 23.0, 4M 31.2, 40.3)
+//   wider ones for small matrices: 32 columns FP32 17 600K 31.5, 17.3; 250000 x 33 99, 144
+//   narrower ones: lengths that differ from 96K (FP32 2 .. 64 local 4 columns 100K 8.1, 8.4, 600K
+//     10.6, 8.5; 8 columns 100K 9.3, 8.4), 8 bytes from 512K (300K 8.0, 8.7, 600K 9.8, 8.8); calm
+//     rows from 2M (FP32 17 in every row 2 columns 300K 5.9, 8.4, 1M 8.3, 8.7, FP64 2M 12.8, 11.5),
+//     32 bytes if scattered (FP32 8 columns 2M 24.6, 21.0, local 12.8, 15.9)
+//   shorter rows where the row kernel spreads a wave over the columns of one row (x rows of 64
+//     bytes and more; 5-point stencil 500^2: 16 columns 75.4, 22.7, INT64 8 columns 113, 22.1, but 8
+//     columns INT32 12.5, 15.5), not 256 bytes with calm local rows above 8 (FP64 12 in every row 3M
+//     90.2, 103.7)
+//   longer rows never (27-point stencil: 18.4, 30.8)
+uint32_t panel_widths(const EvenRows &rows, uint32_t nnz, size_t sv, bool scattered) {
+    const double avg = rows.avg;
+    const bool calm = rows.calm() || rows.maxlen <= 1.25 * avg;
     uint32_t mask = 0;
     for (uint32_t i = 1; i <= 5; i++) {
         const size_t bytes = sv << i;
-        const bool use = avg < 16 ? bytes >= 64 : avg <= 64 && sv >= 4 && (bytes <= 64 || nnz <= 1u << 20);
+        bool use;
+        if (avg < 16)
+            use = bytes >= 64 && !(bytes >= 256 && calm && !scattered && avg > 8);
+        else if (avg > 64 || sv < 4)
+            use = false;
+        else if (bytes >= 64)
+            use = nnz <= (bytes > 64 ? 1u << 20 : calm && !scattered && avg > 40 ? 2560u << 10 : ~0u);
+        else if (calm)
+            use = nnz >= 2u << 20 && (bytes < 32 || scattered);
+        else
+            use = nnz >= (bytes > 8 ? 96u << 10 : 512u << 10);
         mask |= (uint32_t)use << i;
     }
     return mask;
@@ -411,31 +457,15 @@ uint32_t panel_widths(double avg, uint32_t nnz, size_t sv) {
 //   rows shorter than 16 (another row kernel), local: FP32 5 1.2M 7.7, 8.7, 1.4M 11.1, 8.9, 3 1.4M 8.0,
 //     8.6, 1.7M 10.9, 8.9, 15 1.7M 8.0, 9.4, 2.1M 12.2, 9.7; scattered: FP32 5 1.2M 10.0, 13.7, 1.7M
 //     15.6, 14.4, INT8 3 1.4M 9.7, 11.6, 1.7M 13.1, 12.5; FP64 3 2.7M 32.1, 37.1, 3.5M 46.2, 39.9
-uint32_t even_rows_least(const uint32_t *rowptr, uint32_t nrows, uint32_t nnz, size_t sv, bool scattered) {
+uint32_t even_rows_least(const EvenRows &rows, uint32_t nrows, size_t sv, bool scattered) {
     constexpr uint32_t K = 1u << 10;
-    const double avg = (double)nnz / nrows;
+    const double avg = rows.avg;
     if (avg < 16) return scattered ? (sv == 8 ? 3072 * K : 1536 * K) : avg < 12 ? 1400 * K : 1792 * K;
-    // waves of the chunked row kernel: rows side by side, steps of the longest
-    const uint32_t L = chunk_lanes(avg), rows = 64 / L;
-    uint64_t steps = 0, waves = 0;
-    uint32_t maxlen = 0;
-    bool cross = false;
-    for (uint32_t i = 0; i < nrows; i += rows, waves++) {
-        uint32_t most = 0;
-        for (uint32_t r = i; r < std::min(i + rows, nrows); r++) {
-            const uint32_t b = rowptr[r], e = rowptr[r + 1];
-            if (e == b) continue;
-            maxlen = std::max(maxlen, e - b);
-            most = std::max(most, (e + 3) / 4 - b / 4);
-            cross = cross || b / 2048 != (e - 1) / 2048;
-        }
-        steps += (most + L - 1) / L;
-    }
-    if (!cross) return 192 * K;
-    if (2 * steps >= 3 * waves) return 256 * K;
-    if (4 * steps >= 5 * waves || maxlen > 1.6 * avg) return 512 * K;
+    if (!rows.cross) return 192 * K;
+    if (rows.two_steps(0.5)) return 256 * K;
+    if (!rows.calm()) return 512 * K;
     if (scattered) return nrows <= 9216 ? 288 * K : sv == 8 ? 1792 * K : 1536 * K;
-    return maxlen <= 1.25 * avg ? 3584 * K : avg >= 24 ? 1000 * K : 2304 * K;
+    return rows.maxlen <= 1.25 * avg ? 3584 * K : avg >= 24 ? 1000 * K : 2304 * K;
 }
 
 // Whether an automatic 1D CSR/COO plan takes wide tiles, and which.  Against the kernels that
@@ -459,7 +489,7 @@ WideShape wide_shape(const sp_plan *p, const uint32_t *even, const uint32_t *col
     if (p->algo != SP_ALGO_AUTO || !no_knobs(o)) return {};
     if (nnz < (even ? 192u << 10 : 2u << 10) || nnz > 0xF0000000u) return {};  // (entry numbers plus a tile stay below 2^32)
     const bool scattered = row_lines(colind, nnz, sv) > 0.3;
-    if (even && nnz < even_rows_least(even, nrows, nnz, sv, scattered)) return {};
+    if (even && nnz < even_rows_least(EvenRows(even, nrows), nrows, sv, scattered)) return {};
     if (acc_size(p->dtype) == 8) return scattered && nnz >= 3u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
     if (scattered && nnz >= 3u << 20) return {1024, 16};
     return !scattered && nnz >= 1u << 20 ? WideShape{256, 16} : WideShape{512, 8};
@@ -855,7 +885,8 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     if (rc || algo != SP_ALGO_AUTO || !no_knobs(opts) || rows.work.kind != WK_CSR_VEC || A->nnz < 16u << 10 ||
         A->nnz > 0xF0000000u)
         return rc;
-    p->panel_widths = panel_widths((double)A->nnz / A->nrows, A->nnz, sp_dtype_size(A->dtype));
+    const size_t sv = sp_dtype_size(A->dtype);
+    p->panel_widths = panel_widths(EvenRows(A->rowptr, A->nrows), A->nnz, sv, row_lines(A->colind, A->nnz, sv) > 0.3);
     if (!p->panel_widths) return SP_OK;
     p->panel = std::make_unique<PlanWork>(rows);
     if ((rc = build_panel(p, *p->panel, A->rowptr))) {

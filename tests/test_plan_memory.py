@@ -180,6 +180,20 @@ def spread(lo, hi, n):
     return np.random.default_rng(2).integers(lo, hi + 1, n)
 
 
+fake.fake_launches.restype = ctypes.c_size_t
+for lens, local, dt, k, launches in [  # the row kernels take one launch, panels two
+        (np.full(18000, 17), True, sp.F32, 2, 1), (np.full(18000, 17), False, sp.F64, 4, 1),
+        (np.full(130000, 17), True, sp.F64, 2, 2), (np.full(18000, 17), True, sp.F32, 16, 2),
+        (np.full(130000, 17), True, sp.F32, 8, 1), (np.full(130000, 17), False, sp.F32, 8, 2),
+        (spread(2, 64, 2500), True, sp.F32, 4, 1), (spread(2, 64, 3500), True, sp.F32, 4, 2),
+        (spread(2, 64, 14000), True, sp.F32, 2, 1), (spread(2, 64, 18000), True, sp.F32, 2, 2),
+        (np.full(35000, 63), True, sp.F32, 16, 2), (np.full(45000, 63), True, sp.F32, 16, 1),
+        (np.full(100000, 12), True, sp.F64, 32, 1), (np.full(100000, 12), True, sp.F64, 16, 2),
+        (np.full(40000, 33), True, sp.F32, 32, 1), (np.full(30000, 33), True, sp.F32, 32, 2)]:
+    plan = sp.Plan(ctx, "CSR-row", matrix(lens, local, dt))
+    n = fake.fake_launches()
+    plan.spmm(k, 64, k, 64, k)
+    assert fake.fake_launches() - n == launches, (lens[:4], len(lens), local, dt, k, fake.fake_launches() - n)
 ROWS, WIDE = sp.ALGO_VECTOR, sp.ALGO_SEGMENTED_SORTED
 for lens, local, dt, algo in [
         (np.full(100000, 17), True, sp.F32, ROWS), (np.full(290000, 17), True, sp.F32, WIDE),
