@@ -417,10 +417,14 @@ typedef enum sp_algo {
      * and COO ids (0-4); needs ncols <= 2^32 / (256 * items_per_lane).
      * AUTO takes it in place of SEGMENTED wherever the columns fit (COO:
      * any algo but SEGMENTED does).  AUTO with no other knob and no memory
-     * cap (CSR and COO ids, from a few thousand entries on) takes wide tiles
-     * for one right-hand side, of 2048 to 16384 entries whatever the column
-     * count: sums in a fixed order of their own, and a second copy of the
-     * matrix in row order for several right-hand sides. */
+     * cap (CSR and COO ids: COO and uneven rows from a few thousand entries
+     * on, even CSR rows and 2D tilings from where they are faster) takes wide
+     * tiles for one right-hand side, of 2048 to 16384 entries whatever the
+     * column count: sums in a fixed order of their own, and a second copy of
+     * the matrix in row order for several right-hand sides, which is left out
+     * with the tiles where device memory has no room for it.  sp_plan_info
+     * reports SEGMENTED_SORTED for them; asked for by name it is the
+     * merge-path tiles. */
     SP_ALGO_SEGMENTED_SORTED = 3,
     /* SEGMENTED_SORTED with the most frequent columns' x entries staged in
      * LDS (up to 112 KB; 96 KB for 8-byte accumulators): one 1024-thread
@@ -509,7 +513,11 @@ typedef struct sp_plan_info {
     uint64_t algo_bytes;      /* algorithmic HBM bytes of one SpMV        */
     uint64_t device_bytes;    /* device memory owned by the plan, with the *
                                * vectors that it keeps after a solve      */
-    uint32_t nparts, nsub, lanes_per_row, items_per_lane, vert, ntiles;
+    uint32_t nparts, nsub;
+    /* as in sp_opts.  Wide tiles (algo SP_ALGO_SEGMENTED_SORTED with lanes_per_row
+     * not 0; default options only): threads per tile and entries per thread. */
+    uint32_t lanes_per_row, items_per_lane;
+    uint32_t vert, ntiles;
     uint32_t row_block_size, col_block_size;
     uint32_t launches;        /* kernels per SpMV                          */
 } sp_plan_info;

@@ -674,8 +674,8 @@ int finish_wide(sp_plan *p, const std::vector<WidePart> &parts, WideShape s) {
     p->work.lanes = s.nt;
     p->work.ipt = s.ipt;
     p->algo = SP_ALGO_SEGMENTED_SORTED;
-    p->lanes = 0;
-    p->ipt = s.nt * s.ipt / TPB;
+    p->lanes = s.nt;  // (column-ordered merge tiles report 0)
+    p->ipt = s.ipt;
     p->nsub = s.nt;
     return b.finish(WK_WIDE, true, 1);
 }

@@ -147,6 +147,15 @@ for dt, nnz, small in [(sp.F64, 2800000, True), (sp.F64, 3200000, False), (sp.F3
     col = np.sort(np.random.default_rng(1).integers(0, n, (n, 20)), axis=1).ravel().astype(np.uint32)
     i = sp.Plan(ctx, "COO-nnz", sp.Coo.from_arrays(n, n, row, col, np.ones(row.size, sp.NP_DTYPE[dt]))).info()
     assert i["algo"] == sp.ALGO_SEGMENTED_SORTED and (i["ntiles"] > 600) == small, (dt, nnz, i)
+    # threads and entries per thread; merge tiles of the same name report no lanes, and what is
+    # reported can be asked for
+    assert (i["lanes_per_row"], i["items_per_lane"]) == ((512 if dt == sp.F32 else 256, 8) if small
+                                                         else (1024, 16 if dt == sp.F32 else 8))
+    A = sp.Coo.from_arrays(n, n, row, col, np.ones(row.size, sp.NP_DTYPE[dt]))
+    for kern in ("CSR-nnz", "COO-nnz"):
+        j = sp.Plan(ctx, kern, A, sp.opts(algo=i["algo"], items_per_lane=i["items_per_lane"],
+                                          lanes_per_row=i["lanes_per_row"] if kern == "COO-nnz" else 0)).info()
+        assert j["algo"] == i["algo"] and j["lanes_per_row"] == 0 and j["items_per_lane"] == i["items_per_lane"], j
 print("ok")
 """
 
