@@ -78,18 +78,21 @@ static void space_for(const sp_coo *A, int id, std::vector<Pt> &v) {
             p.o.items_per_lane = I;
             v.push_back(p);
         }
-        Pt p{id, base};  // row-ordered tiles (the default takes column order where it fits)
+        Pt p{id, base};  // row-ordered tiles (items_per_lane alone takes column order where it fits)
         p.o.algo = SP_ALGO_SEGMENTED;
         v.push_back(p);
+        Pt q{id, base};  // column-ordered merge tiles of 4 (the default may take wide tiles)
+        q.o.items_per_lane = 4;
+        v.push_back(q);
     } else if (id >= SP_K_BCSR_BLOCK && id <= SP_K_BCOO_NNZ) {
         Pt p{id, base};
         p.o.row_block_size = p.o.col_block_size = 2;
         v.push_back(p);
-        if (id == SP_K_BCSR_BLOCK || id == SP_K_BCSR_NNZ) {  // entry-balanced BCSR (automatic only when skewed)
-            Pt q{id, base};
-            q.o.algo = SP_ALGO_SEGMENTED;
-            v.push_back(q);
-        }
+        // entry-balanced BCSR (automatic only when skewed), block-balanced BCOO (automatic unless
+        // even block rows are faster)
+        Pt q{id, base};
+        q.o.algo = SP_ALGO_SEGMENTED;
+        v.push_back(q);
     } else {
         for (uint32_t vert : {4u, 8u}) {
             Pt p{id, base};
@@ -107,6 +110,18 @@ static void space_for(const sp_coo *A, int id, std::vector<Pt> &v) {
             Pt p{id, base};
             p.o.vert = vs;
             p.o.lds_slice = cap;
+            v.push_back(p);
+        }
+        // two stripes without wide tiles: the row kernel and merge tiles, COO tiles of 8
+        if (id == SP_K_DCSR || id == SP_K_RBDCSR || id == SP_K_BDCSR) {
+            for (int algo : {SP_ALGO_VECTOR, SP_ALGO_SEGMENTED_SORTED}) {
+                Pt p{id, base};
+                p.o.algo = algo;
+                v.push_back(p);
+            }
+        } else if (csr_coo) {
+            Pt p{id, base};
+            p.o.items_per_lane = 8;
             v.push_back(p);
         }
     }
