@@ -377,7 +377,7 @@ bool no_knobs(const sp_opts &o) {
 
 // What the row kernels make of even CSR rows.
 struct EvenRows {
-    double avg;
+    double avg = 0;
     uint32_t maxlen = 0;
     bool cross = false;  // some row crosses a multiple of 2048 entries, where wide tiles end
     // steps that a wave of the chunked row kernel takes (rows side by side, those of its longest)
@@ -385,7 +385,12 @@ struct EvenRows {
     bool two_steps(double share) const { return steps >= (1 + share) * waves; }
     // lengths differ little, or mostly within one step
     bool calm() const { return avg < 16 ? maxlen <= 1.25 * avg : !two_steps(0.25) && maxlen <= 1.6 * avg; }
-    EvenRows(const uint32_t *rowptr, uint32_t nrows) : avg((double)rowptr[nrows] / nrows) {
+    EvenRows() = default;
+    EvenRows(const uint32_t *rowptr, uint32_t nrows) : avg(nrows ? (double)rowptr[nrows] / nrows : 0.0) {
+        if (avg < 16) {  // (another row kernel)
+            for (uint32_t i = 0; i < nrows; i++) maxlen = std::max(maxlen, rowptr[i + 1] - rowptr[i]);
+            return;
+        }
         const uint32_t L = chunk_lanes(avg), rows = 64 / L;
         for (uint32_t i = 0; i < nrows; i += rows, waves++) {
             uint32_t most = 0;
@@ -393,7 +398,7 @@ struct EvenRows {
                 const uint32_t b = rowptr[r], e = rowptr[r + 1];
                 if (e == b) continue;
                 maxlen = std::max(maxlen, e - b);
-                most = std::max(most, (e + 3) / 4 - b / 4);
+                most = std::max(most, (e - 1) / 4 + 1 - b / 4);
                 cross = cross || b / 2048 != (e - 1) / 2048;
             }
             steps += (most + L - 1) / L;
@@ -473,7 +478,7 @@ uint32_t even_rows_least(const EvenRows &rows, uint32_t nrows, size_t sv, bool s
 //   skewed rows and COO from 2K entries on: R-MAT 2^12 x 8 FP32 CSR 8.4 -> 6.5, 2^16 x 16
 //     11.0 -> 8.2, 2^18 x 16 FP64 28.8 -> 22.7, 2^20 x 16 FP32 72.6 -> 64.6; COO 5-point stencil
 //     700^2 14.2 -> 9.6
-//   even CSR rows (`even`: their row pointers) where even_rows_least says so; 2D tilings ask for
+//   even CSR rows (`even`: what they are like) where even_rows_least says so; 2D tilings ask for
 //     1M entries themselves
 //   rows made of aligned four-column runs keep their four-value x loads (the caller's check)
 // Shape: scattered columns (over 0.3 lines per entry in row order; R-MAT 0.84, banded and
@@ -483,13 +488,13 @@ uint32_t even_rows_least(const EvenRows &rows, uint32_t nrows, size_t sv, bool s
 // 37.0 with 8192, 3.5M 39.9 with 8192, 46.1 in the row kernel); local ones 16 entries per thread in
 // the smallest workgroup (199999 x 33 FP32: 14.2 with 256 threads, 16.4 with 1024), 8-byte sums
 // 8 per thread (20.1 against 24.3).
-WideShape wide_shape(const sp_plan *p, const uint32_t *even, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
+WideShape wide_shape(const sp_plan *p, const EvenRows *even, const uint32_t *colind, uint32_t nrows, uint32_t nnz) {
     const sp_opts &o = p->opts;
     const size_t sv = sp_dtype_size(p->dtype);
     if (p->algo != SP_ALGO_AUTO || !no_knobs(o)) return {};
     if (nnz < (even ? 192u << 10 : 2u << 10) || nnz > 0xF0000000u) return {};  // (entry numbers plus a tile stay below 2^32)
     const bool scattered = row_lines(colind, nnz, sv) > 0.3;
-    if (even && nnz < even_rows_least(EvenRows(even, nrows), nrows, sv, scattered)) return {};
+    if (even && nnz < even_rows_least(*even, nrows, sv, scattered)) return {};
     if (acc_size(p->dtype) == 8) return scattered && nnz >= 3u << 20 ? WideShape{1024, 8} : WideShape{256, 8};
     if (scattered && nnz >= 3u << 20) return {1024, 16};
     return !scattered && nnz >= 1u << 20 ? WideShape{256, 16} : WideShape{512, 8};
@@ -500,9 +505,12 @@ WideShape wide_shape(const sp_plan *p, const uint32_t *even, const uint32_t *col
 int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
     const size_t sa = acc_size(p->dtype);
     Prob P = g.h_probs[0];
-    const uint32_t nnz = P.nent, nw = (uint32_t)(((uint64_t)nnz + 31) / 32), emin = spd::panel_entries(32, sa);
+    const uint32_t nnz = P.nent, nw = (uint32_t)(((uint64_t)nnz + 31) / 32);
+    // workgroups take 2^esh entries at one right-hand side, half as many at each wider width
+    const int esh = __builtin_ctz(spd::panel_entries(1, sa));
     std::vector<uint32_t> word(2 * ((size_t)nw + 1), 0), rows, zrows;
-    std::vector<spd::Cross> cross;
+    std::vector<spd::Cross> level[6];  // the rows that cross workgroups at width i and no narrower one
+    rows.reserve(P.nrows);
     for (uint32_t i = 0; i < P.nrows; i++) {
         if (rowptr[i + 1] == rowptr[i]) {
             zrows.push_back(i);
@@ -511,7 +519,10 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
         const uint32_t b = rowptr[i], e = rowptr[i + 1] - 1;
         word[2 * (size_t)(e / 32)] |= 1u << (e % 32);
         rows.push_back(i);
-        if (b / emin != e / emin) cross.push_back(spd::Cross{0, i, b, e, (int64_t)i, P.ldy, 0});
+        if ((b ^ e) >> (esh - 5)) {
+            const int top = 31 - __builtin_clz(b ^ e);  // highest bit in which they differ
+            level[top >= esh ? 0 : esh - top].push_back(spd::Cross{0, i, b, e, (int64_t)i, P.ldy, 0});
+        }
     }
     for (uint32_t w = 0, n = 0; w <= nw; w++) {  // (the closing pair: all rows)
         word[2 * (size_t)w + 1] = n;
@@ -522,22 +533,20 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
     n.work.dtype = p->dtype;
     n.work.nprob = n.work.nunits = 1;
     n.work.panel_nent = nnz;
-    // one block: words, rows, rows without entries, the crossing rows of every width, descriptor
-    std::vector<spd::Cross> lists[6];
+    std::vector<spd::Cross> &cross = n.h_cross;  // a width's crossing rows come first
     uint64_t carries = 0;
-    size_t o_rows = piece(word.size() * 4), o_zrows = o_rows + piece(rows.size() * 4);
-    size_t o_list[7] = {o_zrows + piece(zrows.size() * 4)};
     for (int i = 0; i < 6; i++) {
-        const uint32_t E = spd::panel_entries(1 << i, sa);
-        for (const spd::Cross &C : cross)
-            if (C.b / E != C.e / E) lists[i].push_back(C);
-        n.work.ncross[i] = (uint32_t)lists[i].size();
-        o_list[i + 1] = o_list[i] + piece(lists[i].size() * sizeof(spd::Cross));
+        cross.insert(cross.end(), level[i].begin(), level[i].end());
+        n.work.ncross[i] = (uint32_t)cross.size();
+        const uint32_t E = 1u << (esh - i);
         carries = std::max(carries, (((uint64_t)nnz + E - 1) / E) << i);
     }
+    // one block: words, rows, rows without entries, crossing rows, descriptor
+    const size_t o_rows = piece(word.size() * 4), o_zrows = o_rows + piece(rows.size() * 4);
+    const size_t o_cross = o_zrows + piece(zrows.size() * 4), o_prob = o_cross + piece(cross.size() * sizeof(spd::Cross));
     void *d;
     const size_t mark = p->allocs.size();
-    int rc = plan_alloc(p, o_list[6] + sizeof(Prob), &d);
+    int rc = plan_alloc(p, o_prob + sizeof(Prob), &d);
     if (!rc) rc = plan_alloc(p, carries * sa, &n.work.d_carry_val);
     if (rc) {
         plan_release(p, mark, p->allocs.size());
@@ -548,22 +557,19 @@ int build_panel(sp_plan *p, PlanWork &g, const uint32_t *rowptr) {
     P.rind = (const uint32_t *)(dev + o_rows);
     P.hcol = (const uint32_t *)(dev + o_zrows);
     P.nhcol = (uint32_t)zrows.size();
-    std::vector<char> host(o_list[6] + sizeof(Prob), 0);
+    const std::unique_ptr<char[]> host(new char[o_prob + sizeof(Prob)]);
     auto put = [&](size_t at, const void *src, size_t n) {
-        if (n) memcpy(host.data() + at, src, n);
+        if (n) memcpy(host.get() + at, src, n);
     };
     put(0, word.data(), word.size() * 4);
     put(o_rows, rows.data(), rows.size() * 4);
     put(o_zrows, zrows.data(), zrows.size() * 4);
-    for (int i = 0; i < 6; i++) {
-        put(o_list[i], lists[i].data(), lists[i].size() * sizeof(spd::Cross));
-        n.work.d_cross[i] = (spd::Cross *)(dev + o_list[i]);
-    }
-    put(o_list[6], &P, sizeof(P));
-    n.work.d_prob = (Prob *)(dev + o_list[6]);
-    SP_HIP_TRY(hipMemcpy(d, host.data(), host.size(), hipMemcpyHostToDevice));
+    put(o_cross, cross.data(), cross.size() * sizeof(spd::Cross));
+    put(o_prob, &P, sizeof(P));
+    for (int i = 0; i < 6; i++) n.work.d_cross[i] = (spd::Cross *)(dev + o_cross);
+    n.work.d_prob = (Prob *)(dev + o_prob);
+    SP_HIP_TRY(hipMemcpy(d, host.get(), o_prob + sizeof(Prob), hipMemcpyHostToDevice));
     n.h_probs = {P};
-    n.h_cross = std::move(cross);
     g = std::move(n);
     return SP_OK;
 }
@@ -595,32 +601,49 @@ int wide_part(sp_plan *p, const Prob &rows, const uint32_t *rowptr, WideShape s,
     const uint32_t nt = (uint32_t)(((uint64_t)nnz + tile - 1) / tile);
     const uint64_t tot = (uint64_t)nt * words;
     // the word of every thread, every kept row's sum, the first kept row of each tile's (those that
-    // end in it and the empty ones before the next), the row it carries out
-    std::vector<uint32_t> word((size_t)nt * s.nt, 0), &cent = out.cent, &crow = out.crow, &carry = out.carry;
-    std::vector<uint32_t> kept, gap;  // rows outside and inside long gaps
-    std::vector<uint16_t> rmap;
+    // end in it and the empty ones before the next), the row it carries out; words and sums in the
+    // block that is uploaded, the tile of a row found without a division
+    const size_t o_rmap = piece((size_t)nt * s.nt * 4);
+    const std::unique_ptr<char[]> host(new char[o_rmap + (size_t)P.nrows * 2]);
+    uint32_t *const word = (uint32_t *)host.get();
+    uint16_t *const rmap = (uint16_t *)(host.get() + o_rmap);
+    memset(word, 0, (size_t)nt * s.nt * 4);
+    std::vector<uint32_t> &cent = out.cent, &crow = out.crow, &carry = out.carry;
+    std::vector<uint32_t> kept, gap;  // rows outside (once there are any inside) and inside long gaps
+    uint32_t nkept = 0;
     carry.assign((size_t)nt + 1, spd::NONE);
+    crow.reserve((size_t)nt + 1);
+    cent.reserve((size_t)nt + 1);
     crow.push_back(0);
-    for (uint32_t i = 0, next = 0, ord = 0; i <= P.nrows; i++) {
+    const uint32_t ish = (uint32_t)__builtin_ctz(s.ipt), imask = s.ipt - 1;
+    uint64_t t0 = 0;  // first entry of tile t
+    auto keep = [&](uint32_t i, uint32_t ord) {
+        rmap[nkept++] = (uint16_t)ord;
+        if (!gap.empty()) kept.push_back(i);
+    };
+    for (uint32_t i = 0, next = 0, ord = 0, t = 0; i <= P.nrows; i++) {
         if (i < P.nrows && rowptr[i + 1] == rowptr[i]) continue;
-        for (const bool lng = i - next > spd::WIDE_GAP; next < i; next++) {
-            (lng ? gap : kept).push_back(next);
-            if (!lng) rmap.push_back(0);
+        if (i - next > spd::WIDE_GAP) {
+            if (gap.empty())
+                for (uint32_t k = 0; k < nkept; k++) kept.push_back(k);
+            for (; next < i; next++) gap.push_back(next);
         }
+        for (; next < i; next++) keep(next, 0);
         if (i == P.nrows) break;
         next = i + 1;
-        const uint32_t e = rowptr[i + 1] - 1, t = e / tile, at = e % tile;
-        while (crow.size() <= t) {  // row i is the first that ends in tile t
-            crow.push_back((uint32_t)kept.size());
+        const uint32_t b = rowptr[i], e = rowptr[i + 1] - 1;
+        while (e >= t0 + tile) {  // row i is the first that ends in tile t
+            crow.push_back(nkept);
+            t++;
+            t0 += tile;
             ord = 0;
         }
-        uint32_t &w = word[(size_t)t * s.nt + at / s.ipt];
-        w |= 1u << (at % s.ipt);
-        kept.push_back(i);
-        rmap.push_back((uint16_t)++ord);
-        for (uint32_t q = rowptr[i] / tile; q < t; q++) carry[q] = i;
+        const uint32_t at = (uint32_t)(e - t0);
+        word[(size_t)t * s.nt + (at >> ish)] |= 1u << (at & imask);
+        keep(i, ++ord);
+        if (b < t0)
+            for (uint32_t q = b / tile; q < t; q++) carry[q] = i;
     }
-    const uint32_t nkept = (uint32_t)kept.size();
     while (crow.size() <= nt) crow.push_back(nkept);
     crow[nt] = nkept;
     for (uint32_t t = 0; t < nt; t++) {
@@ -638,13 +661,11 @@ int wide_part(sp_plan *p, const Prob &rows, const uint32_t *rowptr, WideShape s,
     // (words, row map); each piece aligned, with the slack that plan_alloc gives an array
     int rc;
     const size_t o_val = piece(tot * 4), o_base = o_val + piece(tot * sv), o_flag = o_base + piece(tot / 64 * 4);
-    std::vector<char> host(piece(word.size() * 4) + rmap.size() * 2);
-    memcpy(host.data(), word.data(), word.size() * 4);
-    if (!rmap.empty()) memcpy(host.data() + piece(word.size() * 4), rmap.data(), rmap.size() * 2);
     void *sorted, *tables;
-    if ((rc = plan_alloc(p, o_flag + 4, &sorted)) || (rc = plan_upload(p, host.data(), host.size(), &tables))) return rc;
+    if ((rc = plan_alloc(p, o_flag + 4, &sorted)) || (rc = plan_upload(p, host.get(), o_rmap + (size_t)nkept * 2, &tables)))
+        return rc;
     char *const key = (char *)sorted, *const val = key + o_val, *const base = key + o_base, *const flag = key + o_flag;
-    char *const dword = (char *)tables, *const drmap = dword + piece(word.size() * 4);
+    char *const dword = (char *)tables, *const drmap = dword + o_rmap;
     // on the null stream, as the uploads before it
     if ((rc = launch_wide_sort(nullptr, P.cind, P.val, sv, nnz, tile, words, pb, s.ipt, sa, (uint32_t *)key, val,
                                (uint32_t *)base, (uint32_t *)flag)))
@@ -720,7 +741,8 @@ bool coo_sorted(const sp_coo *A) {
 // CSR (ids 0, 1)
 // ---------------------------------------------------------------------------
 // With `wide`, a plan that takes wide tiles gets its row-ordered group here and the shape in *wide.
-static int build_csr_group(sp_plan *p, const sp_csr *A, WideShape *wide) {
+// `even`: what the rows are like (automatic plans).
+static int build_csr_group(sp_plan *p, const sp_csr *A, WideShape *wide, EvenRows &even) {
     const size_t sv = sp_dtype_size(A->dtype);
     if (!A->rowptr || (A->nnz && (!A->colind || !A->values))) return SP_ERR_ARG;
     if (A->rowptr[0] != 0 || A->rowptr[A->nrows] != A->nnz) return SP_ERR_ARG;
@@ -729,11 +751,11 @@ static int build_csr_group(sp_plan *p, const sp_csr *A, WideShape *wide) {
     for (uint32_t k = 0; k < A->nnz; k++)
         if (A->colind[k] >= A->ncols) return SP_ERR_ARG;
     if (p->algo == SP_ALGO_AUTO) {
-        uint32_t maxlen = 0;
-        for (uint32_t i = 0; i < A->nrows; i++) maxlen = std::max(maxlen, A->rowptr[i + 1] - A->rowptr[i]);
-        const double avg = A->nrows ? (double)A->nnz / A->nrows : 0.0;
+        even = EvenRows(A->rowptr, A->nrows);
+        const uint32_t maxlen = even.maxlen;
+        const double avg = even.avg;
         if (wide && !quad_rows(A->rowptr, A->nrows, A->colind, A->nnz, A->ncols))
-            *wide = wide_shape(p, maxlen > 4 * avg + 64 ? nullptr : A->rowptr, A->colind, A->nrows, A->nnz);
+            *wide = wide_shape(p, maxlen > 4 * avg + 64 ? nullptr : &even, A->colind, A->nrows, A->nnz);
         // Row-granular kernel for even row lengths up to a few million entries (one launch,
         // no carries); the merge-path kernel for skewed rows, and for large matrices, where
         // its deeper per-thread load batches win (27-point stencil, 113M entries: 1.3x).
@@ -875,10 +897,11 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
     const sp_opts opts = p->opts;
     const int algo = p->algo;
     WideShape s;
-    int rc = build_csr_group(p, A, &s);
+    EvenRows even;
+    int rc = build_csr_group(p, A, &s, even);
     if (!rc && s.nt && unfit(rc = add_wide(p, A->rowptr, s))) {
         drop_groups(p, opts, algo);
-        rc = build_csr_group(p, A, nullptr);
+        rc = build_csr_group(p, A, nullptr, even);
     }
     // even rows (their group is the row kernels' either way): panels at some widths
     const PlanWork &rows = p->many ? *p->many : *p;
@@ -886,7 +909,7 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
         A->nnz > 0xF0000000u)
         return rc;
     const size_t sv = sp_dtype_size(A->dtype);
-    p->panel_widths = panel_widths(EvenRows(A->rowptr, A->nrows), A->nnz, sv, row_lines(A->colind, A->nnz, sv) > 0.3);
+    p->panel_widths = panel_widths(even, A->nnz, sv, row_lines(A->colind, A->nnz, sv) > 0.3);
     if (!p->panel_widths) return SP_OK;
     p->panel = std::make_unique<PlanWork>(rows);
     if ((rc = build_panel(p, *p->panel, A->rowptr))) {
