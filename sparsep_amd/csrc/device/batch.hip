@@ -131,7 +131,7 @@ extern "C" int sp_batch_create(sp_ctx *ctx, int nprob, sp_plan *const *plans, co
         // even rows, one right-hand side: the row kernel (a group of wide tiles and its fix-up
         // beside it: 158 against 154 us for 24 problems of up to 2M entries)
         const bool rows = k[i] == 1 && p->many && p->many->work.kind == WK_CSR_VEC;
-        const PlanWork &pw = rows ? *p->many : p->group(k[i]);
+        const PlanWork &pw = rows ? *p->many : p->group(k[i], true);
         const Work &w = pw.work;
         b->algo_bytes += p->algo_bytes + (uint64_t)(k[i] - 1) * ((uint64_t)p->nrows + p->ncols) * sp_dtype_size(dt);
         const int kmax = max_rhs_chunk(w);

@@ -67,12 +67,13 @@ struct sp_plan : PlanWork {  // (the base: the main launch group)
     // wide tiles take one right-hand side: several run on this group (even CSR rows: the row
     // kernels; otherwise panels)
     std::unique_ptr<PlanWork> many;
-    // even CSR rows: panels at the widths (powers of two) whose bit is set
+    // even CSR rows: panels at the widths (powers of two) whose bit is set, alone and in batches
     std::unique_ptr<PlanWork> panel;
-    uint32_t panel_widths = 0;
+    uint32_t panel_widths = 0, batch_widths = 0;
     // the group that a call with k right-hand sides runs (by its widest pass)
-    const PlanWork &group(int k) const {
-        if (k > 1 && panel && panel_widths >> (31 - __builtin_clz((unsigned)(k < 32 ? k : 32))) & 1) return *panel;
+    const PlanWork &group(int k, bool batch = false) const {
+        const uint32_t widths = batch ? batch_widths : panel_widths;
+        if (k > 1 && panel && widths >> (31 - __builtin_clz((unsigned)(k < 32 ? k : 32))) & 1) return *panel;
         if (k > 1 && many) return *many;
         return *this;
     }

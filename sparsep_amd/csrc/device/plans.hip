@@ -422,7 +422,12 @@ struct EvenRows {
 //     columns INT32 12.5, 15.5), not 256 bytes with calm local rows above 8 (FP64 12 in every row 3M
 //     90.2, 103.7)
 //   longer rows never (27-point stencil: 18.4, 30.8)
-uint32_t panel_widths(const EvenRows &rows, uint32_t nnz, size_t sv, bool scattered) {
+// In a batch the members share the second launch, and lines by size would split those of one width
+// into two groups: 16 problems of 1000 to 60000 rows, by the lines above and without those for x
+// rows below 64 bytes: 2 .. 64 entries scattered FP32 4 and 8 columns up to 8000 rows 103, 59; local
+// FP64 2 and 4 columns 107, 79; 33 in every row scattered FP32 4 and 8 columns 100.6, 83.0, but
+// local 64.9, 70.6, so calm local rows keep them.
+uint32_t panel_widths(const EvenRows &rows, uint32_t nnz, size_t sv, bool scattered, bool batch) {
     const double avg = rows.avg;
     const bool calm = rows.calm() || rows.maxlen <= 1.25 * avg;
     uint32_t mask = 0;
@@ -435,6 +440,8 @@ uint32_t panel_widths(const EvenRows &rows, uint32_t nnz, size_t sv, bool scatte
             use = false;
         else if (bytes >= 64)
             use = nnz <= (bytes > 64 ? 1u << 20 : calm && !scattered && avg > 40 ? 2560u << 10 : ~0u);
+        else if (batch && (scattered || !calm))
+            use = true;
         else if (calm)
             use = nnz >= 2u << 20 && (bytes < 32 || scattered);
         else
@@ -909,8 +916,10 @@ int build_csr_plan(sp_plan *p, const sp_csr *A) {
         A->nnz > 0xF0000000u)
         return rc;
     const size_t sv = sp_dtype_size(A->dtype);
-    p->panel_widths = panel_widths(even, A->nnz, sv, row_lines(A->colind, A->nnz, sv) > 0.3);
+    const bool scattered = row_lines(A->colind, A->nnz, sv) > 0.3;
+    p->panel_widths = panel_widths(even, A->nnz, sv, scattered, false);
     if (!p->panel_widths) return SP_OK;
+    p->batch_widths = panel_widths(even, A->nnz, sv, scattered, true);
     p->panel = std::make_unique<PlanWork>(rows);
     if ((rc = build_panel(p, *p->panel, A->rowptr))) {
         p->panel.reset();

@@ -65,3 +65,8 @@ hipError_t hipStreamSynchronize(hipStream_t s) { return hipSuccess; }
 hipError_t hipStreamQuery(hipStream_t s) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e) { *e = (hipEvent_t)malloc(1); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { return hipEventCreate(e); }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned f) { return hipStreamCreate(s); }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned f) { return hipSuccess; }

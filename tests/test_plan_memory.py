@@ -203,6 +203,18 @@ for lens, local, dt, k, launches in [  # the row kernels take one launch, panels
     n = fake.fake_launches()
     plan.spmm(k, 64, k, 64, k)
     assert fake.fake_launches() - n == launches, (lens[:4], len(lens), local, dt, k, fake.fake_launches() - n)
+for lens, local, dt, ks, groups in [  # batch members of one width share panels, whatever their sizes
+        ([spread(2, 64, 1000), spread(2, 64, 9000)], True, sp.F32, [4, 4], 1),
+        ([np.full(600, 33), spread(2, 64, 9000)], False, sp.F64, [2, 2], 1),
+        ([np.full(2000, 33), np.full(9000, 33)], False, sp.F32, [8, 8], 1),
+        ([np.full(2000, 33), spread(2, 64, 9000)], True, sp.F32, [8, 8], 2),
+        ([spread(2, 64, 1000), spread(2, 64, 9000)], True, sp.F32, [4, 8], 2)]:
+    plans = [sp.Plan(ctx, "CSR-nnz", matrix(n, local, dt)) for n in lens]
+    batch = sp.Batch(ctx, plans, ks, graph=False)
+    assert batch.info()["groups"] == groups, (dt, ks, local, batch.info())
+    n = fake.fake_launches()
+    batch.run([64] * 2, [64] * 2)
+    assert fake.fake_launches() - n == (3 if len(lens[0]) == 2000 and local else 2 * groups), (dt, ks, local)
 ROWS, WIDE = sp.ALGO_VECTOR, sp.ALGO_SEGMENTED_SORTED
 for lens, local, dt, algo in [
         (np.full(100000, 17), True, sp.F32, ROWS), (np.full(290000, 17), True, sp.F32, WIDE),
