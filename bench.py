@@ -212,7 +212,7 @@ def wl_rmat(sp, ctx, args, orc):
     if os.path.exists(report):
         with open(report) as f:
             ho = json.load(f)["held_out"]
-        sel = {"source": "sparsep_amd/data/selector_report.json (held-out corpus, measured when trained)",
+        sel = {"source": "sparsep_amd/data/selector_report.json (held-out corpus, measured when trained, before wide tiles)",
                "learned_pick_over_exhaustive_best_geomean": ho["learned"]["geomean_ratio"],
                "with_fallback_geomean": ho["learned_with_fallback"]["geomean_ratio"],
                "selection_overhead_median": ho["overhead"]["select_over_exhaustive_median"]}

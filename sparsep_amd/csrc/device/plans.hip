@@ -490,7 +490,8 @@ uint32_t even_rows_least(const EvenRows &rows, uint32_t nrows, size_t sv, bool s
 //   rows made of aligned four-column runs keep their four-value x loads (the caller's check)
 // Shape: scattered columns (over 0.3 lines per entry in row order; R-MAT 0.84, banded and
 // stencils up to 0.2) want the widest tile once it leaves enough of them (R-MAT 2^20: 74.8 with
-// 4096 entries, 66.4 with 8192, 62.1 with 16384; uniform INT8 9.9M entries: 29.5, 22.9, 23.0;
+// 4096 entries, 66.4 with 8192, 62.1 with 16384, which with all that came since, above all sums that
+// round once, are 64.6; uniform INT8 9.9M entries: 29.5, 22.9, 23.0;
 // but 2.9M entries INT16: 13.8 with 4096, 16.4 with 16384; FP64 3 in every row 2.4M: 30.1 with 2048,
 // 37.0 with 8192, 3.5M 39.9 with 8192, 46.1 in the row kernel); local ones 16 entries per thread in
 // the smallest workgroup (199999 x 33 FP32: 14.2 with 256 threads, 16.4 with 1024), 8-byte sums
